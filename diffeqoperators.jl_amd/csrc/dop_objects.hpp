@@ -19,16 +19,14 @@ int set_error(int code, const std::string& msg);
 
 struct dop_plan {
     dop::DevicePlan d;            // host copy (device table pointers), device copy, tiled path
-    dop::PlanDev* dev = nullptr;  // device copy of d.host
+    dop::PlanDev* dev = nullptr;  // device copy of d.host, followed by the plan's tables
     dop::HostPlan H;              // host tables of the current values (dop_plan_update)
     std::atomic<int> tuned{0};    // variant chosen by the autotuner (or the tuning cache)
     std::mutex tune_mu;           // one tuning at a time
-    std::vector<void*> bufs;
     int64_t in_elems = 0, out_elems = 0;
     int device = 0;
     ~dop_plan()
     {
-        for (void* b : bufs) (void)hipFree(b);
         if (dev) (void)hipFree(dev);
     }
 };

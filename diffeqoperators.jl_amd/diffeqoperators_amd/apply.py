@@ -8,7 +8,10 @@ contiguous device tensors (float64, float32 or bfloat16); there is no CPU path.
 from __future__ import annotations
 
 import ctypes as C
+import itertools
 import os
+import threading
+import weakref
 
 import torch
 
@@ -279,87 +282,146 @@ def _bc_structure(bc):
     return ("affine", len(bc.a_l), len(bc.a_r))
 
 
+# The implicit `A*u` / `mul_` paths keep a plan set per live owner (an L*Q object or a sum of
+# them) and kind of array.  When an owner goes, its plans go to a pool, and an owner of the same
+# structure (operators' kinds and sizes, BC kinds and tap counts) takes them over with one
+# dop_plan_update: a method-of-lines RHS that builds a new BC at every call (heat_equation.jl:38-43,
+# KdV.jl:26-30) keeps using one plan, and owners that live side by side never replace each
+# other's values.  (One plan per structure, rebound to whichever owner was applied last, cost two
+# operators of one structure used in turn a table rebuild and upload per call: 460 us on the
+# 4096^2 FP64 Laplacian whose apply takes 50, 10 ms on a 1-D line of 2^18 points.)  The pool holds
+# at most _POOL_MAX sets, the oldest dropped first, and is guarded by a lock.
+_POOL = {}           # number -> (structure, plans, stream they were last applied on)
+_POOL_MAX = 64
+_POOL_LOCK = threading.RLock()
+_POOL_COUNT = itertools.count()
+_MIXED = object()    # applied on several streams
+
+
 class _Bound:
-    """The plans of one owner (an L*Q object) and the descriptors of its values."""
+    """The plans of one owner for one kind of array, the descriptors of its values, and the
+    stream the plans have been applied on (None: not yet; _MIXED: several)."""
 
-    def __init__(self, skey, plans, descs):
-        self.skey, self.plans, self.descs = skey, plans, descs
+    __slots__ = ("skey", "descs", "plans", "stream", "__weakref__")
+
+    def __init__(self, skey, descs):
+        self.skey, self.descs, self.plans, self.stream = skey, descs, None, None
+
+    def __del__(self):
+        # plans applied on several streams are not reused: an update on one of them would not
+        # wait for applies still queued on another
+        try:
+            if self.plans is not None and self.stream is not None and self.stream is not _MIXED:
+                with _POOL_LOCK:
+                    _POOL[next(_POOL_COUNT)] = (self.skey, self.plans, self.stream)
+                    while len(_POOL) > _POOL_MAX:
+                        _POOL.pop(next(iter(_POOL)))
+        except Exception:   # interpreter shutdown
+            pass
 
 
-# Plans shared by owners of the same structure (same operators' kinds and sizes, same BC kinds
-# and tap counts): a method-of-lines RHS that builds a new BC at every call (heat_equation.jl:
-# 38-43, KdV.jl:26-30) reuses one plan and only replaces its values (dop_plan_update) instead
-# of creating a plan per call.  Bounded: the least recently used structures are dropped.
-_SHARED: "collections.OrderedDict" = None
-_SHARED_MAX = 64
+_LIVE = weakref.WeakSet()
 
 
-def _shared():
-    global _SHARED
-    if _SHARED is None:
-        import collections
-        _SHARED = collections.OrderedDict()
-    return _SHARED
-
-
-def ghost_plans(owner, terms, u: torch.Tensor, accum=_abi.ACC_AUTO, shared=False):
-    """Plans evaluating sum_t L_t*Q_t*u, cached on owner.  shared=True (the implicit `A*u` /
-    `mul_` paths, which use the plans at once): plans of the same structure are shared between
-    owners and rebound to an owner's values on use.  shared=False (plans handed to the caller,
-    who may keep them, e.g. in a batch or a server): the owner's own plans."""
+def ghost_plans(owner, terms, u: torch.Tensor, accum=_abi.ACC_AUTO):
+    """Plans evaluating sum_t L_t*Q_t*u, cached on owner: the owner's own plans, for callers who
+    keep them (in a batch, a server, an integrator)."""
     jsize = julia_size(u)
     storage = storage_of(u)
-    key = ("ghost", jsize, storage, accum, u.device.index)
+    key = ("own", jsize, storage, accum, u.device.index)
     cache = _plan_cache(owner)
-    if not shared:
-        own = cache.get(key + ("own",))
-        if own is None:
-            with torch.cuda.device(u.device):
-                own = []
-                for ops, bcs, _, sem in _ghost_groups(terms, len(jsize), jsize):
-                    d, keep = make_desc(ops, jsize, storage, input_kind=_abi.INPUT_GHOST,
-                                        semantics=sem, bcs=bcs, accum=accum)
-                    own.append(Plan(d, keep + [bcs]))
-            cache[key + ("own",)] = own
-        return own
-    bound = cache.get(key)
-    if bound is None:
-        descs, groups = [], _ghost_groups(terms, len(jsize), jsize)
-        for ops, bcs, _, sem in groups:
-            d, keep = make_desc(ops, jsize, storage, input_kind=_abi.INPUT_GHOST,
-                                semantics=sem, bcs=bcs, accum=accum)
-            descs.append((d, keep + [bcs]))
-        # plans are created with the kernel selection the environment asks for
-        env = (os.environ.get("DOP_FORCE_GENERIC"), os.environ.get("DOP_TILE_VARIANT"))
-        skey = key + env + (tuple((sem, tuple(_op_structure(L) for L in ops),
-                             tuple(sorted((ax, _bc_structure(bc)) for ax, bc in bcs.items())))
-                            for ops, bcs, _, sem in groups),)
-        bound = cache[key] = _Bound(skey, None, descs)
-    shared = _shared()
-    plans = shared.get(bound.skey)
-    with torch.cuda.device(u.device):
-        if plans is None:
-            plans = [Plan(d, keep) for d, keep in bound.descs]
-            for p in plans:
-                p._owner = bound
-            shared[bound.skey] = plans
-            while len(shared) > _SHARED_MAX:
-                shared.popitem(last=False)
-        else:
-            shared.move_to_end(bound.skey)
-            for i, p in enumerate(plans):
-                if p._owner is bound:
-                    continue
-                d, keep = bound.descs[i]
-                try:
-                    p.update(d, keep)
-                except _abi.DopError:
-                    # same kinds and sizes but a different row structure (e.g. coefficients
-                    # that are no longer uniform): a plan of its own
-                    p = plans[i] = Plan(d, keep)
-                p._owner = bound
-    bound.plans = plans
-    return plans
+    own = cache.get(key)
+    if own is None:
+        with torch.cuda.device(u.device):
+            own = [Plan(d, keep) for d, keep, _ in _ghost_descs(terms, u, accum)]
+        cache[key] = own
+    return own
+
+
+def _ghost_descs(terms, u, accum):
+    """(descriptor, what it points to, structure) per plan of sum_t L_t*Q_t*u."""
+    jsize = julia_size(u)
+    storage = storage_of(u)
+    out = []
+    for ops, bcs, _, sem in _ghost_groups(terms, len(jsize), jsize):
+        d, keep = make_desc(ops, jsize, storage, input_kind=_abi.INPUT_GHOST, semantics=sem,
+                            bcs=bcs, accum=accum)
+        out.append((d, keep + [bcs], (sem, tuple(_op_structure(L) for L in ops),
+                                      tuple(sorted((ax, _bc_structure(bc)) for ax, bc in bcs.items())))))
+    return out
+
+
+def _take_pooled(skey, stream, any_stream):
+    for k, (s, plans, st) in list(_POOL.items())[::-1]:
+        if s == skey and (any_stream or st == stream) and _POOL.pop(k, None) is not None:
+            return plans
+    return None
+
+
+def _bind(owner, key, u, accum, bound, stream):
+    """The owner's _Bound for arrays like u, with plans holding its values."""
+    with _POOL_LOCK, torch.cuda.device(u.device):
+        if bound is None:
+            bound = _plan_cache(owner).get(key)
+        if bound is None:
+            descs = _ghost_descs(_ghost_terms(owner), u, accum)
+            # plans are created with the kernel selection the environment asks for
+            skey = (julia_size(u), u.dtype, accum, u.device.index,
+                    os.environ.get("DOP_FORCE_GENERIC"), os.environ.get("DOP_TILE_VARIANT"),
+                    tuple(d[2] for d in descs))
+            bound = _Bound(skey, descs)
+        if bound.plans is None:
+            # a stream being captured admits neither allocations nor new plans: there the plans
+            # of any owner of this structure are taken (a live one then gets others on its next use)
+            capturing = torch.cuda.is_current_stream_capturing()
+            plans = _take_pooled(bound.skey, stream, capturing)
+            if plans is None and capturing:
+                other = next((b for b in _LIVE if b.skey == bound.skey and b.plans is not None), None)
+                if other is not None:
+                    plans, other.plans, other.stream = other.plans, None, None
+            if plans is None:
+                plans = [Plan(d, keep) for d, keep, _ in bound.descs]
+            else:
+                for i, (d, keep, _) in enumerate(bound.descs):
+                    try:
+                        plans[i].update(d, keep, stream)
+                    except _abi.DopError:
+                        # same kinds and sizes but a different row structure (e.g. coefficients
+                        # that are no longer uniform): a plan of its own
+                        plans[i] = Plan(d, keep)
+            bound.plans, bound.stream = plans, stream
+        _plan_cache(owner)[key] = bound
+        _LIVE.add(bound)
+    return bound
+
+
+_raw_stream = torch._C._cuda_getCurrentRawStream if hasattr(
+    torch._C, "_cuda_getCurrentRawStream") else lambda i: torch.cuda.current_stream(i).cuda_stream
+
+
+def _apply_bound(owner, du, u, accum=_abi.ACC_AUTO, accumulate=False):
+    """du (+)= owner * u; du and u are contiguous device tensors of one shape."""
+    if du.dtype is not u.dtype:
+        raise TypeError("tensor dtype does not match the plan's storage type")
+    dp, up = du.data_ptr(), u.data_ptr()
+    if dp == up:
+        raise ValueError("du must not alias u")
+    dev = u.device
+    stream = _raw_stream(dev.index)
+    key = (u.shape, u.dtype, dev, accum)
+    bound = owner._plans.get(key)
+    plans = None if bound is None else bound.plans
+    if plans is None:
+        bound = _bind(owner, key, u, accum, bound, stream)
+        plans = bound.plans
+    elif bound.stream != stream:
+        bound.stream = _MIXED
+    apply = _abi.lib().dop_apply
+    for p in plans:
+        rc = apply(p.handle, dp, up, 1 if accumulate else 0, stream)
+        if rc:
+            _abi.check(rc, "dop_apply")
+        accumulate = True
 
 
 def _ghost_terms(A):
@@ -371,15 +433,10 @@ def _ghost_terms(A):
     return None
 
 
-def _apply_plans(plans, du, u, accumulate):
-    for i, p in enumerate(plans):
-        p.apply(du, u, accumulate=(accumulate or i > 0))
-
-
 def ghost_times(G, u):
     _check_device_tensor(u, "u")
     out = torch.empty_like(u)
-    _apply_plans(ghost_plans(G, _ghost_terms(G), u, shared=True), out, u, False)
+    _apply_bound(G, out, u)
     return out
 
 
@@ -429,7 +486,7 @@ def combination_times(A: DiffEqOperatorCombination, x):
     terms = _ghost_terms(A)
     if terms is not None:
         out = torch.empty_like(x)
-        _apply_plans(ghost_plans(A, terms, x, shared=True), out, x, False)
+        _apply_bound(A, out, x)
         return out
     if all(isinstance(op, DerivativeOperator) for op in A.ops):
         shapes = set()
@@ -462,7 +519,7 @@ def mul_(du, A, u, overwrite=True, accum=_abi.ACC_AUTO):
     if terms is not None:
         if tuple(du.shape) != tuple(u.shape):
             raise AssertionError("du must have the unpadded size of u")
-        _apply_plans(ghost_plans(A, terms, u, accum, shared=True), du, u, accumulate)
+        _apply_bound(A, du, u, accum, accumulate)
         return du
     if isinstance(A, DerivativeOperator):
         # derivative_operator_functions.jl:18-69
