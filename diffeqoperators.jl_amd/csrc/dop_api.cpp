@@ -221,8 +221,9 @@ int dop_plan_create(const dop_desc* desc, dop_plan** out)
     const char* fg = std::getenv("DOP_FORCE_GENERIC");
     p->d.generic_only = (fg && fg[0] == '1') ? 1 : 0;
     if (!p->d.generic_only) dop::build_fast(H, &p->d.fast);
+    p->d.variant = dop::fast_default(p->d.fast);
     // DOP_TILE_VARIANT=v pins the tile-shape candidate; otherwise the tuning cache's choice
-    // for this shape, or 0 until the plan is tuned
+    // for this shape, or fast_default's until the plan is tuned
     if (const char* tv = std::getenv("DOP_TILE_VARIANT")) {
         const int v = std::atoi(tv);
         if (v >= 0 && v < dop::apply_variants(p->d)) p->d.variant = v;

@@ -284,4 +284,132 @@ DOP_HD inline double eval_point(const PlanDev& P, const T* src, const int64_t* i
     return acc.value();
 }
 
+// ---------------------------------------------------------------------------------------
+// The same value for points of the shell (boundary rows and their neighbours), written for
+// latency.  eval_point walks a chain of dependent reads -- the row's program, then its taps, then
+// its ghosts' taps, axis by axis -- and a thin shell has too few points to hide it: with four
+// points per thread in turn it took 19 us of a 1024^2 f32 apply (20.4 us per call; 6.9 with this
+// form, one point per thread) and of a 1001 x 1407 one (22.6; 9.2).  Here every axis first issues all that depends on the point
+// alone (row header, weights, ghost taps and their coefficients, the taps of regular rows),
+// then the taps of boundary rows, and only then sums, in eval_point's order and arithmetic (bitwise
+// equal).  Plans must meet shell_point_ok for KM.
+constexpr int kPointGhost = 2;   // ghost taps per end
+
+// Whether shell_point<.., KM> takes the plan: windows within its registers, one affine BC per
+// axis, and axes long enough that a row near one end reads no ghost of the other.  Structural
+// fields only: an update of the plan's values does not change the answer.
+DOP_HD inline bool shell_point_ok(const PlanDev& P, int KM)
+{
+    if (!P.ghost) return false;
+    for (int a = 0; a < P.ndim; ++a) {
+        const AxisDev& X = P.ax[a];
+        const int ends = X.rlo > X.n - X.rhi ? X.rlo : X.n - X.rhi;
+        if (!X.active || X.rhi <= X.rlo || X.K > KM || X.KB > KM + 1 || X.nl > kPointGhost ||
+            X.nr > kPointGhost || X.periodic || X.lbc || X.lstride[0] + X.lstride[1] + X.lstride[2] != 0 ||
+            X.n < 2 * ends + 2 * KM + 4)
+            return false;
+    }
+    return true;
+}
+
+template <typename T, int ACC, int KM, int ND>
+DOP_HD inline double shell_point(const PlanDev& P, const T* src, const int64_t* idx)
+{
+    using C = typename Store<T>::C;
+    using W = typename Acc<ACC>::W;
+    constexpr int KT = KM + 1;
+    double w[ND][KT];                 // the row's weights (f32 tables widened: exact)
+    C v[ND][KT];                      // its taps
+    double ga[ND][kPointGhost], gc[ND];
+    C gv[ND][kPointGhost];
+    int J0[ND], nt[ND], ng[ND];       // boundary rows: header, ghost taps (regular: nt = 0)
+#pragma unroll
+    for (int a = 0; a < ND; ++a) {
+        const AxisDev& X = P.ax[a];
+        int64_t base = P.tshift[a];
+#pragma unroll
+        for (int b = 0; b < ND; ++b)
+            if (b != a) base += idx[b] * P.ssrc[b];
+        const int64_t S = P.ssrc[a];
+        const int r = (int)idx[a];
+        if (r >= X.rlo && r < X.rhi) {
+            nt[a] = ng[a] = J0[a] = 0;
+            const W* wt = Acc<ACC>::table(X) + (X.uniform ? 0 : r);
+            const int64_t ws = X.uniform ? 1 : X.n;
+            const int64_t p0 = base + (int64_t)(r + X.dmin) * S;
+#pragma unroll
+            for (int k = 0; k < KM; ++k) {
+                if (k < X.K) {
+                    w[a][k] = (double)tab(wt, k * ws);
+                    v[a][k] = (C)Store<T>::ld(src, p0 + k * S);
+                }
+            }
+        } else {
+            const bool left = r < X.rlo;
+            const int b = left ? r : X.rlo + (r - X.rhi);
+            J0[a] = tab(X.bJ0, b);
+            nt[a] = tab(X.bn, b);
+            const double* wr = X.bw + (int64_t)b * X.KB;
+#pragma unroll
+            for (int k = 0; k < KT; ++k)
+                if (k < X.KB) w[a][k] = tab(wr, k);
+            ng[a] = left ? X.nl : X.nr;
+            const double* al = left ? X.al : X.ar;
+            const int64_t o = left ? 0 : (int64_t)X.n - X.nr;
+#pragma unroll
+            for (int k = 0; k < kPointGhost; ++k) {
+                if (k < ng[a]) {
+                    ga[a][k] = tab(al, k);
+                    gv[a][k] = (C)Store<T>::ld(src, base + (o + k) * S);
+                }
+            }
+            gc[a] = left ? tab(&X.bl, 0) : tab(&X.br, 0);
+        }
+    }
+    // the taps of boundary rows (a ghost's place is clamped to the line's end)
+#pragma unroll
+    for (int a = 0; a < ND; ++a) {
+        if (nt[a] == 0) continue;
+        const AxisDev& X = P.ax[a];
+        int64_t base = P.tshift[a];
+#pragma unroll
+        for (int b = 0; b < ND; ++b)
+            if (b != a) base += idx[b] * P.ssrc[b];
+#pragma unroll
+        for (int k = 0; k < KT; ++k) {
+            if (k < nt[a]) {
+                int j = J0[a] + k - 1;
+                j = j < 0 ? 0 : j >= X.n ? X.n - 1 : j;
+                v[a][k] = (C)Store<T>::ld(src, base + (int64_t)j * P.ssrc[a]);
+            }
+        }
+    }
+    Acc<ACC> acc;
+#pragma unroll
+    for (int a = 0; a < ND; ++a) {
+        const AxisDev& X = P.ax[a];
+        if (nt[a] == 0) {
+#pragma unroll
+            for (int k = 0; k < KM; ++k)
+                if (k < X.K) acc.add((W)w[a][k], (W)v[a][k]);
+        } else {
+            double g = 0.0;
+#pragma unroll
+            for (int k = 0; k < kPointGhost; ++k)
+                if (k < ng[a]) g = fma(ga[a][k], (double)gv[a][k], g);
+            g = g + gc[a];
+            double s = 0.0;
+#pragma unroll
+            for (int k = 0; k < KT; ++k) {
+                if (k < nt[a]) {
+                    const int J = J0[a] + k;
+                    s = fma(w[a][k], J == 0 || J == X.n + 1 ? g : (double)v[a][k], s);
+                }
+            }
+            acc.add_sum(s);
+        }
+    }
+    return acc.value();
+}
+
 }  // namespace dop

@@ -2,6 +2,8 @@
 // padded symmetric weights, shell decomposition and the tile-shape candidates.
 #include "dop_fast.hpp"
 
+#include "dop_eval.hpp"
+
 #include <algorithm>
 
 namespace dop {
@@ -12,6 +14,9 @@ constexpr int kMaxK2D = 13;
 constexpr int kMaxK3D = 9;   // 3-D stages 2*H halo rows through 8 waves: H <= 4
 
 int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
+
+// 2-D candidates of twice the points per lane: rows of at least two such segments
+bool wide_ok(const FastPlan& fp) { return fp.VX > 1 && fp.args.n[0] >= 256 * fp.VX; }
 
 int64_t shell_boxes(const PlanDev& P, const int32_t* lo, const int32_t* hi, ShellArgs* out)
 {
@@ -44,17 +49,19 @@ int64_t shell_boxes(const PlanDev& P, const int32_t* lo, const int32_t* hi, Shel
 
 // Whether a shell strip that touches x boundary rows finds every x tap and ghost it reads in
 // the kStripStage values at its end of the line (left rows: [0, kStripStage), right rows:
-// [n - kStripStage, n)): strips are kStripPts aligned, so their points lie below
-// roundup(rlo) + kStripPts or at or above rhi - kStripPts.
-bool strips_stage_ok(const PlanDev& P, const AxisTables& T)
+// [n - kStripStage, n)): strips start at multiples of kStripPts, so their points lie below
+// roundup(rlo) + kStripPts or at or above rhi - kStripPts; those of the x sides of the box lie
+// below lo or at or above hi.
+bool strips_stage_ok(const PlanDev& P, const AxisTables& T, int lo, int hi)
 {
     const AxisDev& X = P.ax[0];
     const int n = (int)P.n[0];
-    if (!P.ghost || !X.active || n < 2 * kStripStage || n % kStripPts != 0 || X.periodic) return false;
+    if (!P.ghost || !X.active || n < 2 * kStripStage || X.periodic) return false;
     for (size_t l = 0; l < T.lbc.size(); l += kLineBC)
         if (T.lbc[l] < 0.0) return false;   // a periodic line reads the far end
-    const int lend = std::min(n, (X.rlo + kStripPts - 1) / kStripPts * kStripPts + kStripPts);
-    const int rbeg = std::max(0, X.rhi - kStripPts);
+    const int lend = std::min(n, std::max(lo, (X.rlo + kStripPts - 1) / kStripPts * kStripPts + kStripPts));
+    const int rbeg = std::min(hi, std::max(0, X.rhi - kStripPts));
+    if (lend > n / 2 || rbeg < n / 2) return false;
     auto within = [&](int r, int j) {
         return r < lend ? (j >= 0 && j < kStripStage) : (j >= n - kStripStage && j < n);
     };
@@ -95,18 +102,17 @@ bool build_strips(const PlanDev& P, const HostPlan& H, const int32_t* lo, const 
     S = StripArgs{};
     const int32_t n[3] = {(int32_t)P.n[0], (int32_t)P.n[1], (int32_t)P.n[2]};
     const AxisDev& X0 = P.ax[0];
-    // every item starts a 16-byte group of u and du (inside the array) when n0, the row and
-    // plane strides, the transverse shifts and the x edges of the box are multiples of 4
-    bool al = n[0] % kStripPts == 0 && lo[0] % kStripPts == 0 && hi[0] % kStripPts == 0;
-    for (int a = 1; a < 3; ++a) al = al && P.ssrc[a] % kStripPts == 0 && P.sdu[a] % kStripPts == 0;
-    for (int a = 0; a < 3; ++a) al = al && P.tshift[a] % kStripPts == 0;
-    S.vec_ok = al ? 1 : 0;
-    S.stage_ok = strips_stage_ok(P, H.axis[0]) ? 1 : 0;
+    // items start at multiples of 4 along x and load groups of four values (element-aligned, so
+    // the rows may have any length; the last item of a ragged row is narrower)
+    S.vec_ok = lo[0] % kStripPts == 0 && hi[0] % kStripPts == 0 && n[0] >= kStripStage ? 1 : 0;
+    S.stage_ok = strips_stage_ok(P, H.axis[0], lo[0], hi[0]) ? 1 : 0;
     // x strips of four regular rows
     const int32_t ax = (X0.rlo + kStripPts - 1) / kStripPts * kStripPts;
     const int32_t bx = X0.rhi / kStripPts * kStripPts;
     const bool faces = S.vec_ok && n[0] >= kStripStage && ax < bx;
-    const bool face[3] = {faces && S.stage_ok && !X0.lbc, faces && !P.ax[1].lbc, faces && !P.ax[2].lbc};
+    // (a face's items share one BC; H.meta's own lbc pointers are set at upload)
+    const bool face[3] = {faces && S.stage_ok && H.axis[0].lbc.empty(),
+                          faces && H.axis[1].lbc.empty(), faces && H.axis[2].lbc.empty()};
 
     int nbox = 0;
     auto add_seg = [&](int kind, int r0, int nr, int xend, int64_t items) {
@@ -220,18 +226,29 @@ void build_fast(const HostPlan& H, FastPlan* fp)
         fp->nat_lo[a] = A.lo[a];
         fp->nat_hi[a] = A.hi[a];
     }
-    // points per lane: 16-byte lane loads when rows stay aligned
+    // points per lane: 16-byte lane loads (element-aligned, so rows of any length) except in
+    // rows too short to hold a box aligned to them
     const int vx_native = (P.storage == kF64) ? 2 : 4;
     fp->f64 = P.storage == kF64;
-    fp->VX = (P.n[0] % vx_native == 0) ? vx_native : 1;
-    if (P.ndim >= 2) {
-        // lanes store whole VX groups: the box's x edges are aligned to the widest VX of the
-        // tile variants (the few columns this moves into the shell are evaluated there)
-        const int al = (P.ndim == 2 && fp->VX > 1 && P.n[0] % (2 * fp->VX) == 0) ? 2 * fp->VX : fp->VX;
-        A.lo[0] = (int)ceil_div(A.lo[0], al) * al;
-        A.hi[0] = A.hi[0] / al * al;
-        if (A.hi[0] <= A.lo[0]) return;
+    fp->VX = P.n[0] >= 2 * kStripStage ? vx_native : 1;
+    // Lanes load and store whole groups of VX points at multiples of VX, so the box's x edges
+    // are multiples of the widest group, with room for the halo groups beside it (the few
+    // columns this moves into the shell are evaluated there).
+    if (P.ndim >= 2 && fp->VX > 1) {
+        const int al = P.ndim == 3 ? kStripPts : wide_ok(*fp) ? 2 * fp->VX : fp->VX;
+        const int pad = (int)ceil_div(half, al) * al;
+        const int lo = (int)ceil_div(A.lo[0], al) * al;
+        const int hi = (int)std::min<int64_t>(A.hi[0], P.n[0] - pad) / al * al;
+        if (hi > lo) {
+            A.lo[0] = lo;
+            A.hi[0] = hi;
+        } else {
+            fp->VX = 1;
+        }
     }
+    fp->args.pfast = shell_point_ok(P, K);
+    for (int a = 0; a < P.ndim; ++a)
+        if (!H.axis[a].lbc.empty()) fp->args.pfast = 0;
     // padded weights (rows outside the natural box are zero).  The tiled kernels index every axis
     // per row unless all axes are uniform, so a uniform axis of a mixed plan is expanded to
     // one row per point.
@@ -260,27 +277,15 @@ void build_fast(const HostPlan& H, FastPlan* fp)
     fp->kind = P.ndim;
 }
 
-// Candidates (autotuner).  2-D: chunk height {32,16,64,8} x prefetch {2,4} ({4,8}, FP64 {8,16} edge-loaded) x XCD remap x
-// points per lane {widest 16-byte, twice that} x marches {all downwards, alternating} x
-// segments {overlapping, edge-loaded (when the x half-width is at most the points per lane)}; 3-D:
-// chunk depth {64,32} x block shape (waves, rows per wave) {(8,1), (16,1), (8,2), (16,2),
-// (8,3)} x XCD remap x points per lane {widest, half}, then the edge-loaded forms.  A block
-// stages waves * rows y rows and computes all but the 2H halo rows.
-namespace {
-bool wide_ok(const FastPlan& fp) { return fp.VX > 1 && fp.args.n[0] % (2 * fp.VX) == 0; }
-// 2-D edge-loaded segments: one edge group per side at the narrowest points per lane
-bool edge2_ok(const FastPlan& fp) { return fp.args.K / 2 <= fp.VX; }
-int base2_count(const FastPlan& fp) { return wide_ok(fp) ? 64 : 32; }
-
-int gen1_count(const FastPlan& fp) { return fp.VX > 1 ? 40 : 20; }
-int gen2_count(const FastPlan& fp) { return fp.VX > 1 ? 32 : 16; }
-}  // namespace
-
+// Candidates (autotuner).  2-D: chunk height {32,16,64,8} x prefetch {4,8} (FP64 {8,16};
+// overlapping segments {2,4}) x XCD remap x marches {all downwards, alternating} x points per
+// lane {widest 16-byte, twice that}.  Segments are edge-loaded where the x half-width is at most
+// the points per lane, overlapping otherwise.  3-D (edge-loaded): chunk depth {64,32,16} x block
+// shape (waves, rows per wave) {(8,1),(8,2),(8,3)} x XCD remap x points per lane {widest, half}.
 int fast_variant_count(const FastPlan& fp)
 {
-    if (fp.kind == 1) return 1;
-    if (fp.kind == 2) return base2_count(fp) * (edge2_ok(fp) ? 2 : 1);
-    if (fp.kind == 3) return gen1_count(fp) + gen2_count(fp);
+    if (fp.kind == 2) return wide_ok(fp) ? 64 : 32;
+    if (fp.kind == 3) return fp.VX > 1 ? 36 : 18;
     return 1;
 }
 
@@ -288,19 +293,16 @@ bool fast_variant(const FastPlan& fp, int v, FastArgs* out)
 {
     if (fp.kind < 2 || v < 0 || v >= fast_variant_count(fp)) return false;
     FastArgs A = fp.args;
-    A.gen = 1;
-    if (fp.kind == 3 && v >= gen1_count(fp)) {
-        // edge-loaded segments: chunk depth {64,32} x block shape (waves, rows per wave)
-        // {(8,1),(8,2),(16,1),(8,3)} x XCD remap x points per lane {widest, half}
-        const int w = v - gen1_count(fp);
+    A.xcd_remap = (v & 1) ? 0 : 1;
+    if (fp.kind == 3) {
+        static const int shapes[3][2] = {{8, 2}, {8, 1}, {8, 3}};
+        static const int chunks[3] = {32, 64, 16};
+        const int w = v >> 1;
+        A.W = shapes[w % 3][0];
+        A.VY = shapes[w % 3][1];
+        A.chunk = chunks[(w / 3) % 3];
+        A.VX = w / 9 ? fp.VX / 2 : fp.VX;
         A.gen = 2;
-        A.xcd_remap = (w & 1) ? 0 : 1;
-        static const int chunks[2] = {64, 32};
-        A.chunk = chunks[(w >> 1) & 1];
-        static const int shapes[4][2] = {{8, 1}, {8, 2}, {16, 1}, {8, 3}};
-        A.W = shapes[(w >> 2) & 3][0];
-        A.VY = shapes[(w >> 2) & 3][1];
-        A.VX = (w >> 4) ? fp.VX / 2 : fp.VX;
         A.PF = 1;
         A.xbase = A.lo[0];
         A.nxseg = (int)ceil_div(A.hi[0] - A.lo[0], 64 * A.VX);
@@ -310,36 +312,19 @@ bool fast_variant(const FastPlan& fp, int v, FastArgs* out)
         *out = A;
         return true;
     }
-    if (fp.kind == 2 && v >= base2_count(fp)) {
-        A.gen = 2;
-        v -= base2_count(fp);
-    }
-    A.xcd_remap = (v & 1) ? 0 : 1;
-    if (fp.kind == 2) {
-        static const int chunks[4] = {32, 16, 64, 8};
-        A.chunk = chunks[(v >> 1) & 3];
-        // edge-loaded rings carry H edge values per row, so they afford deeper prefetch (FP64
-        // rows of 2 points per lane: 8 or 16 rows; 4 or 8 otherwise)
-        const bool f64 = fp.f64 != 0;
-        A.PF = A.gen == 2 ? (((v >> 3) & 1) ? (f64 ? 16 : 8) : (f64 ? 8 : 4))
-                          : (((v >> 3) & 1) ? 4 : 2);
-        // bit 4: twice the points per lane (when rows allow), next bit: alternating marches
-        const bool wide = wide_ok(fp);
-        A.VX = (wide && ((v >> 4) & 1)) ? 2 * fp.VX : fp.VX;
-        A.alt = (v >> (wide ? 5 : 4)) & 1;
-        A.W = 4;
-        A.VY = 1;
-    } else {
-        static const int chunks[2] = {64, 32};
-        A.chunk = chunks[(v >> 1) & 1];
-        A.PF = 1;
-        static const int shapes[5][2] = {{8, 1}, {16, 1}, {8, 2}, {16, 2}, {8, 3}};
-        const int sh = (v >> 2) % 5;
-        A.W = shapes[sh][0];
-        A.VY = shapes[sh][1];
-        if (A.VY == 1 && 2 * (A.K / 2) >= 8) A.W = 16;   // a block must compute some rows
-        A.VX = ((v >> 2) / 5) ? fp.VX / 2 : fp.VX;
-    }
+    static const int chunks[4] = {32, 16, 64, 8};
+    A.chunk = chunks[(v >> 1) & 3];
+    A.alt = (v >> 4) & 1;
+    A.VX = ((v >> 5) & 1) ? 2 * fp.VX : fp.VX;
+    A.W = 4;
+    A.VY = 1;
+    A.nyblk = 0;
+    const int H = A.K / 2;
+    A.gen = H <= A.VX ? 2 : 1;
+    // edge-loaded rings carry H edge values per row and afford deeper prefetch (FP64 rows of 2
+    // points per lane: 8 or 16 rows; 4 or 8 otherwise)
+    const bool deep = (v >> 3) & 1;
+    A.PF = A.gen == 2 ? (fp.f64 ? (deep ? 16 : 8) : (deep ? 8 : 4)) : (deep ? 4 : 2);
     if (A.gen == 2) {
         // segments of 64*VX points at multiples of 64*VX, not overlapping
         const int seg = 64 * A.VX;
@@ -347,25 +332,33 @@ bool fast_variant(const FastPlan& fp, int v, FastArgs* out)
         A.nxseg = (int)ceil_div(A.hi[0] - A.xbase, seg);
     } else {
         // segments of 64*VX points overlapping by 2*PADL (the x halo, whole lanes)
-        const int H = A.K / 2;
         const int padl = (H + A.VX - 1) / A.VX * A.VX;
         A.xbase = A.lo[0] - padl;
         A.nxseg = (int)ceil_div(A.hi[0] - A.lo[0], 64 * A.VX - 2 * padl);
     }
-    if (fp.kind == 2) {
-        A.gx = (int)ceil_div(A.nxseg, 4);
-        const int64_t nch = ceil_div(A.hi[1] - A.lo[1], A.chunk);
-        A.nyblk = 0;
-        A.nblocks = (int)(A.gx * nch);
-    } else {
-        // W waves stage W rows and compute the middle W - 2H
-        A.nyblk = (int)ceil_div(A.hi[1] - A.lo[1], A.W * A.VY - 2 * (A.K / 2));
-        const int64_t nzc = ceil_div(A.hi[2] - A.lo[2], A.chunk);
-        A.gx = 0;
-        A.nblocks = (int)(A.nxseg * A.nyblk * nzc);
-    }
+    A.gx = (int)ceil_div(A.nxseg, 4);
+    A.nblocks = (int)(A.gx * ceil_div(A.hi[1] - A.lo[1], A.chunk));
     *out = A;
     return true;
+}
+
+int fast_default(const FastPlan& fp)
+{
+    if (fp.kind < 2) return 0;
+    // the order of preference with plenty of points; the first that gives every CU two blocks
+    // (four waves of a 2-D block, eight of a 3-D one) is taken, else the one of most blocks
+    static const int v2[4] = {4, 0, 2, 6};                    // 2-D chunks 64, 32, 16, 8
+    static const int w3[3] = {0, 6, 7};                       // 3-D (8,2)x32, (8,2)x16, (8,1)x16
+    const bool half = fp.kind == 3 && fp.VX > 1 && fp.args.hi[0] - fp.args.lo[0] <= 32 * fp.VX;
+    const int nc = fp.kind == 2 ? 4 : 3;
+    int v = 0;
+    for (int c = 0; c < nc; ++c) {
+        v = fp.kind == 2 ? v2[c] : 2 * (w3[c] + (half ? 9 : 0));
+        FastArgs A;
+        if (!fast_variant(fp, v, &A)) return 0;
+        if (A.nblocks >= 512) break;
+    }
+    return v;
 }
 
 }  // namespace dop

@@ -46,7 +46,7 @@ struct StripArgs {
     int32_t nblocks;                 // blocks of the launch
     int32_t nfirst;                  // blocks of the leading kind-4 segments (taken in hardware
                                      // order; the rest XCD-contiguous)
-    int32_t vec_ok;                  // every item starts an aligned group of 4 values of u and du
+    int32_t vec_ok;                  // items start at multiples of 4 along x (groups of 4 values)
     int32_t stage_ok;                // every x tap and ghost of a strip touching x boundary rows
                                      // lies in the kStripStage values at its end of the line
     ShellSeg seg[kMaxShellSegs];
@@ -85,9 +85,10 @@ struct FastArgs {
     int32_t gx;            // 2-D: blocks across x (4 segments each)
     int32_t nblocks;
     int32_t xcd_remap;     // keep neighbouring tiles on one XCD
-    int32_t gen;           // 1 overlapping segments (x halo from the segment's own end lanes),
-                           // 2 edge-loaded segments (3-D: k_tiled3e; 2-D: k_tiled2d's EDG form)
+    int32_t gen;           // 2-D: 1 overlapping segments (x halo from the segment's own end
+                           // lanes), 2 edge-loaded segments (k_tiled2d's EDG form; 3-D always)
     int32_t alt;           // 2-D: odd row chunks march upwards (towards their neighbours)
+    int32_t pfast;         // shell points may use shell_point<.., K> (shell_point_ok)
     int32_t uniform[3];    // weights identical for every row of the axis
     const double* w64[3];  // [uniform ? 1 : n][K]
     const float* w32[3];
@@ -96,7 +97,7 @@ struct FastArgs {
 struct FastPlan {
     int kind = 0;          // 0: generic only, 1: 1-D window tables only (batched tiles),
                            // 2: 2-D tiled, 3: 3-D tiled
-    int VX = 1;            // widest points-per-lane the row alignment allows
+    int VX = 1;            // points per lane of a 16-byte load (1: rows too short)
     int f64 = 0;           // FP64 storage
     int kahan = 0;         // Dot2-compensated f32 accumulation: batched tiles only
     FastArgs args{};
@@ -119,5 +120,7 @@ void build_fast(const HostPlan& H, FastPlan* fp);
 // not a valid variant.
 bool fast_variant(const FastPlan& fp, int v, FastArgs* out);
 int fast_variant_count(const FastPlan& fp);
+// The variant of a plan that is not tuned (fewer than 2^20 points, or before its first apply).
+int fast_default(const FastPlan& fp);
 
 }  // namespace dop

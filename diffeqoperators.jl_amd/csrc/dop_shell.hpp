@@ -18,12 +18,13 @@ constexpr int kShellBlock = kStripBlock;
 // Weights (plan tables, global memory): w (<= 4) consecutive values, one 16-byte load (f32)
 // or two (f64) when `vec` (then the whole aligned group of 4 is loaded).
 struct VecW {
-    typedef float f4 __attribute__((ext_vector_type(4)));
-    typedef double d2 __attribute__((ext_vector_type(2)));
+    typedef float f4 __attribute__((ext_vector_type(4), aligned(4)));
+    typedef double d2 __attribute__((ext_vector_type(2), aligned(8)));
+    typedef uint32_t b4 __attribute__((ext_vector_type(2), aligned(2)));
     __device__ static void ldw(const float* p, int w, bool vec, float* o)
     {
         if (vec) {
-            const f4 v = tab(reinterpret_cast<const f4*>(p), 0);
+            const f4 v = *(const __attribute__((address_space(1))) f4*)p;
             o[0] = v.x; o[1] = v.y; o[2] = v.z; o[3] = v.w;
             return;
         }
@@ -33,8 +34,8 @@ struct VecW {
     __device__ static void ldw(const double* p, int w, bool vec, double* o)
     {
         if (vec) {
-            const d2 a = tab(reinterpret_cast<const d2*>(p), 0);
-            const d2 b = tab(reinterpret_cast<const d2*>(p), 1);
+            const d2 a = *(const __attribute__((address_space(1))) d2*)p;
+            const d2 b = *(const __attribute__((address_space(1))) d2*)(p + 2);
             o[0] = a.x; o[1] = a.y; o[2] = b.x; o[3] = b.y;
             return;
         }
@@ -43,8 +44,8 @@ struct VecW {
     }
 };
 
-// w (<= 4) consecutive values at p, as C: when `vec` the aligned group of 4 starting at p in
-// one vector load (16 bytes f32, two 16-byte loads f64, 8 bytes bf16), one load per value
+// w (<= 4) consecutive values at p, as C: when `vec` the group of 4 starting at p in one
+// (element-aligned) vector load (16 bytes f32, two 16-byte loads f64, 8 bytes bf16), one load per value
 // otherwise; st stores a whole group with one vector store when `vec` and w == 4
 template <typename T>
 struct VecLoad;
@@ -54,7 +55,7 @@ struct VecLoad<float> : VecW {
     __device__ static void ld(const float* p, int w, bool vec, float* o)
     {
         if (vec) {
-            const float4 v = *reinterpret_cast<const float4*>(p);
+            const f4 v = *reinterpret_cast<const f4*>(p);
             o[0] = v.x; o[1] = v.y; o[2] = v.z; o[3] = v.w;
             return;
         }
@@ -64,7 +65,7 @@ struct VecLoad<float> : VecW {
     __device__ static void st(float* p, int w, bool vec, const double* v)
     {
         if (vec && w == 4) {
-            *reinterpret_cast<float4*>(p) = make_float4((float)v[0], (float)v[1], (float)v[2], (float)v[3]);
+            *reinterpret_cast<f4*>(p) = f4{(float)v[0], (float)v[1], (float)v[2], (float)v[3]};
             return;
         }
 #pragma unroll
@@ -78,8 +79,8 @@ struct VecLoad<double> : VecW {
     __device__ static void ld(const double* p, int w, bool vec, double* o)
     {
         if (vec) {
-            const double2 a = *reinterpret_cast<const double2*>(p);
-            const double2 b = *reinterpret_cast<const double2*>(p + 2);
+            const d2 a = *reinterpret_cast<const d2*>(p);
+            const d2 b = *reinterpret_cast<const d2*>(p + 2);
             o[0] = a.x; o[1] = a.y; o[2] = b.x; o[3] = b.y;
             return;
         }
@@ -89,8 +90,8 @@ struct VecLoad<double> : VecW {
     __device__ static void st(double* p, int w, bool vec, const double* v)
     {
         if (vec && w == 4) {
-            *reinterpret_cast<double2*>(p) = make_double2(v[0], v[1]);
-            *reinterpret_cast<double2*>(p + 2) = make_double2(v[2], v[3]);
+            *reinterpret_cast<d2*>(p) = d2{v[0], v[1]};
+            *reinterpret_cast<d2*>(p + 2) = d2{v[2], v[3]};
             return;
         }
 #pragma unroll
@@ -104,7 +105,7 @@ struct VecLoad<bf16> : VecW {
     __device__ static void ld(const bf16* p, int w, bool vec, float* o)
     {
         if (vec) {
-            const uint2 v = *reinterpret_cast<const uint2*>(p);
+            const b4 v = *reinterpret_cast<const b4*>(p);
             o[0] = __builtin_bit_cast(float, v.x << 16);
             o[1] = __builtin_bit_cast(float, v.x & 0xffff0000u);
             o[2] = __builtin_bit_cast(float, v.y << 16);
@@ -117,10 +118,10 @@ struct VecLoad<bf16> : VecW {
     __device__ static void st(bf16* p, int w, bool vec, const double* v)
     {
         if (vec && w == 4) {
-            uint2 o;
+            b4 o;
             o.x = (uint32_t)f32_to_bf16((float)v[0]) | ((uint32_t)f32_to_bf16((float)v[1]) << 16);
             o.y = (uint32_t)f32_to_bf16((float)v[2]) | ((uint32_t)f32_to_bf16((float)v[3]) << 16);
-            *reinterpret_cast<uint2*>(p) = o;
+            *reinterpret_cast<b4*>(p) = o;
             return;
         }
 #pragma unroll
@@ -168,6 +169,7 @@ __device__ inline void xface_tile(const PlanDev& P, const StripArgs& SA, const S
     const int x0 = G.r0;
     const int w = min(kSW, G.xend - x0);
     const int g0 = x0 < n0 / 2 ? 0 : n0 - kStage;
+    const int xl = min(x0, n0 - kSW), sh = x0 - xl;   // the strip's group, kept in the row
     const int64_t s1 = P.ssrc[1], s2 = P.ssrc[2];
     const int64_t xb = P.tshift[0] + g0;
     // the strip's group of every line of the tile and border
@@ -175,7 +177,7 @@ __device__ inline void xface_tile(const PlanDev& P, const StripArgs& SA, const S
         const int yy = min(max(yb - kXfHalo + g % EL, 0), n1 - 1);
         const int zz = min(max(zb - kXfHalo + g / EL, 0), n2 - 1);
         C v[kSW];
-        LD::ld(src + xb + (x0 - g0) + yy * s1 + zz * s2, kSW, true, v);
+        LD::ld(src + xb + (xl - g0) + yy * s1 + zz * s2, kSW, true, v);
 #pragma unroll
         for (int i = 0; i < kSW; ++i) Store<T>::st(grp[g], i, (double)v[i]);
     }
@@ -213,7 +215,7 @@ __device__ inline void xface_tile(const PlanDev& P, const StripArgs& SA, const S
                 wv[k] = tab(wt, k * ws);
                 const int L = self + (X.dmin + k) * step;
 #pragma unroll
-                for (int i = 0; i < kSW; ++i) xv[k][i] = (C)Store<T>::ld(grp[L], i);
+                for (int i = 0; i < kSW; ++i) xv[k][i] = (C)Store<T>::ld(grp[L], min(i + sh, kSW - 1));
             }
         }
 #pragma unroll
@@ -228,7 +230,7 @@ __device__ inline void xface_tile(const PlanDev& P, const StripArgs& SA, const S
     regular(X1, y, 1);
     regular(X2, z, EL);
     const int64_t idx[3] = {x0, y, z};
-    strip::store_item<T, ACC, LD>(P, idx, w, true, acc, du, accumulate);
+    strip::store_item<T, ACC, LD>(P, idx, w, sh == 0, acc, du, accumulate);
 }
 
 template <typename T, int ACC, int KM, bool VEC>

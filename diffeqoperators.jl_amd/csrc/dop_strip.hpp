@@ -374,9 +374,9 @@ DOP_HD inline void store_item(const PlanDev& P, const int64_t* idx, int w, bool 
 // One general item (strip l of box b of SA): its points' values written to du.  `stage` holds
 // kStage values and `slots` kSW accumulators of this thread (LDS on the device); LD loads up
 // to kSW consecutive values.  KM >= the window of every regular row (the tiles' window).  VEC:
-// SA.vec_ok (every item starts a 16-byte group of u and du that lies in the array, so whole
-// groups are loaded even for items of fewer than 4 points).  Plans with ghost-point input only
-// (the tiled path's condition).
+// SA.vec_ok (items start at multiples of 4, so whole groups are loaded, also for items of fewer
+// than 4 points, unless the group would leave the row).  Plans with ghost-point input only (the
+// tiled path's condition).
 template <typename T, int ACC, int KM, bool VEC, typename LD>
 DOP_HD inline void eval_strip(const PlanDev& P, const StripArgs& SA, int b, int l, T* stage,
                               Slot<ACC>* slots, T* __restrict__ du, const T* __restrict__ src,
@@ -399,7 +399,7 @@ DOP_HD inline void eval_strip(const PlanDev& P, const StripArgs& SA, int b, int 
     }
     const int64_t wl = SA.org[b][0] + SA.ext[b][0] - idx[0];
     const int w = wl < kSW ? (int)wl : kSW;
-    constexpr bool vec = VEC;
+    const bool vec = VEC && idx[0] + kSW <= P.n[0];   // a whole group lies in the row
     Acc<ACC> acc[kSW];
 
     // x term
@@ -464,6 +464,7 @@ DOP_HD inline void eval_face(const PlanDev& P, const StripArgs& SA, int row, int
         idx[2] = SA.flo[0][1] + v;
         w = xend - row < kSW ? xend - row : kSW;
     }
+    const bool vec = A != 0 || row + kSW <= (int)P.n[0];   // a whole group lies in the row
     Acc<ACC> acc[kSW];
     const AxisDev& X0 = P.ax[0];
     const AxisDev& X1 = P.ax[1];
@@ -481,10 +482,10 @@ DOP_HD inline void eval_face(const PlanDev& P, const StripArgs& SA, int row, int
     const int64_t b1 = P.tshift[1] + idx[0] * P.ssrc[0] + idx[2] * P.ssrc[2];
     const int64_t b2 = P.tshift[2] + idx[0] * P.ssrc[0] + idx[1] * P.ssrc[1];
     if constexpr (A == 1) strip_boundary_or_regular<T, ACC, KM, LD>(X1, src, row, b1, P.ssrc[1], w, acc);
-    else strip_regular<T, ACC, KM, LD>(X1, src, (int)idx[1], b1, P.ssrc[1], w, true, acc);
+    else strip_regular<T, ACC, KM, LD>(X1, src, (int)idx[1], b1, P.ssrc[1], w, vec, acc);
     if constexpr (A == 2) strip_boundary_or_regular<T, ACC, KM, LD>(X2, src, row, b2, P.ssrc[2], w, acc);
-    else strip_regular<T, ACC, KM, LD>(X2, src, (int)idx[2], b2, P.ssrc[2], w, true, acc);
-    store_item<T, ACC, LD>(P, idx, w, true, acc, du, accumulate);
+    else strip_regular<T, ACC, KM, LD>(X2, src, (int)idx[2], b2, P.ssrc[2], w, vec, acc);
+    store_item<T, ACC, LD>(P, idx, w, vec, acc, du, accumulate);
 }
 
 // Work item `l` of row j of segment `s`: the kernel's (and the CPU check's) dispatch.

@@ -37,17 +37,27 @@ namespace tiled {
 template <typename T, int VX>
 struct VecIO;
 
+// (element-aligned: rows of any length start lanes anywhere; a wave's loads of one row stay
+// contiguous, so a misaligned row costs one more cache line per wave, where the form of one point
+// per lane it replaces took four times the memory instructions)
+typedef double Vd2 __attribute__((ext_vector_type(2), aligned(8)));
+typedef float Vf4 __attribute__((ext_vector_type(4), aligned(4)));
+typedef float Vf2 __attribute__((ext_vector_type(2), aligned(4)));
+typedef uint32_t Vb2 __attribute__((aligned(2)));
+typedef uint32_t Vb4 __attribute__((ext_vector_type(2), aligned(2)));
+typedef uint32_t Vb8 __attribute__((ext_vector_type(4), aligned(2)));
+
 template <>
 struct VecIO<double, 2> {
     __device__ static void ld(const double* p, double* o)
     {
-        const double2 v = *reinterpret_cast<const double2*>(p);
+        const Vd2 v = *reinterpret_cast<const Vd2*>(p);
         o[0] = v.x;
         o[1] = v.y;
     }
     __device__ static void st(double* p, const double* v)
     {
-        *reinterpret_cast<double2*>(p) = make_double2(v[0], v[1]);
+        *reinterpret_cast<Vd2*>(p) = Vd2{v[0], v[1]};
     }
 };
 
@@ -55,7 +65,7 @@ template <>
 struct VecIO<float, 4> {
     __device__ static void ld(const float* p, float* o)
     {
-        const float4 v = *reinterpret_cast<const float4*>(p);
+        const Vf4 v = *reinterpret_cast<const Vf4*>(p);
         o[0] = v.x;
         o[1] = v.y;
         o[2] = v.z;
@@ -63,7 +73,7 @@ struct VecIO<float, 4> {
     }
     __device__ static void st(float* p, const float* v)
     {
-        *reinterpret_cast<float4*>(p) = make_float4(v[0], v[1], v[2], v[3]);
+        *reinterpret_cast<Vf4*>(p) = Vf4{v[0], v[1], v[2], v[3]};
     }
 };
 
@@ -71,13 +81,13 @@ template <>
 struct VecIO<float, 2> {
     __device__ static void ld(const float* p, float* o)
     {
-        const float2 v = *reinterpret_cast<const float2*>(p);
+        const Vf2 v = *reinterpret_cast<const Vf2*>(p);
         o[0] = v.x;
         o[1] = v.y;
     }
     __device__ static void st(float* p, const float* v)
     {
-        *reinterpret_cast<float2*>(p) = make_float2(v[0], v[1]);
+        *reinterpret_cast<Vf2*>(p) = Vf2{v[0], v[1]};
     }
 };
 
@@ -85,13 +95,13 @@ template <>
 struct VecIO<bf16, 2> {
     __device__ static void ld(const bf16* p, float* o)
     {
-        const uint32_t v = *reinterpret_cast<const uint32_t*>(p);
+        const uint32_t v = *reinterpret_cast<const Vb2*>(p);
         o[0] = __builtin_bit_cast(float, v << 16);
         o[1] = __builtin_bit_cast(float, v & 0xffff0000u);
     }
     __device__ static void st(bf16* p, const float* v)
     {
-        *reinterpret_cast<uint32_t*>(p) =
+        *reinterpret_cast<Vb2*>(p) =
             (uint32_t)f32_to_bf16(v[0]) | ((uint32_t)f32_to_bf16(v[1]) << 16);
     }
 };
@@ -100,7 +110,7 @@ template <>
 struct VecIO<bf16, 4> {
     __device__ static void ld(const bf16* p, float* o)
     {
-        const uint2 v = *reinterpret_cast<const uint2*>(p);
+        const Vb4 v = *reinterpret_cast<const Vb4*>(p);
         o[0] = __builtin_bit_cast(float, v.x << 16);
         o[1] = __builtin_bit_cast(float, v.x & 0xffff0000u);
         o[2] = __builtin_bit_cast(float, v.y << 16);
@@ -108,10 +118,10 @@ struct VecIO<bf16, 4> {
     }
     __device__ static void st(bf16* p, const float* v)
     {
-        uint2 w;
+        Vb4 w;
         w.x = (uint32_t)f32_to_bf16(v[0]) | ((uint32_t)f32_to_bf16(v[1]) << 16);
         w.y = (uint32_t)f32_to_bf16(v[2]) | ((uint32_t)f32_to_bf16(v[3]) << 16);
-        *reinterpret_cast<uint2*>(p) = w;
+        *reinterpret_cast<Vb4*>(p) = w;
     }
 };
 
@@ -148,7 +158,7 @@ template <>
 struct VecIO<bf16, 8> {
     __device__ static void ld(const bf16* p, float* o)
     {
-        const uint4 v = *reinterpret_cast<const uint4*>(p);
+        const Vb8 v = *reinterpret_cast<const Vb8*>(p);
         const uint32_t w[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
@@ -162,7 +172,7 @@ struct VecIO<bf16, 8> {
 #pragma unroll
         for (int i = 0; i < 4; ++i)
             w[i] = (uint32_t)f32_to_bf16(v[2 * i]) | ((uint32_t)f32_to_bf16(v[2 * i + 1]) << 16);
-        *reinterpret_cast<uint4*>(p) = make_uint4(w[0], w[1], w[2], w[3]);
+        *reinterpret_cast<Vb8*>(p) = Vb8{w[0], w[1], w[2], w[3]};
     }
 };
 
@@ -282,11 +292,12 @@ __device__ inline int tile_of(int b, int nb, int remap)
 template <typename T>
 constexpr int acc_of() { return std::is_same<T, double>::value ? kAccF64 : kAccF32; }
 
-// generic evaluation of shell points [first, first + count)
-template <typename T, int ACC>
-__device__ inline void shell_points(const PlanDev& P, const ShellArgs& S, T* __restrict__ du,
-                                    const T* __restrict__ src, int accumulate, int64_t first,
-                                    int64_t count)
+// shell points [first, first + count): shell_point where the plan allows it, else the generic
+// evaluation (the same values)
+template <typename T, int ACC, int K>
+__device__ inline void shell_points(const PlanDev& P, const ShellArgs& S, int pfast,
+                                    T* __restrict__ du, const T* __restrict__ src, int accumulate,
+                                    int64_t first, int64_t count)
 {
     const int64_t total = S.start[S.nbox];
     const int64_t end = min(first + count, total);
@@ -310,13 +321,15 @@ __device__ inline void shell_points(const PlanDev& P, const ShellArgs& S, T* __r
             idx[2] = S.org[b][2] + l / e1;
         }
         const int64_t lin = idx[0] + idx[1] * P.sdu[1] + idx[2] * P.sdu[2];
-        double v = eval_point<T, ACC>(P, src, idx);
+        double v = pfast ? shell_point<T, ACC, K, 2>(P, src, idx) : eval_point<T, ACC>(P, src, idx);
         if (accumulate) v += (double)Store<T>::ld(du, lin);
         Store<T>::st(du, lin, v);
     }
 }
 
-constexpr int kShellPtsPerThread = 4;
+// one point per thread: the shell is a thin rim, and a second point would wait for the first
+// (four in turn made the shell 19 us of a 1024^2 f32 apply, the tiles 6)
+constexpr int kShellPtsPerThread = 1;
 
 // x window of a lane's VX consecutive points from its own registers and its neighbours'
 // through DPP shifts: xw[e] = u(xs - H + e), e < VX + 2H.  Lanes within ceil(H/VX) of the
@@ -478,7 +491,7 @@ __global__ __launch_bounds__(256) void k_tiled2d(const FastArgs A, const PlanDev
     int bi;
     if (!block_role((int)blockIdx.x, A.nblocks, nshell, &bi)) {
         const int64_t per = 256 * kShellPtsPerThread;
-        shell_points<T, ACC>(*Pp, SH, du, u, accumulate, (int64_t)bi * per, per);
+        shell_points<T, ACC, K>(*Pp, SH, A.pfast, du, u, accumulate, (int64_t)bi * per, per);
         return;
     }
     const int lane = threadIdx.x & 63;
@@ -580,192 +593,7 @@ __global__ __launch_bounds__(256) void k_tiled2d(const FastArgs A, const PlanDev
     else march(std::integral_constant<int, 1>{});
 }
 
-// ---------------------------------------------------------------------------------------
-// 3-D: a block of W waves stages W consecutive y rows of one x segment and computes the
-// middle W - 2H of them (the first and last H waves load halo rows only).  Every wave walks
-// a chunk of z planes with a register ring of K + PF planes of its row, loaded PF + H
-// planes ahead, and each step copies its centre plane into LDS (double-buffered, one
-// barrier per step), so every staged value was loaded several steps before it is used.
-// A wave loads an aligned 64*VX-point row segment whose first and last PADL points (whole
-// lanes) are the x halo: segments overlap by 2*PADL and only the middle lanes store.  The
-// memory operations of a step are the same on every path (addresses are clamped into the
-// array and out-of-range values selected to zero), which keeps the hardware's in-order
-// load counters precise so that a wait never drains the prefetched ring.  x and y taps come
-// from LDS, z taps from the ring; non-uniform x weights (per column) and z weights (per
-// plane of the chunk) are staged in LDS once.
 constexpr int kMaxChunk3D = 64;
-// planes prefetched beyond the deepest z tap (the ring holds K + PF planes), as deep as the
-// registers allow without spills
-template <typename T, int K>
-constexpr int kPF3D = sizeof(T) == 8 ? 1 : K <= 3 ? 4 : K <= 7 ? 2 : 1;
-
-template <typename T, int VX, int K, bool UNI, int PF, int W, int VY, int ACC>
-__global__ __launch_bounds__(64 * W) void k_tiled3d(const FastArgs A, const PlanDev* __restrict__ Pp,
-                                                     const ShellArgs SH, int nshell,
-                                                     T* __restrict__ du, const T* __restrict__ u,
-                                                     int accumulate)
-{
-    using C = typename Store<T>::C;
-    constexpr int H = K / 2;
-    constexpr int R = K + PF;
-    constexpr int SR = W * VY;                            // staged rows per block
-    constexpr int ROWW = 64 * VX;
-    constexpr int PADL = (H + VX - 1) / VX * VX;          // x halo, whole lanes
-    constexpr int LEDGE = PADL / VX;                      // load-only lanes at each end
-    constexpr int NRD = (PADL + H + VX + VX - 1) / VX;    // VX-wide reads covering a window
-    static_assert(2 * H < SR, "a block computes at least one row");
-    static_assert((64 - 2 * LEDGE - 1) * VX + NRD * VX <= ROWW, "x window inside the row");
-    __shared__ __attribute__((aligned(16))) C lds[2][SR][ROWW];
-    __shared__ C wzs[UNI ? 1 : kMaxChunk3D][K];
-    __shared__ __attribute__((aligned(16))) C wxs[UNI ? 1 : K][UNI ? 1 : ROWW];   // per column
-    int bi;
-    if (!block_role((int)blockIdx.x, A.nblocks, nshell, &bi)) {   // whole block: no barrier
-        const int64_t per = 64 * W * kShellPtsPerThread;
-        shell_points<T, ACC>(*Pp, SH, du, u, accumulate, (int64_t)bi * per, per);
-        return;
-    }
-
-    const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int b = tile_of(bi, A.nblocks, A.xcd_remap);
-    const int xseg = b % A.nxseg;
-    const int t = b / A.nxseg;
-    const int yblk = t % A.nyblk;
-    const int zch = t / A.nyblk;
-    // staged row r of the block is y = yb0 + r; wave w stages rows w + i*W (i < VY) and
-    // computes those in [H, SR - H)
-    const int yb0 = A.lo[1] + yblk * (SR - 2 * H) - H;
-    const int z0 = A.lo[2] + zch * A.chunk;
-    const int z1 = min(z0 + A.chunk, A.hi[2]);
-    const int64_t n0 = A.n[0];
-    const int n1 = (int)A.n[1], n2 = (int)A.n[2];
-    const int64_t s1 = A.s1, s2 = A.s2;
-    const int64_t xs0 = (int64_t)A.xbase + (int64_t)xseg * (ROWW - 2 * PADL);
-    const int64_t xs = xs0 + lane * VX;
-    // Loads are clamped into the array.  A lane whose segment lies outside [0, n0) (or a
-    // row / plane past the edge) then holds other points' values: only outputs in the box
-    // [lo, hi) are stored, and their x / y / z windows reach no further than H points past the
-    // box, i.e. never outside the array, so those values are never used.
-    const int64_t xl = min(max(xs, (int64_t)0), n0 - VX);  // clamped load column (rows are
-                                                           // whole VX groups)
-    const bool xst = lane >= LEDGE && lane < 64 - LEDGE && xs >= A.lo[0] && xs < A.hi[0];
-    const int lr = min(max(lane, LEDGE), 63 - LEDGE);      // window reads of load-only lanes
-    const int wcol = (lr - LEDGE) * VX;                     // first column of the window reads
-
-    int row[VY], y[VY], yc[VY];
-    bool computes[VY], st_ok[VY];
-#pragma unroll
-    for (int i = 0; i < VY; ++i) {
-        row[i] = wave + i * W;
-        y[i] = yb0 + row[i];
-        yc[i] = min(max(y[i], 0), n1 - 1);
-        computes[i] = row[i] >= H && row[i] < SR - H;      // wave-uniform
-        st_ok[i] = computes[i] && y[i] < A.hi[1] && xst;
-    }
-
-    const C* wxt = wtab<C>(A, 0);
-    const C* wyt = wtab<C>(A, 1);
-    const C* wzt = wtab<C>(A, 2);
-    C wxu[K], wzu[K];
-    C wy[VY][K];
-#pragma unroll
-    for (int i = 0; i < VY; ++i) {
-        const int64_t yr = UNI ? 0 : yc[i];
-#pragma unroll
-        for (int k = 0; k < K; ++k) wy[i][k] = wyt[yr * K + k];
-    }
-    if constexpr (UNI) {
-#pragma unroll
-        for (int k = 0; k < K; ++k) {
-            wxu[k] = wxt[k];
-            wzu[k] = wzt[k];
-        }
-    } else {
-        // visible to every wave after the first step's barrier
-        for (int i = threadIdx.x; i < (z1 - z0) * K; i += 64 * W)
-            wzs[i / K][i % K] = wzt[(int64_t)(z0 + i / K) * K + i % K];
-        for (int i = threadIdx.x; i < ROWW * K; i += 64 * W) {
-            const int c = i / K, k = i % K;
-            const int64_t x = min(max(xs0 + c, (int64_t)0), n0 - 1);
-            wxs[k][c] = wxt[x * K + k];
-        }
-    }
-
-    // one VX-wide load per call, on every path, straight into its ring slot
-    const T* urow[VY];
-#pragma unroll
-    for (int i = 0; i < VY; ++i) urow[i] = u + (int64_t)yc[i] * s1 + xl;
-    // planes past the chunk's last tap plane reload that plane (cached) instead of reading
-    // planes this wave never uses
-    const int zlast = min(z1 + H - 1, n2 - 1);
-    auto load_plane = [&](int i, int zz, C* dst) {
-        zz = min(max(zz, 0), zlast);
-        VecIO<T, VX>::ld(urow[i] + (int64_t)zz * s2, dst);
-    };
-
-    C q[VY][R][VX];
-#pragma unroll
-    for (int s = 0; s < R - 1; ++s) {
-#pragma unroll
-        for (int i = 0; i < VY; ++i) load_plane(i, z0 - H + s, q[i][s]);
-    }
-
-    int buf = 0;
-    for (int zb = z0; zb < z1; zb += R) {
-        auto step = [&](auto jc) -> bool {
-            constexpr int j = decltype(jc)::value;
-            const int z = zb + j;
-            if (z >= z1) return false;   // block-uniform
-#pragma unroll
-            for (int i = 0; i < VY; ++i) load_plane(i, z + H + PF, q[i][(j + K - 1 + PF) % R]);
-#pragma unroll
-            for (int i = 0; i < VY; ++i) {
-#pragma unroll
-                for (int v = 0; v < VX; ++v) lds[buf][row[i]][lane * VX + v] = q[i][(j + H) % R][v];
-            }
-            __syncthreads();
-            C wz[K];
-#pragma unroll
-            for (int k = 0; k < K; ++k) {
-                if constexpr (UNI) wz[k] = wzu[k];
-                else wz[k] = wzs[z - z0][k];
-            }
-#pragma unroll
-            for (int i = 0; i < VY; ++i) {
-                if (!computes[i]) continue;   // wave-uniform
-                C xw[NRD * VX];
-#pragma unroll
-                for (int r = 0; r < NRD; ++r) {
-#pragma unroll
-                    for (int v = 0; v < VX; ++v) xw[r * VX + v] = lds[buf][row[i]][wcol + r * VX + v];
-                }
-                Sum<C, ACC> out[VX];
-#pragma unroll
-                for (int v = 0; v < VX; ++v) {
-                    Sum<C, ACC> s = 0;
-#pragma unroll
-                    for (int k = 0; k < K; ++k) {
-                        C w;
-                        if constexpr (UNI) w = wxu[k];
-                        else w = wxs[k][lane * VX + v];
-                        s = fsum<C, ACC>(w, xw[PADL - H + v + k], s);
-                    }
-#pragma unroll
-                    for (int k = 0; k < K; ++k)
-                        s = fsum<C, ACC>(wy[i][k], lds[buf][row[i] - H + k][lane * VX + v], s);
-#pragma unroll
-                    for (int k = 0; k < K; ++k) s = fsum<C, ACC>(wz[k], q[i][(j + k) % R][v], s);
-                    out[v] = s;
-                }
-                if (st_ok[i])
-                    store_sums<T, VX, ACC>(du + (int64_t)z * s2 + (int64_t)y[i] * s1 + xs, out, accumulate);
-            }
-            buf ^= 1;
-            return true;
-        };
-        if (!ring_steps<0, R>(step)) break;
-    }
-}
 
 // ---------------------------------------------------------------------------------------
 // 3-D, edge-loaded form.  Segments do not overlap: a wave owns an aligned 64*VX-point x
@@ -1028,10 +856,7 @@ hipError_t launch_interior_tiles(const DevicePlan& p, const FastArgs& A, void* d
     // per-row indexing needs a row of weights for every point of every axis
     for (int a = 0; a < fp.kind; ++a)
         if (fp.w64[a].size() != (size_t)(uni ? 1 : A.n[a]) * K) return hipErrorInvalidValue;
-    const int64_t per = (int64_t)256 * kShellPtsPerThread;
-    // 2-D: the (thin) shell rides in the tile launch; 3-D: a launch of its own first
-    const int nshell = fp.kind == 2 ? (int)((fp.shell_total + per - 1) / per) : 0;
-    if (fp.kind == 3 && A.gen == 2) {
+    if (fp.kind == 3) {
         if constexpr (K <= 9 && VX <= 16 / (int)sizeof(T) && VX <= 4) {
 #define DOP_L3E(UNI, W, VY)                                                                  \
     hipLaunchKernelGGL((k_tiled3e<T, VX, K, UNI, 1, W, VY, ACC>), dim3((unsigned)A.nblocks),   \
@@ -1040,11 +865,10 @@ hipError_t launch_interior_tiles(const DevicePlan& p, const FastArgs& A, void* d
     do {                                                                                     \
         if (uni) DOP_L3E(true, W, VY); else DOP_L3E(false, W, VY);                           \
     } while (0)
-            const int shape = A.W * 8 + A.VY;
-            if (shape == 8 * 8 + 1) DOP_L3EU(8, 1);
-            else if (shape == 8 * 8 + 2) DOP_L3EU(8, 2);
-            else if (shape == 16 * 8 + 1) DOP_L3EU(16, 1);
-            else if (shape == 8 * 8 + 3) DOP_L3EU(8, 3);
+            if (A.W != 8) return hipErrorInvalidValue;
+            if (A.VY == 1) DOP_L3EU(8, 1);
+            else if (A.VY == 2) DOP_L3EU(8, 2);
+            else if (A.VY == 3) DOP_L3EU(8, 3);
             else return hipErrorInvalidValue;
 #undef DOP_L3EU
 #undef DOP_L3E
@@ -1053,61 +877,22 @@ hipError_t launch_interior_tiles(const DevicePlan& p, const FastArgs& A, void* d
             return hipErrorInvalidValue;
         }
     }
+    // 2-D: the (thin) shell rides in the tile launch
+    const int64_t per = (int64_t)256 * kShellPtsPerThread;
+    const int nshell = (int)((fp.shell_total + per - 1) / per);
     const dim3 grid((unsigned)(A.nblocks + nshell));
-    if (fp.kind == 2) {
-#define DOP_L2E(UNI, PF, EDG)                                                                \
+    constexpr bool EDG = K / 2 <= VX;
+    constexpr int P0 = EDG ? (sizeof(T) == 8 ? 8 : 4) : 2;
+    if (A.gen != (EDG ? 2 : 1)) return hipErrorInvalidValue;
+#define DOP_L2(UNI, PF)                                                                      \
     hipLaunchKernelGGL((k_tiled2d<T, VX, K, UNI, PF, ACC, EDG>), grid, dim3(256), 0, s, A, p.dev, \
                        fp.shell, nshell, (T*)du, (const T*)u, accumulate)
-#define DOP_L2(UNI)                                                                          \
-    do {                                                                                     \
-        if (A.gen == 2) {                                                                    \
-            if constexpr (K / 2 <= VX) {                                                     \
-                if constexpr (sizeof(T) == 8) {                                              \
-                    if (A.PF == 16) DOP_L2E(UNI, 16, true); else DOP_L2E(UNI, 8, true);      \
-                } else {                                                                     \
-                    if (A.PF == 8) DOP_L2E(UNI, 8, true); else DOP_L2E(UNI, 4, true);        \
-                }                                                                            \
-                break;                                                                       \
-            }                                                                                \
-            return hipErrorInvalidValue;                                                     \
-        }                                                                                    \
-        if (A.PF == 4) DOP_L2E(UNI, 4, false); else DOP_L2E(UNI, 2, false);                  \
-    } while (0)
-        if (uni) DOP_L2(true); else DOP_L2(false);
-#undef DOP_L2
-#undef DOP_L2E
+    if (uni) {
+        if (A.PF == P0) DOP_L2(true, P0); else DOP_L2(true, 2 * P0);
     } else {
-        if constexpr (K <= 9 && VX <= 16 / (int)sizeof(T) && VX <= 4) {
-#define DOP_L3(UNI, W, VY)                                                                   \
-    hipLaunchKernelGGL((k_tiled3d<T, VX, K, UNI, kPF3D<T, K>, W, VY, ACC>), grid, dim3(64 * W), 0, s, \
-                       A, p.dev, fp.shell, nshell, (T*)du, (const T*)u, accumulate)
-            constexpr bool w8 = 2 * (K / 2) < 8;   // 8-wave blocks of one row compute 8 - 2H rows
-#define DOP_L3U(W, VY)                                                                       \
-    do {                                                                                     \
-        if (uni) DOP_L3(true, W, VY); else DOP_L3(false, W, VY);                             \
-    } while (0)
-            // (waves per block, rows per wave): the shapes fast_variant produces
-            const int shape = A.W * 8 + A.VY;
-            if (shape == 8 * 8 + 1) {
-                if constexpr (w8) DOP_L3U(8, 1);
-                else return hipErrorInvalidValue;
-            } else if (shape == 16 * 8 + 1) {
-                DOP_L3U(16, 1);
-            } else if (shape == 8 * 8 + 2) {
-                DOP_L3U(8, 2);
-            } else if (shape == 16 * 8 + 2) {
-                DOP_L3U(16, 2);
-            } else if (shape == 8 * 8 + 3) {
-                DOP_L3U(8, 3);
-            } else {
-                return hipErrorInvalidValue;
-            }
-#undef DOP_L3U
-#undef DOP_L3
-        } else {
-            return hipErrorInvalidValue;
-        }
+        if (A.PF == P0) DOP_L2(false, P0); else DOP_L2(false, 2 * P0);
     }
+#undef DOP_L2
     return hipGetLastError();
 }
 

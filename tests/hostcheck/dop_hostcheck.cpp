@@ -133,6 +133,61 @@ void run_shell(const dop::PlanDev& P, const dop::StripArgs& S, int K, T* du, con
 }
 }  // namespace
 
+namespace {
+template <typename T, int ACC, int KM>
+void run_points(const dop::PlanDev& P, T* du, const T* src, int accumulate)
+{
+    for (int64_t p = 0; p < P.total; ++p) {
+        const int64_t idx[3] = {p % P.n[0], p / P.n[0] % P.n[1], 0};
+        double v = P.ndim == 1 ? dop::shell_point<T, ACC, KM, 1>(P, src, idx)
+                               : dop::shell_point<T, ACC, KM, 2>(P, src, idx);
+        if (accumulate) v += (double)dop::Store<T>::ld(du, p);
+        dop::Store<T>::st(du, p, v);
+    }
+}
+
+template <typename T, int ACC>
+int run_points_k(int K, const dop::PlanDev& P, T* du, const T* src, int accumulate)
+{
+    switch (K) {
+    case 3: run_points<T, ACC, 3>(P, du, src, accumulate); return 1;
+    case 5: run_points<T, ACC, 5>(P, du, src, accumulate); return 1;
+    case 7: run_points<T, ACC, 7>(P, du, src, accumulate); return 1;
+    case 9: run_points<T, ACC, 9>(P, du, src, accumulate); return 1;
+    case 11: run_points<T, ACC, 11>(P, du, src, accumulate); return 1;
+    case 13: run_points<T, ACC, 13>(P, du, src, accumulate); return 1;
+    }
+    return -1;
+}
+}  // namespace
+
+extern "C" {
+// Every point of a 1-D or 2-D plan through shell_point (the latency form of the per-point
+// evaluation).  1; 0 when shell_point_ok refuses the plan; -1 without a tiled path.
+int hc_shell_point(const dop_desc* d, void* du, const void* u, int accumulate)
+{
+    dop::HostPlan H;
+    if (dop::build_host_plan(*d, &H, &g_err) != DOP_OK) return -1;
+    dop::FastPlan F;
+    dop::build_fast(H, &F);
+    if (F.kind != 1 && F.kind != 2) return -1;
+    const dop::PlanDev P = bind(H);
+    using namespace dop;
+    if (!F.args.pfast) return 0;
+    switch (P.storage) {
+    case kF64: return run_points_k<double, kAccF64>(F.args.K, P, (double*)du, (const double*)u, accumulate);
+    case kF32:
+        if (P.accum == kAccF32Wide)
+            return run_points_k<float, kAccF32Wide>(F.args.K, P, (float*)du, (const float*)u, accumulate);
+        return run_points_k<float, kAccF32>(F.args.K, P, (float*)du, (const float*)u, accumulate);
+    default:
+        if (P.accum == kAccF32Wide)
+            return run_points_k<bf16, kAccF32Wide>(F.args.K, P, (bf16*)du, (const bf16*)u, accumulate);
+        return run_points_k<bf16, kAccF32>(F.args.K, P, (bf16*)du, (const bf16*)u, accumulate);
+    }
+}
+}  // extern "C"
+
 extern "C" {
 // The 3-D shell of the tiled path (every point outside the tiles' box) evaluated strip by strip
 // with the device kernel's per-strip code; other points of du are left as they are.  Returns the

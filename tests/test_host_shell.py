@@ -162,3 +162,31 @@ def test_shell_strips_per_line_bcs(hc, storage, periodic):
     u = values(shape, storage, rng)
     check(hc, d, u, storage, 0)
     check(hc, d, u, storage, 1)
+
+
+@pytest.mark.parametrize("storage", ["f64", "f32"])
+@pytest.mark.parametrize("axes", [(1,), (2,), (1, 2, 3)])
+@pytest.mark.parametrize("n0", [64, 70, 73])
+def test_shell_strips_per_line_bcs_any_axis(hc, storage, axes, n0):
+    # one atomic BC per line along y and z too: no face item (its points share one BC) may cover
+    # such an axis's rows
+    rng = np.random.default_rng(17)
+    shape = (24, 20, n0)
+    ops, jsize = operators(shape, 2, rng, False, upwind=True)
+    Qs = []
+    for N in (1, 2, 3):
+        other = tuple(jsize[k] for k in range(3) if k != N - 1)
+        if N not in axes:
+            Qs.append(D.MultiDimBC[N](D.NeumannBC((0.1, -0.3), 0.05, 1), jsize))
+            continue
+        arr = np.empty(other, dtype=object)
+        for i in np.ndindex(*other):
+            arr[i] = D.RobinBC(tuple(rng.uniform(0.5, 1.5, 3)), tuple(rng.uniform(0.5, 1.5, 3)), 0.02, 1)
+        Qs.append(D.MultiDimBC[N](arr))
+    bcs = _bcs_of(D.compose(*Qs), 3, jsize)[0]
+    d, keep = make_desc(ops, jsize, STORAGE[storage][0], input_kind=_abi.INPUT_GHOST,
+                        semantics=_abi.SEM_LINES, bcs=bcs)
+    u = values(shape, storage, rng)
+    check(hc, d, u, storage, 0)
+    check(hc, d, u, storage, 1)
+    assert all(kinds(hc, d)[N - 1] == 0 for N in axes)
