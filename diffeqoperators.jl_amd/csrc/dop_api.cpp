@@ -404,7 +404,8 @@ namespace {
 int batch_upload(dop_batch* b, int chunk)
 {
     for (auto& P : b->probs) P.chunk = chunk;
-    dop::batch_items(b->probs, &b->items, &b->groups);
+    dop::batch_march_chunks(&b->probs);
+    dop::batch_items(b->probs, b->rk4, &b->items, &b->groups);
     b->chunk = chunk;
     b->nitems = (int)b->items.size();
     if (!b->d_probs) {
@@ -423,9 +424,10 @@ int batch_upload(dop_batch* b, int chunk)
     return DOP_OK;
 }
 
-int batch_init(dop_batch* b, int n, const dop_plan* const* plans)
+int batch_init(dop_batch* b, int n, const dop_plan* const* plans, bool rk4 = false)
 {
     b->storage = plans[0]->d.host.storage;
+    b->rk4 = rk4;
     b->grid = device_grid(8);
     b->probs.resize(n);
     for (int i = 0; i < n; ++i) {
@@ -433,7 +435,7 @@ int batch_init(dop_batch* b, int n, const dop_plan* const* plans)
             return fail(DOP_EINVAL, "mixed storage types in batch");
         dop::BProb& P = b->probs[i];
         P = dop::BProb{};
-        dop::batch_geometry(plans[i]->d, b->chunk, &P);
+        dop::batch_geometry(plans[i]->d, b->chunk, &P, rk4);
     }
     return DOP_OK;
 }
@@ -527,21 +529,68 @@ int dop_batch_autotune(dop_batch* batch, void* stream, int* choice)
 void dop_batch_destroy(dop_batch* batch) { delete batch; }
 
 namespace {
-// One stage of a batch captured with its groups on ns forked streams (fresh events per stage:
-// each fork and join becomes its own graph edge).
-int capture_stage_forked(const dop_batch* b, int stage, hipStream_t cs, hipStream_t* ws, int ns,
-                         std::vector<hipEvent_t>* evs)
+// One RK4 step captured on cs.  The fused passes run on streams of their own beside the chain of
+// the four stages (the rims and the other problems; the two write disjoint points), whose groups
+// are spread over forked streams too and joined after each stage (fresh events each time: every
+// fork and join becomes its own graph edge).  ns = 1: all in order on cs.
+int capture_step(const dop_batch* b, int parity, hipStream_t cs, hipStream_t* ws, int ns,
+                 std::vector<hipEvent_t>* evs)
 {
-    const size_t first = evs->size();
-    for (int i = 0; i <= ns; ++i) {
-        hipEvent_t e = nullptr;
-        if (hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess)
+    auto events = [&](int n) {
+        for (int i = 0; i < n; ++i) {
+            hipEvent_t e = nullptr;
+            if (hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) return false;
+            evs->push_back(e);
+        }
+        return true;
+    };
+    auto march = [&](const std::vector<dop::BGroup>& g, hipStream_t s) {
+        return dop::launch_batch_pass(b->storage, b->d_probs, b->d_items, g, false, parity, b->grid,
+                                       s) == hipSuccess;
+    };
+    // fused groups, largest first, on the least loaded of nm streams
+    std::vector<dop::BGroup> fused;
+    for (const auto& g : b->groups)
+        if (dop::group_is_pass(g)) fused.push_back(g);
+    std::sort(fused.begin(), fused.end(),
+              [](const dop::BGroup& x, const dop::BGroup& y) { return x.count > y.count; });
+    bool stages = false;   // problems that go stage by stage
+    for (const auto& g : b->groups) stages = stages || dop::group_is_stage(g);
+    const int nm = ns > 1 && !fused.empty() ? (stages ? ns / 2 : ns) : 0;
+    const int nc = ns > 1 ? ns - nm : 1;
+    const size_t fork = evs->size();
+    if (nm > 0) {
+        if (!events(1 + nm) || hipEventRecord((*evs)[fork], cs) != hipSuccess)
             return fail(DOP_EHIP, "rk4: event creation failed");
-        evs->push_back(e);
+        std::vector<int64_t> load(nm, 0);
+        for (int i = 0; i < nm; ++i)
+            if (hipStreamWaitEvent(ws[i], (*evs)[fork], 0) != hipSuccess)
+                return fail(DOP_EHIP, "rk4: fork failed");
+        for (const auto& g : fused) {
+            const int i = (int)(std::min_element(load.begin(), load.end()) - load.begin());
+            if (!march({g}, ws[i])) return fail(DOP_EHIP, "rk4: launch during capture failed");
+            load[i] += g.count;
+        }
+    } else if (!march(b->groups, cs)) {
+        return fail(DOP_EHIP, "rk4: launch during capture failed");
     }
-    if (dop::launch_batch_items_forked(b->storage, b->d_probs, b->d_items, b->groups, stage, 0,
-                                       b->grid, cs, ws, evs->data() + first, ns) != hipSuccess)
-        return fail(DOP_EHIP, "rk4: stage launch during capture failed");
+    for (int st = 0; st < 4 && stages; ++st) {
+        hipError_t e;
+        if (ns == 1) {
+            e = dop::launch_batch_items(b->storage, b->d_probs, b->d_items, b->groups, st, 0,
+                                        b->grid, cs);
+        } else {
+            const size_t first = evs->size();
+            if (!events(1 + nc)) return fail(DOP_EHIP, "rk4: event creation failed");
+            e = dop::launch_batch_items_forked(b->storage, b->d_probs, b->d_items, b->groups, st, 0,
+                                               b->grid, cs, ws + nm, evs->data() + first, nc);
+        }
+        if (e != hipSuccess) return fail(DOP_EHIP, "rk4: stage launch during capture failed");
+    }
+    for (int i = 0; i < nm; ++i)
+        if (hipEventRecord((*evs)[fork + 1 + i], ws[i]) != hipSuccess ||
+            hipStreamWaitEvent(cs, (*evs)[fork + 1 + i], 0) != hipSuccess)
+            return fail(DOP_EHIP, "rk4: join failed");
     return DOP_OK;
 }
 }  // namespace
@@ -558,7 +607,7 @@ int dop_rk4_create(int n, const dop_plan* const* plans, const double* scale, con
     if (storage != DOP_F64 && storage != DOP_F32)
         return fail(DOP_EUNSUPPORTED, "rk4 needs f32 or f64 storage");
     dop_rk4* rk = new dop_rk4();
-    int r = batch_init(&rk->b, n, plans);
+    int r = batch_init(&rk->b, n, plans, true);
     const size_t sb = storage_bytes(storage);
     for (int i = 0; i < n && r == DOP_OK; ++i) {
         dop::BProb& P = rk->b.probs[i];
@@ -566,7 +615,8 @@ int dop_rk4_create(int n, const dop_plan* const* plans, const double* scale, con
         P.scale = scale[i];
         P.dt = dt[i];
         void* bufs[3] = {nullptr, nullptr, nullptr};
-        for (int k = 0; k < 3 && r == DOP_OK; ++k) {
+        // (one-pass steps use u and acc only)
+        for (int k = P.fused ? 2 : 0; k < 3 && r == DOP_OK; ++k) {
             if (hipMalloc(&bufs[k], plans[i]->d.host.total * sb) != hipSuccess)
                 r = fail(DOP_ENOMEM, "rk4: stage buffer allocation failed");
             else
@@ -580,11 +630,13 @@ int dop_rk4_create(int n, const dop_plan* const* plans, const double* scale, con
     // tile shape: stage 0 only reads u and writes acc / s1, so it can be timed repeatedly
     const char* at = std::getenv("DOP_RK4_AUTOTUNE");
     if (r == DOP_OK) {
-        if (at && at[0] == '0') r = batch_upload(&rk->b, rk->b.chunk);
+        bool tiles = false;   // (one-pass steps have no tiles to tune)
+        for (const auto& P : rk->b.probs) tiles = tiles || (P.tiled == 1 && !P.fused);
+        if (!tiles || (at && at[0] == '0')) r = batch_upload(&rk->b, rk->b.chunk);
         else r = batch_tune(&rk->b, 0, s, nullptr);
     }
-    // capture one step (four stages; each stage's groups on forked streams) into a graph.
-    // DOP_RK4_STREAMS sets the number of streams (1: every group in order on one stream).
+    // capture two steps, and one step with the copy back, each into a graph.  DOP_RK4_STREAMS sets
+    // the number of streams (1: every group in order on one stream).
     hipStream_t cs = nullptr;
     int ns = 4;
     if (const char* e = std::getenv("DOP_RK4_STREAMS")) ns = std::max(1, std::min(8, std::atoi(e)));
@@ -595,24 +647,22 @@ int dop_rk4_create(int n, const dop_plan* const* plans, const double* scale, con
     for (int i = 0; i < ns && r == DOP_OK; ++i)
         if (hipStreamCreateWithFlags(&ws[i], hipStreamNonBlocking) != hipSuccess)
             r = fail(DOP_EHIP, "rk4: stream creation failed");
-    if (r == DOP_OK) {
+    for (int k = 0; k < 2 && r == DOP_OK; ++k) {
         if (hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal) != hipSuccess) {
             r = fail(DOP_EHIP, "rk4: begin capture failed");
-        } else {
-            for (int st = 0; st < 4 && r == DOP_OK; ++st) {
-                if (ns == 1) {
-                    if (batch_launch(&rk->b, st, 0, cs) != hipSuccess)
-                        r = fail(DOP_EHIP, "rk4: stage launch during capture failed");
-                } else {
-                    r = capture_stage_forked(&rk->b, st, cs, ws.data(), ns, &evs);
-                }
-            }
-            if (hipStreamEndCapture(cs, &rk->graph) != hipSuccess && r == DOP_OK)
-                r = fail(DOP_EHIP, "rk4: end capture failed");
-            if (r == DOP_OK &&
-                hipGraphInstantiate(&rk->exec, rk->graph, nullptr, nullptr, 0) != hipSuccess)
-                r = fail(DOP_EHIP, "rk4: graph instantiation failed");
+            break;
         }
+        r = capture_step(&rk->b, 0, cs, ws.data(), ns, &evs);
+        if (r == DOP_OK && k == 0) r = capture_step(&rk->b, 1, cs, ws.data(), ns, &evs);
+        if (r == DOP_OK && k == 1 &&
+            dop::launch_batch_pass(storage, rk->b.d_probs, rk->b.d_items, rk->b.groups, true, 0,
+                                    rk->b.grid, cs) != hipSuccess)
+            r = fail(DOP_EHIP, "rk4: copy launch during capture failed");
+        if (hipStreamEndCapture(cs, &rk->graph[k]) != hipSuccess && r == DOP_OK)
+            r = fail(DOP_EHIP, "rk4: end capture failed");
+        if (r == DOP_OK &&
+            hipGraphInstantiate(&rk->exec[k], rk->graph[k], nullptr, nullptr, 0) != hipSuccess)
+            r = fail(DOP_EHIP, "rk4: graph instantiation failed");
     }
     for (hipEvent_t e : evs) (void)hipEventDestroy(e);
     for (hipStream_t w : ws)
@@ -629,7 +679,8 @@ int dop_rk4_create(int n, const dop_plan* const* plans, const double* scale, con
 int dop_rk4_step(dop_rk4* rk, int nsteps, void* stream)
 {
     if (!rk || nsteps < 0) return fail(DOP_EINVAL, "bad rk4 step arguments");
-    for (int i = 0; i < nsteps; ++i) DOP_HIP(hipGraphLaunch(rk->exec, (hipStream_t)stream));
+    for (int i = 0; i + 1 < nsteps; i += 2) DOP_HIP(hipGraphLaunch(rk->exec[0], (hipStream_t)stream));
+    if (nsteps & 1) DOP_HIP(hipGraphLaunch(rk->exec[1], (hipStream_t)stream));
     return DOP_OK;
 }
 

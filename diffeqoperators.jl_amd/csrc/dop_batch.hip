@@ -28,6 +28,7 @@ hipError_t launch_batch_items(int storage, const BProb* probs, const BItem* item
                               int grid, hipStream_t s)
 {
     for (const BGroup& g : groups) {
+        if (!group_is_stage(g)) continue;
         const hipError_t e = launch_batch_group(storage, g, probs, items, stage, accumulate, grid, s);
         if (e != hipSuccess) return e;
     }
@@ -48,8 +49,9 @@ hipError_t launch_batch_items_forked(int storage, const BProb* probs, const BIte
     for (int i = 0; i < ns; ++i)
         if ((e = hipStreamWaitEvent(ws[i], evs[0], 0)) != hipSuccess) return e;
     std::vector<int64_t> load(ns, 0);
-    std::vector<int> order(groups.size());
-    for (size_t i = 0; i < order.size(); ++i) order[i] = (int)i;
+    std::vector<int> order;
+    for (size_t i = 0; i < groups.size(); ++i)
+        if (group_is_stage(groups[i])) order.push_back((int)i);
     std::sort(order.begin(), order.end(),
               [&](int x, int y) { return groups[x].count > groups[y].count; });
     for (int gi : order) {
@@ -62,6 +64,22 @@ hipError_t launch_batch_items_forked(int storage, const BProb* probs, const BIte
     for (int i = 0; i < ns; ++i) {
         if ((e = hipEventRecord(evs[1 + i], ws[i])) != hipSuccess) return e;
         if ((e = hipStreamWaitEvent(s, evs[1 + i], 0)) != hipSuccess) return e;
+    }
+    return hipSuccess;
+}
+
+hipError_t launch_pass_f64(const BGroup&, const BProb*, const BItem*, int, int, hipStream_t);
+hipError_t launch_pass_f32(const BGroup&, const BProb*, const BItem*, int, int, hipStream_t);
+
+hipError_t launch_batch_pass(int storage, const BProb* probs, const BItem* items,
+                              const std::vector<BGroup>& groups, bool back, int parity, int grid,
+                              hipStream_t s)
+{
+    for (const BGroup& g : groups) {
+        if (back ? !group_is_back(g) : !group_is_pass(g)) continue;
+        const hipError_t e = storage == kF64 ? launch_pass_f64(g, probs, items, parity, grid, s)
+                                             : launch_pass_f32(g, probs, items, parity, grid, s);
+        if (e != hipSuccess) return e;
     }
     return hipSuccess;
 }

@@ -4,6 +4,7 @@
 #include <tuple>
 
 #include "dop_batch.hpp"
+#include "dop_eval.hpp"
 
 namespace dop {
 
@@ -11,7 +12,107 @@ namespace {
 int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 }  // namespace
 
-void batch_geometry(const DevicePlan& p, int chunk, BProb* B)
+namespace {
+
+// The box of a 2-D tiled problem that marching segments take: the points whose four-stage cone (4H
+// in x and y) holds regular rows only, whole lane groups along x.  False when it is too small to
+// pay (its rim, 4H to 5H points a side, and the 4H columns beside every segment are recomputed).
+constexpr int kMarchMin = 96;
+
+bool march_box(const PlanDev& P, const FastArgs& A, BProb* B)
+{
+    const int VX = march_vx(P.storage, P.accum, A.K), H = A.K / 2;
+    const int pad = (int)ceil_div(4 * H, VX) * VX;
+    const int out = 64 * VX - 2 * pad;
+    B->flo[0] = std::max(B->lo[0] + 3 * H, pad);
+    B->fhi[0] = (int)std::min<int64_t>(B->hi[0] - 3 * H, B->n0 - pad);
+    B->fhi[0] = B->flo[0] + (B->fhi[0] - B->flo[0]) / VX * VX;
+    B->flo[1] = B->lo[1] + 3 * H;
+    B->fhi[1] = B->hi[1] - 3 * H;
+    for (int a = 0; a < 2; ++a)
+        if (B->fhi[a] - B->flo[a] < kMarchMin) return false;
+    B->fnseg = (int)ceil_div(B->fhi[0] - B->flo[0], out);
+    B->fchunk = 64;
+    return true;
+}
+
+// LDS bytes of a patch (k_rk4_patch): u and two stage arrays over all that its points' cones
+// reach, the stage sums over its points
+int64_t patch_bytes(const PlanDev& P, int H, int x0, int x1, int y0, int y1)
+{
+    const int64_t own = (int64_t)(x1 - x0) * (y1 - y0);
+    for (int s = 0; s < 4; ++s) {
+        rows_reach(P.ax[0], H, &x0, &x1);
+        if (P.ndim == 2) rows_reach(P.ax[1], H, &y0, &y1);
+    }
+    return kPatchHead + (3 * (int64_t)((x1 - x0) | 1) * (y1 - y0) + own) * (P.storage == kF64 ? 8 : 4);
+}
+
+// Patch extents (w, h) for a rectangle of points of the grid: lines of up to 128 loaded points
+// (two waves of lanes) by what the LDS then holds, at most 16 or 32 rows of own points beyond the
+// recomputed ones; thin rectangles keep their width.  False when even small patches do not fit.
+bool patch_size(const PlanDev& P, int H, int rw, int rh, int* w, int* h)
+{
+    // how far the patch's points reach, over four stages, at its widest: windows on both sides
+    // and, on one side, boundary rows (whose windows may be one longer than the reach in)
+    int ext[2] = {0, 0};
+    for (int a = 0; a < P.ndim; ++a) {
+        const AxisDev& X = P.ax[a];
+        ext[a] = 8 * H + X.KB;
+    }
+    const int64_t sb = P.storage == kF64 ? 8 : 4;
+    auto fits = [&](int ww, int hh) {
+        return kPatchHead + (3 * (int64_t)((ww + ext[0]) | 1) * (hh + ext[1]) + (int64_t)ww * hh) * sb <=
+               kPatchLds;
+    };
+    if (P.ndim == 1) {
+        *w = std::min(rw, 1024);
+        *h = 1;
+        return fits(*w, 1);
+    }
+    if (rw <= 64 && rw < rh) {   // a strip along y
+        *w = rw;
+        for (*h = std::min(rh, 128 - std::min(ext[1], 96)); *h >= 8; *h -= 4)
+            if (fits(*w, *h)) return true;
+        return false;
+    }
+    for (*h = std::min(rh, 32); *h >= 4; *h = *h > 8 ? (*h + 1) / 2 : *h - 2) {
+        for (*w = std::min(rw, 128 - std::min(ext[0], 96)); *w >= 16 || *w == rw; *w -= 4)
+            if (fits(*w, *h)) return true;
+    }
+    return false;
+}
+
+template <typename F>
+void patches(const PlanDev& P, int H, int x0, int x1, int y0, int y1, const F& f)
+{
+    int w, h;
+    if (x1 <= x0 || y1 <= y0 || !patch_size(P, H, x1 - x0, y1 - y0, &w, &h)) return;
+    // even pieces
+    const int nx = (int)ceil_div(x1 - x0, w), ny = (int)ceil_div(y1 - y0, h);
+    for (int j = 0; j < ny; ++j)
+        for (int i = 0; i < nx; ++i)
+            f(x0 + (int)((int64_t)(x1 - x0) * i / nx), x0 + (int)((int64_t)(x1 - x0) * (i + 1) / nx),
+              y0 + (int)((int64_t)(y1 - y0) * j / ny), y0 + (int)((int64_t)(y1 - y0) * (j + 1) / ny));
+}
+
+// the rim of the box [flo, fhi) as up to four rectangles, or the whole grid
+template <typename F>
+void patch_rects(const BProb& B, int n0, int n1, const F& f)
+{
+    if (B.fused != 2) {
+        f(0, n0, 0, n1);
+        return;
+    }
+    f(0, n0, 0, B.flo[1]);
+    f(0, n0, B.fhi[1], n1);
+    f(0, B.flo[0], B.flo[1], B.fhi[1]);
+    f(B.fhi[0], n0, B.flo[1], B.fhi[1]);
+}
+
+}  // namespace
+
+void batch_geometry(const DevicePlan& p, int chunk, BProb* B, bool rk4)
 {
     const PlanDev& P = p.host;
     const FastPlan& f = p.fast;
@@ -21,6 +122,10 @@ void batch_geometry(const DevicePlan& p, int chunk, BProb* B)
     // 2-D and 1-D tiles exist for windows up to 11 taps (the batched tile kernels'
     // instantiations); they cover the natural box (one point per lane, no alignment)
     B->tiled = (f.args.K <= kMaxBatchTileK) ? (f.kind == 2 ? 1 : f.kind == 1 ? 2 : 0) : 0;
+    B->nd = P.ndim;
+    B->hplan = &p.host;
+    B->pfast = B->tiled && f.args.pfast ? f.args.K : 0;
+    B->fused = 0;
     if (B->tiled) {
         const FastArgs& A = f.args;
         const int H = A.K / 2;
@@ -38,6 +143,20 @@ void batch_geometry(const DevicePlan& p, int chunk, BProb* B)
         B->n1 = A.n[1];
         B->ys = A.s1;
         B->shell = f.nat_shell;
+        if (rk4 && B->pfast && (P.storage == kF64 || P.storage == kF32)) {
+            B->fused = B->tiled == 1 && march_box(P, A, B) ? 2 : 1;
+            // every patch must fit the LDS (and be there: patches() leaves out none it could make)
+            bool fits = true;
+            patch_rects(*B, (int)P.n[0], (int)P.n[1], [&](int x0, int x1, int y0, int y1) {
+                int w, h;
+                if (x1 <= x0 || y1 <= y0) return;
+                fits = fits && patch_size(P, B->K / 2, x1 - x0, y1 - y0, &w, &h);
+                if (fits) patches(P, B->K / 2, x0, x1, y0, y1, [&](int xa, int xb, int ya, int yb) {
+                    fits = fits && patch_bytes(P, B->K / 2, xa, xb, ya, yb) <= kPatchLds;
+                });
+            });
+            if (!fits) B->fused = 0;
+        }
     } else {
         B->K = 0;
         ShellArgs& S = B->shell;
@@ -52,26 +171,66 @@ void batch_geometry(const DevicePlan& p, int chunk, BProb* B)
     }
 }
 
-void batch_items(const std::vector<BProb>& probs, std::vector<BItem>* items,
+void batch_march_chunks(std::vector<BProb>* probs)
+{
+    // Rows per chunk: a wave's march is serial, so its chunk is as short as keeps the waves the chip
+    // holds at once (two a SIMD, 2048) in one round, at least 16 rows (6H more are recomputed); where
+    // there is work for more rounds, chunks of 64 rows.
+    auto waves = [&](int chunk) {
+        int64_t w = 0;
+        for (const BProb& B : *probs)
+            if (B.fused == 2) w += (int64_t)B.fnseg * ceil_div(B.fhi[1] - B.flo[1], chunk);
+        return w;
+    };
+    int chunk = 16;
+    while (chunk < 64 && waves(chunk) > 2048) chunk += 4;
+    for (BProb& B : *probs) B.fchunk = chunk;
+}
+
+void batch_items(const std::vector<BProb>& probs, bool rk4, std::vector<BItem>* items,
                  std::vector<BGroup>* groups)
 {
-    // group key: kind, window, accumulator
     auto key = [&](const BItem& I) {
         const BProb& B = probs[I.prob];
-        return std::make_tuple(I.kind, I.kind != 1 ? B.K : 0, B.plan_accum);
+        if (I.kind == kItemBack) return std::make_tuple((int)kItemBack, 0, 0, 0);
+        if (I.kind == kItemPatch) return std::make_tuple((int)kItemPatch, B.K, B.plan_accum, 0);
+        if (I.kind == kItemMarch)
+            return std::make_tuple((int)kItemMarch, B.K, B.plan_accum, B.uniform[0] && B.uniform[1] ? 1 : 0);
+        if (rk4) return std::make_tuple(I.kind == kItemPoints ? (int)kItemPoints : (int)kItemStage, 0, B.plan_accum, 0);
+        return std::make_tuple(I.kind, I.kind == kItemPoints ? B.pfast : B.K, B.plan_accum, 0);
     };
     items->clear();
     for (size_t i = 0; i < probs.size(); ++i) {
         const BProb& B = probs[i];
+        const int32_t p = (int32_t)i;
+        if (B.fused) {
+            const PlanDev& P = *B.hplan;
+            patch_rects(B, (int)P.n[0], (int)P.n[1], [&](int x0, int x1, int y0, int y1) {
+                patches(P, B.K / 2, x0, x1, y0, y1, [&](int xa, int xb, int ya, int yb) {
+                    items->push_back({p, kItemPatch, xa, xb, ya, yb});
+                });
+            });
+            if (B.fused == 2) {
+                const int64_t nch = ceil_div(B.fhi[1] - B.flo[1], B.fchunk);
+                for (int64_t ch = 0; ch < nch; ++ch)
+                    for (int sg = 0; sg < B.fnseg; ++sg)
+                        items->push_back({p, kItemMarch, sg, (int32_t)ch, 0, 0});
+            }
+            const int64_t nb = ceil_div(P.total, kBackPts);
+            for (int64_t c = 0; c < nb; ++c) items->push_back({p, kItemBack, (int32_t)c, 0, 0, 0});
+            continue;
+        }
         if (B.tiled == 1) {
             const int64_t nch = ceil_div(B.hi[1] - B.lo[1], B.chunk);
             for (int64_t ch = 0; ch < nch; ++ch)
-                for (int xg = 0; xg < B.gx; ++xg) items->push_back({(int32_t)i, 0, xg, (int32_t)ch});
+                for (int xg = 0; xg < B.gx; ++xg) items->push_back({p, kItemTile, xg, (int32_t)ch, 0, 0});
         } else if (B.tiled == 2) {
-            for (int xg = 0; xg < B.gx; ++xg) items->push_back({(int32_t)i, 2, xg, 0});
+            for (int xg = 0; xg < B.gx; ++xg) items->push_back({p, kItemTile1, xg, 0, 0, 0});
         }
-        const int64_t ns = ceil_div(B.shell.start[B.shell.nbox], kChunkPts);
-        for (int64_t c = 0; c < ns; ++c) items->push_back({(int32_t)i, 1, (int32_t)c, 0});
+        // (a stage's points launch takes shell_point where it can at any window, so kRimPts there
+        // too)
+        const int64_t ns = ceil_div(B.shell.start[B.shell.nbox], B.pfast ? kRimPts : kChunkPts);
+        for (int64_t c = 0; c < ns; ++c) items->push_back({p, kItemPoints, (int32_t)c, 0, 0, 0});
     }
     std::stable_sort(items->begin(), items->end(),
                      [&](const BItem& a, const BItem& b) { return key(a) < key(b); });
@@ -80,9 +239,13 @@ void batch_items(const std::vector<BProb>& probs, std::vector<BItem>* items,
         const BItem& I = (*items)[k];
         if (groups->empty() || key((*items)[groups->back().first]) != key(I)) {
             const auto t = key(I);
-            groups->push_back({std::get<0>(t), std::get<1>(t), std::get<2>(t), (int32_t)k, 0});
+            groups->push_back({std::get<0>(t), std::get<1>(t), std::get<2>(t), std::get<3>(t),
+                               (int32_t)k, 0, 0});
         }
-        ++groups->back().count;
+        BGroup& g = groups->back();
+        ++g.count;
+        if (I.kind == kItemPatch)
+            g.lds = std::max(g.lds, (int32_t)patch_bytes(*probs[I.prob].hplan, probs[I.prob].K / 2, I.a, I.b, I.c, I.d));
     }
 }
 

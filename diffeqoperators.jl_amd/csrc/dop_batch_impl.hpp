@@ -59,7 +59,7 @@ struct StageBufs {
     T* nxt;
 };
 
-// store of one point: plain apply, or RK4 stage `stage` (see dop_kernels.hip)
+// store of one point: plain apply, or RK4 stage `stage`
 template <typename T>
 __device__ inline void epilogue(const BProb& B, const StageBufs<T>& S, int stage, int accumulate,
                                 int64_t p, double v)
@@ -278,16 +278,18 @@ __device__ void tile1d(const BProb& B, const StageBufs<T>& S, int xg)
     if (out_ok) epilogue_side<T, STAGE>(B, S, x, acc.value(), (double)sa, (double)sb);
 }
 
-// generic chunk: points [c*kChunkPts, ...) of the problem's shell boxes
-template <typename T, int ACC>
+// chunk c of the points of the problem's shell boxes: through shell_point with window KP (1-D and
+// 2-D problems whose plans allow it), or the generic evaluator (KP = 0)
+template <typename T, int ACC, int KP>
 __device__ void shell_chunk(const BProb& B, const StageBufs<T>& S, int stage, int accumulate,
                             int64_t c)
 {
     const PlanDev& P = *B.plan;
     const ShellArgs& SH = B.shell;
     const int64_t total = SH.start[SH.nbox];
-    const int64_t first = c * kChunkPts;
-    for (int j = threadIdx.x; j < kChunkPts; j += kBlock) {
+    constexpr int per = KP ? kRimPts : kChunkPts;
+    const int64_t first = c * per;
+    for (int j = threadIdx.x; j < per; j += kBlock) {
         const int64_t p = first + j;
         if (p >= total) break;
         int b = 0;
@@ -300,11 +302,17 @@ __device__ void shell_chunk(const BProb& B, const StageBufs<T>& S, int stage, in
         idx[1] = SH.org[b][1] + l % e1;
         idx[2] = SH.org[b][2] + l / e1;
         const int64_t lin = idx[0] + idx[1] * P.sdu[1] + idx[2] * P.sdu[2];
-        epilogue<T>(B, S, stage, accumulate, lin, eval_point<T, ACC>(P, S.X, idx));
+        double v;
+        if constexpr (KP != 0) {
+            v = B.nd == 1 ? shell_point<T, ACC, KP, 1>(P, S.X, idx) : shell_point<T, ACC, KP, 2>(P, S.X, idx);
+        } else {
+            v = eval_point<T, ACC>(P, S.X, idx);
+        }
+        epilogue<T>(B, S, stage, accumulate, lin, v);
     }
 }
 
-// one group of 2-D tiles with window K and accumulator ACC, for epilogue STAGE
+// an apply's 2-D tiles with window K and accumulator ACC (STAGE -1, or -2 accumulating)
 template <typename T, int ACC, int K, int STAGE>
 __global__ __launch_bounds__(kBlock) void k_batch_tiles(const BProb* __restrict__ probs,
                                                       const BItem* __restrict__ items, int nitems)
@@ -312,11 +320,11 @@ __global__ __launch_bounds__(kBlock) void k_batch_tiles(const BProb* __restrict_
     for (int it = blockIdx.x; it < nitems; it += gridDim.x) {
         const BItem I = items[it];
         const BProb& B = probs[I.prob];
-        tile2d<T, ACC, K, STAGE>(B, stage_bufs<T>(B, STAGE < 0 ? -1 : STAGE), I.a, I.b);
+        tile2d<T, ACC, K, STAGE>(B, stage_bufs<T>(B, -1), I.a, I.b);
     }
 }
 
-// one group of 1-D tiles with window K and accumulator ACC, for epilogue STAGE
+// an apply's 1-D tiles with window K and accumulator ACC (STAGE -1, or -2 accumulating)
 template <typename T, int ACC, int K, int STAGE>
 __global__ __launch_bounds__(kBlock) void k_batch_tiles1d(const BProb* __restrict__ probs,
                                                         const BItem* __restrict__ items, int nitems)
@@ -324,41 +332,81 @@ __global__ __launch_bounds__(kBlock) void k_batch_tiles1d(const BProb* __restric
     for (int it = blockIdx.x; it < nitems; it += gridDim.x) {
         const BItem I = items[it];
         const BProb& B = probs[I.prob];
-        tile1d<T, ACC, K, STAGE>(B, stage_bufs<T>(B, STAGE < 0 ? -1 : STAGE), I.a);
+        tile1d<T, ACC, K, STAGE>(B, stage_bufs<T>(B, -1), I.a);
     }
 }
 
-// one group of generic point chunks with accumulator ACC
-template <typename T, int ACC>
+// an apply's point chunks with accumulator ACC (KP: shell_point's window, 0 generic)
+template <typename T, int ACC, int KP>
 __global__ __launch_bounds__(kBlock) void k_batch_points(const BProb* __restrict__ probs,
                                                        const BItem* __restrict__ items, int nitems,
-                                                       int stage, int accumulate)
+                                                       int accumulate)
 {
     for (int it = blockIdx.x; it < nitems; it += gridDim.x) {
         const BItem I = items[it];
         const BProb& B = probs[I.prob];
-        shell_chunk<T, ACC>(B, stage_bufs<T>(B, stage), stage, accumulate, I.a);
+        shell_chunk<T, ACC, KP>(B, stage_bufs<T>(B, -1), -1, accumulate, I.a);
+    }
+}
+
+// One RK4 stage's items of one accumulator, any window, of the problems that do not take the
+// one-pass step: the tiles in one launch, the points in another (a launch per kind and window, 25
+// of 5-25 us each for a mixed batch, made the chain of the four stages 1.45 ms of a step).
+template <typename T, int ACC, int K, int STAGE>
+__device__ void stage_item(const BProb& B, const StageBufs<T>& S, const BItem& I)
+{
+    if (I.kind == kItemTile1) tile1d<T, ACC, K, STAGE>(B, S, I.a);
+    else tile2d<T, ACC, K, STAGE>(B, S, I.a, I.b);
+}
+
+template <typename T, int ACC, int STAGE>
+__global__ __launch_bounds__(kBlock) void k_batch_stage(const BProb* __restrict__ probs,
+                                                      const BItem* __restrict__ items, int nitems)
+{
+    for (int it = blockIdx.x; it < nitems; it += gridDim.x) {
+        const BItem I = items[it];
+        const BProb& B = probs[I.prob];
+        const StageBufs<T> S = stage_bufs<T>(B, STAGE);
+        switch (B.K) {
+        case 3: stage_item<T, ACC, 3, STAGE>(B, S, I); break;
+        case 5: stage_item<T, ACC, 5, STAGE>(B, S, I); break;
+        case 7: stage_item<T, ACC, 7, STAGE>(B, S, I); break;
+        case 9: stage_item<T, ACC, 9, STAGE>(B, S, I); break;
+        case 11: stage_item<T, ACC, 11, STAGE>(B, S, I); break;
+        }
+    }
+}
+
+template <typename T, int ACC>
+__global__ __launch_bounds__(kBlock) void k_batch_stage_points(const BProb* __restrict__ probs,
+                                                             const BItem* __restrict__ items,
+                                                             int nitems, int stage)
+{
+    for (int it = blockIdx.x; it < nitems; it += gridDim.x) {
+        const BItem I = items[it];
+        const BProb& B = probs[I.prob];
+        const StageBufs<T> S = stage_bufs<T>(B, stage);
+        if (B.pfast) shell_chunk<T, ACC, kMaxBatchTileK>(B, S, stage, 0, I.a);
+        else shell_chunk<T, ACC, 0>(B, S, stage, 0, I.a);
     }
 }
 
 template <typename T, int ACC, int K>
-hipError_t launch_tiles(int kind, int st, dim3 gr, const BProb* probs, const BItem* it, int n,
+hipError_t launch_tiles(int kind, int accumulate, dim3 gr, const BProb* probs, const BItem* it, int n,
                         hipStream_t s)
 {
-    switch (st) {
 #define DOP_BS(SS)                                                                               \
-    case SS:                                                                                      \
-        if (kind == 2)                                                                            \
+    do {                                                                                          \
+        if (kind == kItemTile1)                                                                   \
             hipLaunchKernelGGL((k_batch_tiles1d<T, ACC, K, SS>), gr, dim3(kBlock), 0, s, probs,  \
                                it, n);                                                            \
         else                                                                                      \
             hipLaunchKernelGGL((k_batch_tiles<T, ACC, K, SS>), gr, dim3(kBlock), 0, s, probs, it, \
                                n);                                                                \
-        return hipGetLastError();
-        DOP_BS(-2) DOP_BS(-1) DOP_BS(0) DOP_BS(1) DOP_BS(2) DOP_BS(3)
+    } while (0)
+    if (accumulate) DOP_BS(-2); else DOP_BS(-1);
 #undef DOP_BS
-    }
-    return hipErrorInvalidValue;
+    return hipGetLastError();
 }
 
 template <typename T, int ACC>
@@ -367,18 +415,41 @@ hipError_t launch_group(const BGroup& g, const BProb* probs, const BItem* items,
 {
     const dim3 gr((unsigned)(g.count < grid ? g.count : grid));
     const BItem* it = items + g.first;
-    if (g.kind == 1) {
-        hipLaunchKernelGGL((k_batch_points<T, ACC>), gr, dim3(kBlock), 0, s, probs, it, g.count,
-                           stage, accumulate);
+    if (g.kind == kItemStage) {
+        switch (stage) {
+#define DOP_BR(SS)                                                                                \
+    case SS:                                                                                      \
+        hipLaunchKernelGGL((k_batch_stage<T, ACC, SS>), gr, dim3(kBlock), 0, s, probs, it, g.count);\
+        return hipGetLastError();
+            DOP_BR(0) DOP_BR(1) DOP_BR(2) DOP_BR(3)
+#undef DOP_BR
+        }
+        return hipErrorInvalidValue;
+    }
+    if (stage >= 0) {
+        if (g.kind != kItemPoints) return hipErrorInvalidValue;
+        hipLaunchKernelGGL((k_batch_stage_points<T, ACC>), gr, dim3(kBlock), 0, s, probs, it, g.count,
+                           stage);
         return hipGetLastError();
     }
-    const int st = stage < 0 ? (accumulate ? -2 : -1) : stage;
+    if (g.kind == kItemPoints) {
+        switch (g.K) {
+#define DOP_BP(KP)                                                                                \
+    case KP:                                                                                      \
+        hipLaunchKernelGGL((k_batch_points<T, ACC, KP>), gr, dim3(kBlock), 0, s, probs, it, g.count, \
+                           accumulate);                                                           \
+        return hipGetLastError();
+            DOP_BP(0) DOP_BP(3) DOP_BP(5) DOP_BP(7) DOP_BP(9) DOP_BP(11)
+#undef DOP_BP
+        }
+        return hipErrorInvalidValue;
+    }
     switch (g.K) {
-    case 3: return launch_tiles<T, ACC, 3>(g.kind, st, gr, probs, it, g.count, s);
-    case 5: return launch_tiles<T, ACC, 5>(g.kind, st, gr, probs, it, g.count, s);
-    case 7: return launch_tiles<T, ACC, 7>(g.kind, st, gr, probs, it, g.count, s);
-    case 9: return launch_tiles<T, ACC, 9>(g.kind, st, gr, probs, it, g.count, s);
-    case 11: return launch_tiles<T, ACC, 11>(g.kind, st, gr, probs, it, g.count, s);
+    case 3: return launch_tiles<T, ACC, 3>(g.kind, accumulate, gr, probs, it, g.count, s);
+    case 5: return launch_tiles<T, ACC, 5>(g.kind, accumulate, gr, probs, it, g.count, s);
+    case 7: return launch_tiles<T, ACC, 7>(g.kind, accumulate, gr, probs, it, g.count, s);
+    case 9: return launch_tiles<T, ACC, 9>(g.kind, accumulate, gr, probs, it, g.count, s);
+    case 11: return launch_tiles<T, ACC, 11>(g.kind, accumulate, gr, probs, it, g.count, s);
     }
     return hipErrorInvalidValue;
 }
@@ -397,7 +468,7 @@ hipError_t launch_group_any(const BGroup& g, const BProb* probs, const BItem* it
         if (g.acc == kAccF32Wide)
             return launch_group<T, kAccF32Wide>(g, probs, items, stage, accumulate, grid, s);
         if (g.acc == kAccF64) {
-            if (g.kind != 1) return hipErrorInvalidValue;
+            if (g.kind != kItemPoints) return hipErrorInvalidValue;
             return launch_group<T, kAccF64>(g, probs, items, stage, accumulate, grid, s);
         }
         return launch_group<T, kAccF32>(g, probs, items, stage, accumulate, grid, s);

@@ -312,8 +312,9 @@ DOP_HD inline bool shell_point_ok(const PlanDev& P, int KM)
     return true;
 }
 
-template <typename T, int ACC, int KM, int ND>
-DOP_HD inline double shell_point(const PlanDev& P, const T* src, const int64_t* idx)
+// ld(a, j): element j of the point's line along axis a, as T's compute type
+template <typename T, int ACC, int KM, int ND, typename F>
+DOP_HD inline double shell_point_f(const PlanDev& P, const int64_t* idx, const F& ld)
 {
     using C = typename Store<T>::C;
     using W = typename Acc<ACC>::W;
@@ -326,22 +327,16 @@ DOP_HD inline double shell_point(const PlanDev& P, const T* src, const int64_t* 
 #pragma unroll
     for (int a = 0; a < ND; ++a) {
         const AxisDev& X = P.ax[a];
-        int64_t base = P.tshift[a];
-#pragma unroll
-        for (int b = 0; b < ND; ++b)
-            if (b != a) base += idx[b] * P.ssrc[b];
-        const int64_t S = P.ssrc[a];
         const int r = (int)idx[a];
         if (r >= X.rlo && r < X.rhi) {
             nt[a] = ng[a] = J0[a] = 0;
             const W* wt = Acc<ACC>::table(X) + (X.uniform ? 0 : r);
             const int64_t ws = X.uniform ? 1 : X.n;
-            const int64_t p0 = base + (int64_t)(r + X.dmin) * S;
 #pragma unroll
             for (int k = 0; k < KM; ++k) {
                 if (k < X.K) {
                     w[a][k] = (double)tab(wt, k * ws);
-                    v[a][k] = (C)Store<T>::ld(src, p0 + k * S);
+                    v[a][k] = ld(a, r + X.dmin + k);
                 }
             }
         } else {
@@ -355,12 +350,12 @@ DOP_HD inline double shell_point(const PlanDev& P, const T* src, const int64_t* 
                 if (k < X.KB) w[a][k] = tab(wr, k);
             ng[a] = left ? X.nl : X.nr;
             const double* al = left ? X.al : X.ar;
-            const int64_t o = left ? 0 : (int64_t)X.n - X.nr;
+            const int o = left ? 0 : X.n - X.nr;
 #pragma unroll
             for (int k = 0; k < kPointGhost; ++k) {
                 if (k < ng[a]) {
                     ga[a][k] = tab(al, k);
-                    gv[a][k] = (C)Store<T>::ld(src, base + (o + k) * S);
+                    gv[a][k] = ld(a, o + k);
                 }
             }
             gc[a] = left ? tab(&X.bl, 0) : tab(&X.br, 0);
@@ -371,16 +366,12 @@ DOP_HD inline double shell_point(const PlanDev& P, const T* src, const int64_t* 
     for (int a = 0; a < ND; ++a) {
         if (nt[a] == 0) continue;
         const AxisDev& X = P.ax[a];
-        int64_t base = P.tshift[a];
-#pragma unroll
-        for (int b = 0; b < ND; ++b)
-            if (b != a) base += idx[b] * P.ssrc[b];
 #pragma unroll
         for (int k = 0; k < KT; ++k) {
             if (k < nt[a]) {
                 int j = J0[a] + k - 1;
                 j = j < 0 ? 0 : j >= X.n ? X.n - 1 : j;
-                v[a][k] = (C)Store<T>::ld(src, base + (int64_t)j * P.ssrc[a]);
+                v[a][k] = ld(a, j);
             }
         }
     }
@@ -410,6 +401,42 @@ DOP_HD inline double shell_point(const PlanDev& P, const T* src, const int64_t* 
         }
     }
     return acc.value();
+}
+
+template <typename T, int ACC, int KM, int ND>
+DOP_HD inline double shell_point(const PlanDev& P, const T* src, const int64_t* idx)
+{
+    using C = typename Store<T>::C;
+    int64_t base[ND];   // start of the point's line along each axis
+#pragma unroll
+    for (int a = 0; a < ND; ++a) {
+        base[a] = P.tshift[a];
+#pragma unroll
+        for (int b = 0; b < ND; ++b)
+            if (b != a) base[a] += idx[b] * P.ssrc[b];
+    }
+    return shell_point_f<T, ACC, KM, ND>(P, idx, [&](int a, int j) -> C {
+        return (C)Store<T>::ld(src, base[a] + (int64_t)j * P.ssrc[a]);
+    });
+}
+
+// The rows of a line that rows [*lo, *hi) read: their windows, the tiles' window of H on each side
+// included, boundary rows' windows and ghosts (plans that meet shell_point_ok).
+DOP_HD inline void rows_reach(const AxisDev& X, int H, int* lo, int* hi)
+{
+    const int l = *lo, h = *hi, n = X.n;
+    const bool left = l < X.rlo, right = h > X.rhi;   // boundary rows among them
+    int a = l - H, b = h + H;
+    if (left) {
+        a = 0;
+        if (b < X.rlo + X.KB) b = X.rlo + X.KB;
+    }
+    if (right) {
+        b = n;
+        if (a > X.rhi - X.KB) a = X.rhi - X.KB;
+    }
+    *lo = a < 0 ? 0 : a;
+    *hi = b > n ? n : b;
 }
 
 }  // namespace dop

@@ -19,6 +19,7 @@ struct DevicePlan {
     int generic_only = 0;   // every point on k_apply_generic (no tiles, no single-axis kernel)
 };
 
+#if defined(__clang__)   // (device code; the host-only check builds with g++)
 // Four consecutive values as one vector load / store (element-aligned: addresses need not be
 // 16-byte aligned).
 template <typename T>
@@ -55,6 +56,8 @@ struct Quad<double> {
         *reinterpret_cast<V*>(p + 2) = b;
     }
 };
+
+#endif
 
 constexpr int kBlock = 256;        // threads per block
 constexpr int kChunkPts = 1024;    // points per chunk of a persistent launch

@@ -43,6 +43,7 @@ struct dop_batch {
     int storage = 0;
     int grid = 0;
     int chunk = 16;
+    bool rk4 = false;             // work items of RK4 steps
     ~dop_batch()
     {
         if (d_probs) (void)hipFree(d_probs);
@@ -53,12 +54,15 @@ struct dop_batch {
 struct dop_rk4 {
     dop_batch b;
     std::vector<void*> bufs;
-    hipGraph_t graph = nullptr;
-    hipGraphExec_t exec = nullptr;
+    // [0]: two steps (fused problems end in u again); [1]: one step and the copy back to u
+    hipGraph_t graph[2] = {nullptr, nullptr};
+    hipGraphExec_t exec[2] = {nullptr, nullptr};
     ~dop_rk4()
     {
-        if (exec) (void)hipGraphExecDestroy(exec);
-        if (graph) (void)hipGraphDestroy(graph);
+        for (int k = 0; k < 2; ++k) {
+            if (exec[k]) (void)hipGraphExecDestroy(exec[k]);
+            if (graph[k]) (void)hipGraphDestroy(graph[k]);
+        }
         for (void* p : bufs) (void)hipFree(p);
     }
 };

@@ -1,0 +1,506 @@
+// dop_rk4_impl.hpp -- classical RK4 steps of 1-D and 2-D problems in one pass over their grids.
+//
+// Stage by stage a step moves 16 values per point through memory (stage 0 reads u and writes the
+// stage sum and the next stage's input, ...: 64 bytes per f32 point) and is a chain of four launch
+// sets.  Here u is read once and the new state written once (8 bytes per point), by two kernels that
+// do not depend on each other:
+//
+// k_rk4_march, the bulk of a 2-D grid: a wave marches down a segment of rows with the four stages
+// following each other H rows apart.  While row c of u arrives, stage 0 forms row c of its output,
+// stage 1 row c - H, stage 2 row c - 2H and stage 3 the new state's row c - 3H, each from a
+// register ring of the K rows of the stage before it.  Segments overlap by the 4H columns a step's
+// cone reaches on each side and chunks of rows by 3H rows, recomputed: 10 % and 14 % more work at
+// K = 7 and 64 rows.  It covers the box [flo, fhi) whose cone holds regular rows only.
+// Registers: four rings of K + 1 rows of VX points (f32, K = 7: 128), two waves per SIMD; the stage
+// sums between stages wait in LDS (3H + 1 rows per lane), u of stage 2's row is read again (it is
+// in L2).  Bound by its own instructions (f32, K = 7: 22 a point and stage, DPP shifts at a third
+// of the FMA rate among them).
+//
+// k_rk4_patch, the rim of the box (or all of a small or 1-D grid): a block loads a patch with all
+// that its points' cones reach (rows_reach: windows, boundary rows, ghosts) into LDS and runs the
+// four stages there, each over the region the next one reads.
+//
+// Every stage value is rounded to the storage type exactly where the stage-wise kernels store it,
+// and every sum runs in their order, so the new state is the same bit for bit.  The new state goes
+// to acc, so u and acc swap roles from step to step.
+// Measured against the stage-wise step: 256 mixed f32 problems (1-D to 65536, 2-D to 2048 squared,
+// orders 2 to 8) 2.08 -> 1.71 ms a step, 24 served 2-D requests of 100 steps 36.7 -> 25.1 ms.
+#pragma once
+#include "dop_batch_impl.hpp"
+
+namespace dop {
+namespace batch {
+
+// VX consecutive values, element-aligned
+template <typename T, int VX>
+struct RowIO {
+    static constexpr int N = VX * (int)sizeof(T) < 16 ? VX : 16 / (int)sizeof(T);
+    static_assert(VX % N == 0, "whole vector loads");
+    typedef T V __attribute__((ext_vector_type(N), aligned(sizeof(T))));
+    __device__ static void ld(const T* p, T* o)
+    {
+#pragma unroll
+        for (int g = 0; g < VX / N; ++g) {
+            const V v = *reinterpret_cast<const V*>(p + g * N);
+#pragma unroll
+            for (int i = 0; i < N; ++i) o[g * N + i] = v[i];
+        }
+    }
+    __device__ static void st(T* p, const T* o)
+    {
+#pragma unroll
+        for (int g = 0; g < VX / N; ++g) {
+            V v;
+#pragma unroll
+            for (int i = 0; i < N; ++i) v[i] = o[g * N + i];
+            *reinterpret_cast<V*>(p + g * N) = v;
+        }
+    }
+};
+
+// x windows xw[e] = u(xs - H + e), e < VX + 2H, of a lane's VX points (DPP shifts; the lanes at
+// the wave's ends get zeros for what lies beyond it, and their outputs are never used)
+template <typename T, int VX, int H>
+__device__ inline void march_window(const T* own, T* xw)
+{
+    constexpr int DL = (H + VX - 1) / VX;
+#pragma unroll
+    for (int v = 0; v < VX; ++v) xw[H + v] = own[v];
+    T l[VX], r[VX];
+#pragma unroll
+    for (int v = 0; v < VX; ++v) l[v] = r[v] = own[v];
+#pragma unroll
+    for (int d = 1; d <= DL; ++d) {
+#pragma unroll
+        for (int v = 0; v < VX; ++v) {
+            // value v of the lane at distance d lands in the window (and so do the nearer ones)
+            const int el = H - d * VX + v, er = H + VX + (d - 1) * VX + v;
+            if (el >= 0) {
+                l[v] = shr1(l[v]);
+                xw[el] = l[v];
+            }
+            if (er < VX + 2 * H) {
+                r[v] = shl1(r[v]);
+                xw[er] = r[v];
+            }
+        }
+    }
+}
+
+template <typename W>
+__device__ inline W const_tab(const W* p, int64_t i)
+{
+    // plan tables do not change while a launch reads them: scalar loads for uniform indices
+    return ((const __attribute__((address_space(4))) W*)p)[i];
+}
+
+template <typename T, int ACC, int K, bool UNI>
+__global__ __launch_bounds__(64, 2) void k_rk4_march(const BProb* __restrict__ probs,
+                                                     const BItem* __restrict__ items, int nitems,
+                                                     int parity)
+{
+    using W = typename Acc<ACC>::W;
+    constexpr int VX = march_vx(sizeof(T) == 8 ? kF64 : kF32, ACC, K);
+    constexpr int H = K / 2;
+    constexpr int R = K + 1;                       // ring rows: the window and one row ahead
+    constexpr int PAD = (4 * H + VX - 1) / VX * VX;   // columns recomputed on each side
+    constexpr int OUT = 64 * VX - 2 * PAD;
+    constexpr int D = 3 * H + 1;                   // rows a stage sum waits
+    __shared__ __attribute__((aligned(16))) T sums[D][64][VX];
+    const int lane = threadIdx.x;
+    for (int it = blockIdx.x; it < nitems; it += gridDim.x) {
+        const BItem I = items[it];
+        const BProb& B = probs[I.prob];
+        const int seg = I.a;
+        const T* u = (const T*)(parity ? B.acc : B.u);
+        T* out = (T*)(parity ? B.u : B.acc);
+        const int y0 = B.flo[1] + I.b * B.fchunk;
+        const int y1 = min(y0 + B.fchunk, B.fhi[1]);
+        const int n0 = (int)B.n0, n1 = (int)B.n1;
+        const int64_t s1 = B.ys;
+        const int xb = B.flo[0] + seg * OUT;        // first output column of the segment
+        const int xs = xb - PAD + lane * VX;
+        const int xe = min(xb + OUT, B.fhi[0]);
+        const bool st_ok = xs >= xb && xs < xe;     // whole groups: OUT and the box are multiples of VX
+        // lanes beyond the array load another group; no output's cone reaches them
+        const int xl = min(max(xs, 0), n0 - VX);
+        const T* ucol = u + xl;
+        const W* wxt = btab<ACC>(B, 0);
+        const W* wyt = btab<ACC>(B, 1);
+        W wx[UNI ? 1 : VX][K], wyu[UNI ? K : 1];
+#pragma unroll
+        for (int v = 0; v < (UNI ? 1 : VX); ++v) {
+            const int64_t xr = UNI ? 0 : min(max(xs + v, 0), n0 - 1);
+#pragma unroll
+            for (int k = 0; k < K; ++k) wx[v][k] = UNI ? const_tab(wxt, k) : wxt[xr * K + k];
+        }
+        if constexpr (UNI) {
+#pragma unroll
+            for (int k = 0; k < K; ++k) wyu[k] = const_tab(wyt, k);
+        }
+        const double scale = B.scale, dt = B.dt;
+        const int ylast = min(y1 + 4 * H - 1, n1 - 1);
+        auto load_row = [&](int row, T* dst) {
+            RowIO<T, VX>::ld(ucol + (int64_t)min(max(row, 0), ylast) * s1, dst);
+        };
+        // rings: slot (t + k) % R of step t holds row c - H + k of u (q[0]) and row
+        // c - jH - H + k of stage j's input (q[j])
+        T q[4][R][VX];
+        const int c0 = y0 - 3 * H;
+#pragma unroll
+        for (int s = 0; s < R - 1; ++s) load_row(c0 - H + s, q[0][s]);
+        // slots of the waiting sums: rows c, c - H, c - 2H, c - 3H
+        int d0 = 0, d1 = D - H, d2 = D - 2 * H, d3 = D - 3 * H;
+        const int steps = (y1 - y0) + 6 * H;
+        for (int t0 = 0; t0 < steps; t0 += R) {
+            auto step = [&](auto jc) -> bool {
+                constexpr int j = decltype(jc)::value;
+                const int t = t0 + j;
+                if (t >= steps) return false;
+                const int c = c0 + t;
+                load_row(c + H + 1, q[0][(j + K) % R]);
+                T ue[VX];   // u at stage 2's row
+                load_row(c - 2 * H, ue);
+                // one stage: row y of its values v from the window rows of ring Q
+                auto values = [&](const T(*Q)[VX], int y, double* val) {
+                    T xw[VX + 2 * H];
+                    march_window<T, VX, H>(Q[(j + H) % R], xw);
+                    W wy[K];
+#pragma unroll
+                    for (int k = 0; k < K; ++k) wy[k] = UNI ? wyu[UNI ? k : 0] : const_tab(wyt, (int64_t)y * K + k);
+#pragma unroll
+                    for (int v = 0; v < VX; ++v) {
+                        Acc<ACC> a;
+#pragma unroll
+                        for (int k = 0; k < K; ++k) a.add(wx[UNI ? 0 : v][k], (W)xw[v + k]);
+#pragma unroll
+                        for (int k = 0; k < K; ++k) a.add(wy[k], (W)Q[(j + k) % R][v]);
+                        val[v] = a.value();
+                    }
+                };
+                double val[VX];
+                T sum[VX];
+                constexpr int nw = (j + K - 1) % R;   // slot of the row a stage adds to the next ring
+                // stage 0, row c
+                values(q[0], c, val);
+#pragma unroll
+                for (int v = 0; v < VX; ++v) {
+                    const double k = scale * val[v];
+                    const double up = (double)q[0][(j + H) % R][v];
+                    sum[v] = (T)(up + (dt / 6.0) * k);
+                    q[1][nw][v] = (T)(up + (0.5 * dt) * k);
+                }
+                RowIO<T, VX>::st(&sums[d0][lane][0], sum);
+                if (t >= 2 * H) {   // stage 1, row c - H (wave-uniform)
+                    RowIO<T, VX>::ld(&sums[d1][lane][0], sum);
+                    values(q[1], c - H, val);
+#pragma unroll
+                    for (int v = 0; v < VX; ++v) {
+                        const double k = scale * val[v];
+                        const double up = (double)q[0][j % R][v];
+                        sum[v] = (T)((double)sum[v] + (dt / 3.0) * k);
+                        q[2][nw][v] = (T)(up + (0.5 * dt) * k);
+                    }
+                    RowIO<T, VX>::st(&sums[d1][lane][0], sum);
+                }
+                if (t >= 4 * H) {   // stage 2, row c - 2H
+                    RowIO<T, VX>::ld(&sums[d2][lane][0], sum);
+                    values(q[2], c - 2 * H, val);
+#pragma unroll
+                    for (int v = 0; v < VX; ++v) {
+                        const double k = scale * val[v];
+                        const double up = (double)ue[v];
+                        sum[v] = (T)((double)sum[v] + (dt / 3.0) * k);
+                        q[3][nw][v] = (T)(up + dt * k);
+                    }
+                    RowIO<T, VX>::st(&sums[d2][lane][0], sum);
+                }
+                if (t >= 6 * H) {   // stage 3, row c - 3H: the new state
+                    RowIO<T, VX>::ld(&sums[d3][lane][0], sum);
+                    values(q[3], c - 3 * H, val);
+#pragma unroll
+                    for (int v = 0; v < VX; ++v) {
+                        const double k = scale * val[v];
+                        sum[v] = (T)((double)sum[v] + (dt / 6.0) * k);
+                    }
+                    if (st_ok) RowIO<T, VX>::st(out + (int64_t)(c - 3 * H) * s1 + xs, sum);
+                }
+                d0 = d0 + 1 == D ? 0 : d0 + 1;
+                d1 = d1 + 1 == D ? 0 : d1 + 1;
+                d2 = d2 + 1 == D ? 0 : d2 + 1;
+                d3 = d3 + 1 == D ? 0 : d3 + 1;
+                return true;
+            };
+            if (!ring_steps<0, R>(step)) break;
+        }
+    }
+}
+
+// A patch in LDS, all of it addressed by offsets into one array (elements of T after the head; never
+// by a pointer biased by the patch's origin, which would leave the LDS aperture): u at 0, the two
+// stage arrays at sz and 2 sz, the sums of the patch's own points at 3 sz.  The head holds the
+// regions of the four stages: lo[x], hi[x], lo[y], hi[y] of stage s at 4 s.
+struct Patch {
+    int o0, o1;          // grid coordinates of the first loaded point
+    int pitch, sz;       // row pitch (odd: lanes along y hit different banks), points loaded
+    int a0, a1, ow;      // first own point, own points per row
+};
+
+extern __shared__ __attribute__((aligned(16))) char patch_lds[];
+
+__device__ inline int patch_region(int s, int i)
+{
+    return __builtin_amdgcn_readfirstlane(reinterpret_cast<const int*>(patch_lds)[4 * s + i]);
+}
+template <typename T>
+__device__ inline T& patch_at(int i)
+{
+    return reinterpret_cast<T*>(patch_lds + kPatchHead)[i];
+}
+
+// Stage s of a point: its row's sum v to the stage sum and the next stage's input (own: one of the
+// patch's own points, p its offset in the loaded area, q among the own points)
+template <typename T>
+__device__ inline void patch_update(const Patch& Q, int s, double k, double dt, int p, int q, bool own,
+                                    T* o)
+{
+    if (s == 3) {
+        *o = (T)((double)patch_at<T>(3 * Q.sz + q) + (dt / 6.0) * k);
+        return;
+    }
+    const double up = (double)patch_at<T>(p);
+    if (own) {
+        T& sum = patch_at<T>(3 * Q.sz + q);
+        sum = s == 0 ? (T)(up + (dt / 6.0) * k) : (T)((double)sum + (dt / 3.0) * k);
+    }
+    const double h = (s == 2) ? dt : 0.5 * dt;
+    patch_at<T>((s == 1 ? 2 : 1) * Q.sz + p) = (T)(up + h * k);
+}
+
+// Stage s of a patch over the block: lanes along axis L (0: x), rows along the other one.  A wave
+// takes 64 lines along L and a part of the rows; the weights along L stay in its registers, a
+// row's are the same for the wave.  Points whose rows are regular on both axes (in the tiles'
+// natural box) read their windows from LDS; the others go through shell_point_f.
+template <typename T, int ACC, int K, int L>
+__device__ inline void patch_stage(const BProb& B, const PlanDev& P, const Patch& Q, int s,
+                                   T* __restrict__ out)
+{
+    using W = typename Acc<ACC>::W;
+    constexpr int H = K / 2, M = 1 - L;
+    const int l0 = patch_region(s, 2 * L), l1 = patch_region(s, 2 * L + 1);
+    const int m0 = patch_region(s, 2 * M), m1 = patch_region(s, 2 * M + 1);
+    const int ol = L == 0 ? Q.o0 : Q.o1, om = L == 0 ? Q.o1 : Q.o0;
+    const int b0 = patch_region(3, 1), b1 = patch_region(3, 3);   // the own points' end
+    const int in = (s == 0 ? 0 : s == 2 ? 2 : 1) * Q.sz;
+    const double scale = B.scale, dt = B.dt;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int nl = (l1 - ol + 63) >> 6;             // groups of lines (from the patch's origin)
+    const int parts = nl == 1 ? 4 : nl <= 3 ? 2 : 1;
+    const int per = (m1 - m0 + parts - 1) / parts;
+    const bool uL = B.uniform[L] != 0, uM = B.uniform[M] != 0;
+    const W* wlt = btab<ACC>(B, L);
+    const W* wmt = btab<ACC>(B, M);
+    const int sl = L == 0 ? 1 : Q.pitch, sm = L == 0 ? Q.pitch : 1;   // LDS strides
+    for (int unit = wave; unit < nl * parts; unit += 4) {
+        const int g = unit % nl, part = unit / nl;
+        const int l = ol + g * 64 + lane;
+        const bool lin = l >= l0 && l < l1;
+        if (__builtin_amdgcn_ballot_w64(lin) == 0) continue;
+        const bool lreg = l >= B.lo[L] && l < B.hi[L];
+        W wl[K];
+#pragma unroll
+        for (int k = 0; k < K; ++k)
+            wl[k] = lin && lreg ? wlt[(uL ? 0 : (int64_t)l * K) + k] : W(0);
+        const int mb = m0 + part * per, me = min(mb + per, m1);
+        for (int m = mb; m < me; ++m) {
+            if (!lin) continue;
+            const bool mreg = m >= B.lo[M] && m < B.hi[M];   // wave-uniform
+            const int p = (l - ol) * sl + (m - om) * sm;
+            const int x = L == 0 ? l : m, y = L == 0 ? m : l;
+            double v;
+            if (lreg && mreg) {
+                T tl[K], tm[K];
+                W wm[K];
+#pragma unroll
+                for (int k = 0; k < K; ++k) {
+                    tl[k] = patch_at<T>(in + (p + (k - H) * sl));
+                    tm[k] = patch_at<T>(in + (p + (k - H) * sm));
+                    wm[k] = const_tab(wmt, (uM ? 0 : (int64_t)m * K) + k);
+                }
+                Acc<ACC> a;
+#pragma unroll
+                for (int k = 0; k < K; ++k) a.add(L == 0 ? wl[k] : wm[k], (W)(L == 0 ? tl[k] : tm[k]));
+#pragma unroll
+                for (int k = 0; k < K; ++k) a.add(L == 0 ? wm[k] : wl[k], (W)(L == 0 ? tm[k] : tl[k]));
+                v = a.value();
+            } else {
+                const int64_t idx[3] = {x, y, 0};
+                const int px = x - Q.o0, py = y - Q.o1;
+                v = shell_point_f<T, ACC, K, 2>(P, idx, [&](int a, int j) -> T {
+                    return a == 0 ? patch_at<T>(in + (py * Q.pitch + (j - Q.o0)))
+                                  : patch_at<T>(in + ((j - Q.o1) * Q.pitch + px));
+                });
+            }
+            const bool own = x >= Q.a0 && x < b0 && y >= Q.a1 && y < b1;
+            patch_update<T>(Q, s, scale * v, dt, p, (y - Q.a1) * Q.ow + (x - Q.a0), own,
+                            out + ((int64_t)y * B.ys + x));
+        }
+    }
+}
+
+// The same for a 1-D patch: lines of one point
+template <typename T, int ACC, int K>
+__device__ inline void patch_stage1(const BProb& B, const PlanDev& P, const Patch& Q, int s,
+                                    T* __restrict__ out)
+{
+    using W = typename Acc<ACC>::W;
+    constexpr int H = K / 2;
+    const int x0 = patch_region(s, 0), x1 = patch_region(s, 1), b0 = patch_region(3, 1);
+    const int in = (s == 0 ? 0 : s == 2 ? 2 : 1) * Q.sz;
+    const double scale = B.scale, dt = B.dt;
+    const W* wt = btab<ACC>(B, 0);
+    const bool uni = B.uniform[0] != 0;
+    for (int x = x0 + (int)threadIdx.x; x < x1; x += kBlock) {
+        const int p = x - Q.o0;
+        double v;
+        if (x >= B.lo[0] && x < B.hi[0]) {
+            Acc<ACC> a;
+#pragma unroll
+            for (int k = 0; k < K; ++k)
+                a.add(wt[(uni ? 0 : (int64_t)x * K) + k], (W)patch_at<T>(in + (p - H + k)));
+            v = a.value();
+        } else {
+            const int64_t idx[3] = {x, 0, 0};
+            v = shell_point_f<T, ACC, K, 1>(
+                P, idx, [&](int, int j) -> T { return patch_at<T>(in + (j - Q.o0)); });
+        }
+        patch_update<T>(Q, s, scale * v, dt, p, x - Q.a0, x >= Q.a0 && x < b0, out + x);
+    }
+}
+
+// The points [a, b) x [c, d) of a problem.
+template <typename T, int ACC, int K>
+__global__ __launch_bounds__(kBlock) void k_rk4_patch(const BProb* __restrict__ probs,
+                                                    const BItem* __restrict__ items, int nitems,
+                                                    int parity)
+{
+    for (int it = blockIdx.x; it < nitems; it += gridDim.x) {
+        const BItem I = items[it];
+        const BProb& B = probs[I.prob];
+        const PlanDev& P = *B.plan;
+        const T* src = (const T*)(parity ? B.acc : B.u);
+        T* out = (T*)(parity ? B.u : B.acc);
+        int x0 = I.a, x1 = I.b, y0 = I.c, y1 = I.d;
+        int* reg = reinterpret_cast<int*>(patch_lds);
+#pragma unroll
+        for (int s = 3; s >= 0; --s) {
+            if (threadIdx.x == 0) {
+                reg[4 * s] = x0;
+                reg[4 * s + 1] = x1;
+                reg[4 * s + 2] = y0;
+                reg[4 * s + 3] = y1;
+            }
+            rows_reach(P.ax[0], K / 2, &x0, &x1);
+            if (B.nd == 2) rows_reach(P.ax[1], K / 2, &y0, &y1);
+        }
+        const int lh = y1 - y0;
+        Patch Q;
+        Q.o0 = x0;
+        Q.o1 = y0;
+        Q.pitch = (x1 - x0) | 1;
+        Q.sz = Q.pitch * lh;
+        Q.a0 = I.a;
+        Q.a1 = I.c;
+        Q.ow = I.b - I.a;
+        // load: rows in turn (32-bit reciprocal of the width, exact for the fewer than 2^14 points
+        // of a patch)
+        const uint32_t w = (uint32_t)(x1 - x0), n = w * (uint32_t)lh;
+        const uint32_t mul = w > 1 ? (uint32_t)((0x100000000ull + w - 1) / w) : 0;
+        const T* s0 = src + (int64_t)y0 * B.ys + x0;
+        for (uint32_t p = threadIdx.x; p < n; p += kBlock) {
+            const uint32_t q = w > 1 ? __umulhi(p, mul) : p;
+            patch_at<T>((int)(q * Q.pitch + (p - q * w))) = s0[(int64_t)q * B.ys + (p - q * w)];
+        }
+        __syncthreads();
+#pragma unroll 1
+        for (int s = 0; s < 4; ++s) {
+            if (B.nd == 1) patch_stage1<T, ACC, K>(B, P, Q, s, out);
+            else if ((int)w >= lh) patch_stage<T, ACC, K, 0>(B, P, Q, s, out);
+            else patch_stage<T, ACC, K, 1>(B, P, Q, s, out);
+            __syncthreads();
+        }
+    }
+}
+
+// the copy that brings a fused problem's new state back from acc to u after an odd number of steps
+template <typename T>
+__global__ __launch_bounds__(kBlock) void k_rk4_back(const BProb* __restrict__ probs,
+                                                     const BItem* __restrict__ items, int nitems)
+{
+    constexpr int VX = 16 / (int)sizeof(T);
+    for (int it = blockIdx.x; it < nitems; it += gridDim.x) {
+        const BItem I = items[it];
+        const BProb& B = probs[I.prob];
+        const T* src = (const T*)B.acc;
+        T* dst = (T*)B.u;
+        const int64_t total = B.plan->total;
+        const int64_t first = (int64_t)I.a * kBackPts;
+        const int64_t end = min(first + kBackPts, total);
+        int64_t p = first + (int64_t)threadIdx.x * VX;
+        for (; p + VX <= end; p += kBlock * VX) {
+            T v[VX];
+            RowIO<T, VX>::ld(src + p, v);
+            RowIO<T, VX>::st(dst + p, v);
+        }
+        for (; p < end; ++p) dst[p] = src[p];   // the end's partial group (one thread)
+    }
+}
+
+template <typename T, int ACC, int K>
+hipError_t launch_march(bool uni, dim3 gr, const BProb* probs, const BItem* it, int n, int parity,
+                        hipStream_t s)
+{
+    if (uni)
+        hipLaunchKernelGGL((k_rk4_march<T, ACC, K, true>), gr, dim3(64), 0, s, probs, it, n, parity);
+    else
+        hipLaunchKernelGGL((k_rk4_march<T, ACC, K, false>), gr, dim3(64), 0, s, probs, it, n, parity);
+    return hipGetLastError();
+}
+
+template <typename T, int ACC>
+hipError_t launch_pass_group(const BGroup& g, const BProb* probs, const BItem* items, int parity,
+                             int grid, hipStream_t s)
+{
+    const BItem* it = items + g.first;
+    if (g.kind != kItemMarch) {
+        const dim3 gr((unsigned)(g.count < grid ? g.count : grid));
+        if (g.kind == kItemBack) {
+            hipLaunchKernelGGL((k_rk4_back<T>), gr, dim3(kBlock), 0, s, probs, it, g.count);
+            return hipGetLastError();
+        }
+        switch (g.K) {
+#define DOP_RP(KK)                                                                                \
+    case KK:                                                                                      \
+        hipLaunchKernelGGL((k_rk4_patch<T, ACC, KK>), gr, dim3(kBlock), (size_t)g.lds, s, probs, it, \
+                           g.count, parity);                                                      \
+        return hipGetLastError();
+            DOP_RP(3) DOP_RP(5) DOP_RP(7) DOP_RP(9) DOP_RP(11)
+#undef DOP_RP
+        }
+        return hipErrorInvalidValue;
+    }
+    const dim3 gr((unsigned)(g.count / 4 < grid ? g.count : 4 * grid));   // blocks of one wave
+    const bool uni = g.uniform != 0;
+    switch (g.K) {
+    case 3: return launch_march<T, ACC, 3>(uni, gr, probs, it, g.count, parity, s);
+    case 5: return launch_march<T, ACC, 5>(uni, gr, probs, it, g.count, parity, s);
+    case 7: return launch_march<T, ACC, 7>(uni, gr, probs, it, g.count, parity, s);
+    case 9: return launch_march<T, ACC, 9>(uni, gr, probs, it, g.count, parity, s);
+    case 11: return launch_march<T, ACC, 11>(uni, gr, probs, it, g.count, parity, s);
+    }
+    return hipErrorInvalidValue;
+}
+
+}  // namespace batch
+}  // namespace dop

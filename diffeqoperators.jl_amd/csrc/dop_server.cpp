@@ -109,6 +109,7 @@ struct Request {
     double release = 0, admitted = -1, completed = -1;
     size_t off = 0, bytes = 0;
     int cls = 0;
+    bool fused = false;   // its steps alternate the state between u and acc
     hipEvent_t done_ev = nullptr;
     State state = kScheduled;
 };
@@ -131,6 +132,7 @@ struct Class {
     TableSlot slots[kTableSlots];
     int cur_slot = -1;
     bool dirty = true;
+    int parity = 0;       // steps since the work list was built, mod 2
     std::deque<hipEvent_t> inflight;
     std::vector<hipEvent_t> step_events;
     size_t ev_i = 0;
@@ -232,7 +234,7 @@ int class_step(dop_server* srv, Class& C, size_t sb, std::vector<Request*>* drai
             Request& r = *C.active[k];
             dop::BProb& B = probs[k];
             B = dop::BProb{};
-            dop::batch_geometry(r.plan->d, srv->chunk, &B);
+            dop::batch_geometry(r.plan->d, srv->chunk, &B, true);
             const size_t n = round_up((size_t)r.plan->d.host.total * sb);
             B.u = srv->arena.ptr(r.off);
             B.s1 = srv->arena.ptr(r.off + n);
@@ -240,8 +242,12 @@ int class_step(dop_server* srv, Class& C, size_t sb, std::vector<Request*>* drai
             B.acc = srv->arena.ptr(r.off + 3 * n);
             B.scale = r.scale;
             B.dt = r.dt;
+            r.fused = B.fused != 0;
+            if (r.fused && (r.done_steps & 1)) std::swap(B.u, B.acc);
         }
-        dop::batch_items(probs, &items, &groups);
+        C.parity = 0;
+        dop::batch_march_chunks(&probs);
+        dop::batch_items(probs, true, &items, &groups);
         int rc = ensure_slot(S, probs.size(), items.size());
         if (rc != DOP_OK) return rc;
         std::copy(probs.begin(), probs.end(), S.h_probs);
@@ -258,17 +264,23 @@ int class_step(dop_server* srv, Class& C, size_t sb, std::vector<Request*>* drai
     TableSlot& S = C.slots[C.cur_slot];
     // one block per work item (no persistent blocks): blocks retire all the time, so the
     // classes' streams share the CUs instead of the largest class holding them for a whole step
+    if (dop::launch_batch_pass(srv->storage, S.d_probs, S.d_items, S.groups, false, C.parity,
+                               INT32_MAX / 4, C.st) != hipSuccess)
+        return dop::set_error(DOP_EHIP, "server: step launch failed");
     for (int stage = 0; stage < 4; ++stage)
         if (dop::launch_batch_items(srv->storage, S.d_probs, S.d_items, S.groups, stage, 0,
-                                    INT32_MAX, C.st) != hipSuccess)
+                                    INT32_MAX / 4, C.st) != hipSuccess)
             return dop::set_error(DOP_EHIP, "server: stage launch failed");
+    C.parity ^= 1;
     (void)hipEventRecord(S.used, C.st);
     S.armed = true;
     for (size_t k = 0; k < C.active.size();) {
         Request& r = *C.active[k];
         if (++r.done_steps >= r.nsteps) {
             const size_t n = (size_t)r.plan->d.host.total * sb;
-            if (hipMemcpyAsync(r.result, srv->arena.ptr(r.off), n, hipMemcpyDeviceToHost, C.st) !=
+            // a fused request's state after an odd number of steps lies in acc
+            const size_t at = r.fused && (r.done_steps & 1) ? 3 * round_up(n) : 0;
+            if (hipMemcpyAsync(r.result, srv->arena.ptr(r.off + at), n, hipMemcpyDeviceToHost, C.st) !=
                 hipSuccess)
                 return dop::set_error(DOP_EHIP, "server: result copy failed");
             (void)hipEventRecord(r.done_ev, C.st);

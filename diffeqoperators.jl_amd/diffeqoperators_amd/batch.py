@@ -82,7 +82,7 @@ class Batch:
 
 class RK4:
     """du_i/dt = scale_i * A_i u_i, classical RK4 with step dt_i, updating u_i in place;
-    the four stage launches of one step are a captured hipGraph (dop_rk4_*)."""
+    the launches of a step are captured hipGraphs (dop_rk4_*)."""
 
     def __init__(self, ops, us, scale, dt, stream=None):
         n = len(ops)

@@ -210,11 +210,13 @@ void dop_batch_destroy(dop_batch* batch);
 /* ---- explicit time stepping (no counterpart in the reference; its RHS is called from
  * OrdinaryDiffEq, heat_equation.jl:30-33) ----
  * A batch of method-of-lines problems du/dt = scale_i * (sum_t L_t Q u) advanced with
- * classical RK4, every stage of the whole batch one grouped launch set (as dop_batch_apply; the
- * groups of a stage run on forked streams inside the graph), the four stages of
- * a step captured once in a hipGraph and replayed.  Storage f32 or f64.  Creation tunes
- * the tile shape (DOP_RK4_AUTOTUNE=0 skips it) by timing stage-0 launches, which read u and
- * write only the internal stage buffers. */
+ * classical RK4.  1-D and 2-D problems whose rows the tiles take (windows up to 11 points) go
+ * through a whole step in one pass (u read once, the new state written once to a buffer that
+ * swaps roles with u; after dop_rk4_step the state is in u); the others stage by stage, every
+ * stage one grouped launch set (as dop_batch_apply).  The launches of a step run on forked
+ * streams inside hipGraphs captured once and replayed.  Storage f32 or f64.  Creation tunes the
+ * tile shape of problems that go stage by stage (DOP_RK4_AUTOTUNE=0 skips it) by timing stage-0
+ * launches, which read u and write only the internal stage buffers. */
 typedef struct dop_rk4 dop_rk4;
 int dop_rk4_create(int n, const dop_plan* const* plans, const double* scale,
                    const double* dt, void* const* u, void* stream, dop_rk4** out);
@@ -231,7 +233,7 @@ void dop_rk4_destroy(dop_rk4* rk);
  * down to 256 bytes) fits and fewer than `max_active` are resident, and advances the resident
  * requests by RK4 steps: they are split into size classes by grid points (up to 256^2, up to
  * 1024^2, larger), each class on a stream of its own advancing all its requests one step per
- * iteration (each stage one grouped launch set over the class), the classes side by side on
+ * iteration (the passes and stage launches of dop_rk4 over the class), the classes side by side on
  * the GPU, so a small request is not held to the pace of the largest resident grid.  A
  * finished state is copied back asynchronously.  Storage f32 or f64 (one type per server).
  * dop_server_submit may be called from any thread, also while dop_server_run runs: such a

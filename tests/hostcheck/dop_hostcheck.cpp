@@ -2,8 +2,10 @@
 // plan builder (dop_build.cpp, dop_rows.cpp) and the same per-point arithmetic
 // (dop_eval.hpp) that the gfx950 kernels run, so that the index math of the device path
 // can be compared with the FP64 oracle without a GPU.  Never part of libdop.so.
+#include <algorithm>
 #include <cstdint>
 #include <string>
+#include <vector>
 
 #include "../../diffeqoperators.jl_amd/csrc/dop_build.hpp"
 #include "../../diffeqoperators.jl_amd/csrc/dop_concrete.hpp"
@@ -286,3 +288,101 @@ int hc_csr(const dop_desc* d, int64_t* row_ptr, int64_t* col, double* val, doubl
     return DOP_OK;
 }
 }
+
+// ---------------------------------------------------------------------------------------
+// The one-pass RK4 work list of a plan: every point must be an own point of exactly one patch or
+// marching segment, and every value a patch's points read (windows, boundary rows, ghosts, stage
+// by stage) must lie in the region the patch holds of the stage before.
+#include "../../diffeqoperators.jl_amd/csrc/dop_batch.hpp"
+
+namespace {
+// the line elements that row r of axis X reads through its program: calls f(j)
+template <typename F>
+void row_reads(const dop::AxisDev& X, const dop::AxisTables& T, int r, const F& f)
+{
+    if (r >= X.rlo && r < X.rhi) {
+        for (int k = 0; k < X.K; ++k) f(r + X.dmin + k);
+        return;
+    }
+    const bool left = r < X.rlo;
+    const int b = left ? r : X.rlo + (r - X.rhi);
+    for (int k = 0; k < (left ? X.nl : X.nr); ++k) f(left ? k : X.n - X.nr + k);
+    for (int k = 0; k < T.bn[b]; ++k) f(std::min(std::max(T.bJ0[b] + k - 1, 0), X.n - 1));
+}
+}  // namespace
+
+extern "C" {
+// fused (0, 1, 2), or -1 on a build error; *bad: 0 when the list is right, otherwise which rule
+// fails first (1 cover, 2 reads of a patch, 3 LDS, 4 a segment's cone), info: where.
+int hc_rk4_items(const dop_desc* d, int* bad, int64_t* info)
+{
+    *bad = 0;
+    dop::HostPlan H;
+    if (dop::build_host_plan(*d, &H, &g_err) != DOP_OK) return -1;
+    dop::DevicePlan D;
+    D.host = H.meta;
+    dop::build_fast(H, &D.fast);
+    std::vector<dop::BProb> probs(1);
+    dop::batch_geometry(D, 16, &probs[0], true);
+    dop::batch_march_chunks(&probs);
+    std::vector<dop::BItem> items;
+    std::vector<dop::BGroup> groups;
+    dop::batch_items(probs, true, &items, &groups);
+    const dop::BProb& B = probs[0];
+    if (!B.fused) return 0;
+    const dop::PlanDev& P = H.meta;
+    const int n0 = (int)P.n[0], n1 = (int)P.n[1];
+    std::vector<unsigned char> cover((size_t)n0 * n1, 0);
+    auto fail = [&](int what, int64_t a, int64_t b, int64_t c, int64_t e) {
+        *bad = what;
+        info[0] = a; info[1] = b; info[2] = c; info[3] = e;
+        return (int)B.fused;
+    };
+    const int HW = B.K / 2, VX = dop::march_vx(P.storage, P.accum, B.K);
+    const int pad = (4 * HW + VX - 1) / VX * VX, out = 64 * VX - 2 * pad;
+    for (const dop::BItem& I : items) {
+        if (I.kind == dop::kItemMarch) {
+            const int xb = B.flo[0] + I.a * out, xe = std::min(xb + out, B.fhi[0]);
+            const int y0 = B.flo[1] + I.b * B.fchunk, y1 = std::min(y0 + B.fchunk, B.fhi[1]);
+            // whole groups in the array; the cone (4H) in the array, its centres (3H) regular
+            if (xb - pad < 0 || (xe - xb) % VX || xe + pad > n0 || y0 - 4 * HW < 0 || y1 + 4 * HW > n1 ||
+                xb - 3 * HW < B.lo[0] || xe + 3 * HW > B.hi[0] || y0 - 3 * HW < B.lo[1] ||
+                y1 + 3 * HW > B.hi[1] || xe <= xb || y1 <= y0)
+                return fail(4, xb, xe, y0, y1);
+            for (int y = y0; y < y1; ++y)
+                for (int x = xb; x < xe; ++x) ++cover[(size_t)y * n0 + x];
+        } else if (I.kind == dop::kItemPatch) {
+            int lo[2][5], hi[2][5];   // [1 + s]: stage s's points; [0]: loaded
+            lo[0][4] = I.a; hi[0][4] = I.b; lo[1][4] = I.c; hi[1][4] = I.d;
+            for (int a = 0; a < 2; ++a)
+                for (int s = 3; s >= 0; --s) {
+                    lo[a][s] = lo[a][s + 1];
+                    hi[a][s] = hi[a][s + 1];
+                    if (a < P.ndim) dop::rows_reach(P.ax[a], B.K / 2, &lo[a][s], &hi[a][s]);
+                }
+            const int64_t loaded = ((int64_t)(hi[0][0] - lo[0][0]) | 1) * (hi[1][0] - lo[1][0]);
+            const int64_t own = (int64_t)(I.b - I.a) * (I.d - I.c);
+            if ((3 * loaded + own) * (P.storage == dop::kF64 ? 8 : 4) > dop::kPatchLds ||
+                loaded >= (1 << 14))
+                return fail(3, I.a, I.b, I.c, I.d);
+            for (int a = 0; a < P.ndim; ++a)
+                for (int s = 4; s >= 1; --s) {
+                    if (lo[a][s - 1] < 0 || hi[a][s - 1] > P.n[a]) return fail(2, a, s, I.a, I.c);
+                    for (int r = lo[a][s]; r < hi[a][s]; ++r) {
+                        bool ok = true;
+                        auto in = [&](int j) { ok = ok && j >= lo[a][s - 1] && j < hi[a][s - 1]; };
+                        row_reads(P.ax[a], H.axis[a], r, in);
+                        if (r >= B.lo[a] && r < B.hi[a])
+                            for (int k = -HW; k <= HW; ++k) in(r + k);
+                        if (!ok) return fail(2, a, s, r, a ? I.c : I.a);
+                    }
+                }
+            for (int y = I.c; y < I.d; ++y)
+                for (int x = I.a; x < I.b; ++x) ++cover[(size_t)y * n0 + x];
+        }
+    }
+    for (int64_t p = 0; p < (int64_t)cover.size(); ++p)
+        if (cover[p] != 1) return fail(1, p % n0, p / n0, cover[p], 0);
+    return B.fused;
+}
+}  // extern "C"
