@@ -62,7 +62,7 @@ constexpr int march_vx(int storage, int accum, int K)
 }
 constexpr int kBackPts = 16384;    // points per item of the copy back
 constexpr int kRimPts = 256;       // shell points per item where shell_point takes them
-constexpr int kPatchLds = 64 << 10;   // bytes of LDS a patch may use, its head included
+constexpr int kPatchLds = 80 << 10;   // bytes of LDS a patch may use, its head included (two a CU)
 constexpr int kPatchHead = 64;         // bytes before a patch's arrays (the stages' regions)
 
 // A run of items that one launch takes.  An apply's items: one kind, window width K (points:

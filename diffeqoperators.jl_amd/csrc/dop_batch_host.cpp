@@ -40,7 +40,7 @@ bool march_box(const PlanDev& P, const FastArgs& A, BProb* B)
 // reach, the stage sums over its points
 int64_t patch_bytes(const PlanDev& P, int H, int x0, int x1, int y0, int y1)
 {
-    const int64_t own = (int64_t)(x1 - x0) * (y1 - y0);
+    const int64_t own = (int64_t)((x1 - x0) | 1) * (y1 - y0);
     for (int s = 0; s < 4; ++s) {
         rows_reach(P.ax[0], H, &x0, &x1);
         if (P.ndim == 2) rows_reach(P.ax[1], H, &y0, &y1);
@@ -49,20 +49,26 @@ int64_t patch_bytes(const PlanDev& P, int H, int x0, int x1, int y0, int y1)
 }
 
 // Patch extents (w, h) for a rectangle of points of the grid: lines of up to 128 loaded points
-// (two waves of lanes) by what the LDS then holds, at most 16 or 32 rows of own points beyond the
-// recomputed ones; thin rectangles keep their width.  False when even small patches do not fit.
-bool patch_size(const PlanDev& P, int H, int rw, int rh, int* w, int* h)
+// (two waves of lanes) by all of a rim's rows if the LDS holds them, else by what it holds; thin
+// rectangles keep their width.  False when even small patches do not fit.
+bool patch_size(const PlanDev& P, int H, int x0, int x1, int y0, int y1, int* w, int* h)
 {
-    // how far the patch's points reach, over four stages, at its widest: windows on both sides
-    // and, on one side, boundary rows (whose windows may be one longer than the reach in)
-    int ext[2] = {0, 0};
+    // what the patch's points reach beyond them over four stages: along an axis that is not split,
+    // what the rectangle reaches; else at its widest (windows on both sides and, on one side,
+    // boundary rows, whose windows may be one longer than the reach in)
+    const int lo[2] = {x0, y0}, hi[2] = {x1, y1};
+    int ext[2] = {0, 0}, all[2] = {0, 0};
     for (int a = 0; a < P.ndim; ++a) {
-        const AxisDev& X = P.ax[a];
-        ext[a] = 8 * H + X.KB;
+        int l = lo[a], r = hi[a];
+        for (int s = 0; s < 4; ++s) rows_reach(P.ax[a], H, &l, &r);
+        all[a] = (r - l) - (hi[a] - lo[a]);
+        ext[a] = 8 * H + P.ax[a].KB;
     }
+    const int rw = x1 - x0, rh = y1 - y0;
     const int64_t sb = P.storage == kF64 ? 8 : 4;
     auto fits = [&](int ww, int hh) {
-        return kPatchHead + (3 * (int64_t)((ww + ext[0]) | 1) * (hh + ext[1]) + (int64_t)ww * hh) * sb <=
+        const int64_t ew = ww == rw ? all[0] : ext[0], eh = hh == rh ? all[1] : ext[1];
+        return kPatchHead + (3 * ((ww + ew) | 1) * (hh + eh) + (int64_t)(ww | 1) * hh) * sb <=
                kPatchLds;
     };
     if (P.ndim == 1) {
@@ -72,12 +78,12 @@ bool patch_size(const PlanDev& P, int H, int rw, int rh, int* w, int* h)
     }
     if (rw <= 64 && rw < rh) {   // a strip along y
         *w = rw;
-        for (*h = std::min(rh, 128 - std::min(ext[1], 96)); *h >= 8; *h -= 4)
+        for (*h = std::min(rh, 128 - std::min(8 * H, 96)); *h >= 8; *h -= 4)
             if (fits(*w, *h)) return true;
         return false;
     }
     for (*h = std::min(rh, 32); *h >= 4; *h = *h > 8 ? (*h + 1) / 2 : *h - 2) {
-        for (*w = std::min(rw, 128 - std::min(ext[0], 96)); *w >= 16 || *w == rw; *w -= 4)
+        for (*w = std::min(rw, 128 - std::min(8 * H, 96)); *w >= 16 || *w == rw; *w -= 4)
             if (fits(*w, *h)) return true;
     }
     return false;
@@ -87,7 +93,7 @@ template <typename F>
 void patches(const PlanDev& P, int H, int x0, int x1, int y0, int y1, const F& f)
 {
     int w, h;
-    if (x1 <= x0 || y1 <= y0 || !patch_size(P, H, x1 - x0, y1 - y0, &w, &h)) return;
+    if (x1 <= x0 || y1 <= y0 || !patch_size(P, H, x0, x1, y0, y1, &w, &h)) return;
     // even pieces
     const int nx = (int)ceil_div(x1 - x0, w), ny = (int)ceil_div(y1 - y0, h);
     for (int j = 0; j < ny; ++j)
@@ -150,7 +156,7 @@ void batch_geometry(const DevicePlan& p, int chunk, BProb* B, bool rk4)
             patch_rects(*B, (int)P.n[0], (int)P.n[1], [&](int x0, int x1, int y0, int y1) {
                 int w, h;
                 if (x1 <= x0 || y1 <= y0) return;
-                fits = fits && patch_size(P, B->K / 2, x1 - x0, y1 - y0, &w, &h);
+                fits = fits && patch_size(P, B->K / 2, x0, x1, y0, y1, &w, &h);
                 if (fits) patches(P, B->K / 2, x0, x1, y0, y1, [&](int xa, int xb, int ya, int yb) {
                     fits = fits && patch_bytes(P, B->K / 2, xa, xb, ya, yb) <= kPatchLds;
                 });

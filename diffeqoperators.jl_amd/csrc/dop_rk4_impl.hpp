@@ -18,13 +18,18 @@
 //
 // k_rk4_patch, the rim of the box (or all of a small or 1-D grid): a block loads a patch with all
 // that its points' cones reach (rows_reach: windows, boundary rows, ghosts) into LDS and runs the
-// four stages there, each over the region the next one reads.
+// four stages there, each over the region the next one reads.  Bound by instruction issue and the
+// latency of a block's chain of rows.  A line's weights and boundary data stay in registers over
+// the rows: with shell_point_f at every point near an edge the mixed problems below took 1.71 ms a
+// step and the served ones 25.1 ms, against 1.52 and 20.9.  Patches of all a rim's rows, for which
+// the LDS holds 80 KB (two blocks a CU), halve the recomputed points at K = 9 and 11: 1.30 ms.
+// Tried: 512 threads and four rows side by side, 1.75 ms (the scalar registers spill).
 //
 // Every stage value is rounded to the storage type exactly where the stage-wise kernels store it,
 // and every sum runs in their order, so the new state is the same bit for bit.  The new state goes
 // to acc, so u and acc swap roles from step to step.
 // Measured against the stage-wise step: 256 mixed f32 problems (1-D to 65536, 2-D to 2048 squared,
-// orders 2 to 8) 2.08 -> 1.71 ms a step, 24 served 2-D requests of 100 steps 36.7 -> 25.1 ms.
+// orders 2 to 8) 2.08 -> 1.30 ms a step, 24 served 2-D requests of 100 steps 36.7 -> 20.6 ms.
 #pragma once
 #include "dop_batch_impl.hpp"
 
@@ -243,7 +248,7 @@ __global__ __launch_bounds__(64, 2) void k_rk4_march(const BProb* __restrict__ p
 struct Patch {
     int o0, o1;          // grid coordinates of the first loaded point
     int pitch, sz;       // row pitch (odd: lanes along y hit different banks), points loaded
-    int a0, a1, ow;      // first own point, own points per row
+    int a0, a1, ow;      // first own point, pitch of the sums
 };
 
 extern __shared__ __attribute__((aligned(16))) char patch_lds[];
@@ -258,93 +263,227 @@ __device__ inline T& patch_at(int i)
     return reinterpret_cast<T*>(patch_lds + kPatchHead)[i];
 }
 
-// Stage s of a point: its row's sum v to the stage sum and the next stage's input (own: one of the
-// patch's own points, p its offset in the loaded area, q among the own points)
+// Stage s of a point: k = scale * its row's sum to the stage sum and the next stage's input (own: one
+// of the patch's own points; p its offset in the loaded area, q among the own points).  c is dt / 6
+// for the first and last stage, else dt / 3; h dt for the third stage, else dt / 2.
 template <typename T>
-__device__ inline void patch_update(const Patch& Q, int s, double k, double dt, int p, int q, bool own,
-                                    T* o)
+__device__ inline void patch_update(const Patch& Q, int s, double k, double c, double h, int p, int q,
+                                    bool own, T* o)
 {
     if (s == 3) {
-        *o = (T)((double)patch_at<T>(3 * Q.sz + q) + (dt / 6.0) * k);
+        *o = (T)((double)patch_at<T>(3 * Q.sz + q) + c * k);
         return;
     }
     const double up = (double)patch_at<T>(p);
     if (own) {
         T& sum = patch_at<T>(3 * Q.sz + q);
-        sum = s == 0 ? (T)(up + (dt / 6.0) * k) : (T)((double)sum + (dt / 3.0) * k);
+        sum = (T)((s == 0 ? up : (double)sum) + c * k);
     }
-    const double h = (s == 2) ? dt : 0.5 * dt;
     patch_at<T>((s == 1 ? 2 : 1) * Q.sz + p) = (T)(up + h * k);
 }
 
+template <int ACC>
+__device__ inline auto btabs(const BProb& B)
+{
+    if constexpr (std::is_same<typename Acc<ACC>::W, double>::value) return &B.w64[0];
+    else return &B.w32[0];
+}
+template <typename W>
+__device__ inline const W* const& axis_table(const AxisDev& X)
+{
+    if constexpr (std::is_same<W, double>::value) return X.w64;
+    else return X.w32;
+}
+
+// A field of a plan or problem (they do not change while a launch reads them), in scalar registers
+template <typename X>
+__device__ inline X patch_field(const X& f)
+{
+    return const_tab(&f, 0);
+}
+
+constexpr int kPatchBlock = 256;   // threads of a patch's block
+
 // Stage s of a patch over the block: lanes along axis L (0: x), rows along the other one.  A wave
-// takes 64 lines along L and a part of the rows; the weights along L stay in its registers, a
-// row's are the same for the wave.  Points whose rows are regular on both axes (in the tiles'
-// natural box) read their windows from LDS; the others go through shell_point_f.
+// takes 64 lines along L and a part of the rows.  What a line's row along L needs stays in its
+// registers over the rows: the weights of a regular row (in the tiles' natural box), or a boundary
+// row's (and the few regular rows' that lie outside the box) with its ghost's coefficients; a row's
+// along the other axis are the same for the wave, in scalar registers.  Sums run as in
+// shell_point_f outside the box (a tap that the tiles' window adds to the row's with weight 0 is
+// taken as 0 there) and as in the tiles inside.
 template <typename T, int ACC, int K, int L>
 __device__ inline void patch_stage(const BProb& B, const PlanDev& P, const Patch& Q, int s,
                                    T* __restrict__ out)
 {
     using W = typename Acc<ACC>::W;
-    constexpr int H = K / 2, M = 1 - L;
+    constexpr int H = K / 2, M = 1 - L, KT = K + 1;
     const int l0 = patch_region(s, 2 * L), l1 = patch_region(s, 2 * L + 1);
     const int m0 = patch_region(s, 2 * M), m1 = patch_region(s, 2 * M + 1);
     const int ol = L == 0 ? Q.o0 : Q.o1, om = L == 0 ? Q.o1 : Q.o0;
     const int b0 = patch_region(3, 1), b1 = patch_region(3, 3);   // the own points' end
     const int in = (s == 0 ? 0 : s == 2 ? 2 : 1) * Q.sz;
-    const double scale = B.scale, dt = B.dt;
+    const double scale = patch_field(B.scale), dt = patch_field(B.dt);
+    const double c = dt / (s == 0 || s == 3 ? 6.0 : 3.0), h = s == 2 ? dt : 0.5 * dt;
+    const int64_t ys = patch_field(B.ys);
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int nl = (l1 - ol + 63) >> 6;             // groups of lines (from the patch's origin)
-    const int parts = nl == 1 ? 4 : nl <= 3 ? 2 : 1;
+    const int parts = max(kPatchBlock / 64 / nl, 1);
     const int per = (m1 - m0 + parts - 1) / parts;
-    const bool uL = B.uniform[L] != 0, uM = B.uniform[M] != 0;
-    const W* wlt = btab<ACC>(B, L);
-    const W* wmt = btab<ACC>(B, M);
+    const bool uL = patch_field(B.uniform[L]) != 0, uM = patch_field(B.uniform[M]) != 0;
+    const int bl0 = patch_field(B.lo[L]), bl1 = patch_field(B.hi[L]);
+    const int bm0 = patch_field(B.lo[M]), bm1 = patch_field(B.hi[M]);
+    const W* wlt = patch_field(btabs<ACC>(B)[L]);
+    const W* wmt = patch_field(btabs<ACC>(B)[M]);
+    const AxisDev &XL = P.ax[L], &XM = P.ax[M];
+    const int nL = patch_field(XL.n), nM = patch_field(XM.n);
+    // the row's own taps in the window of K
+    const int kl0 = H + patch_field(XL.dmin), kl1 = kl0 + patch_field(XL.K);
+    const int km0 = H + patch_field(XM.dmin), km1 = km0 + patch_field(XM.K);
+    const bool padl = kl0 > 0 || kl1 < K, padm = km0 > 0 || km1 < K;
     const int sl = L == 0 ? 1 : Q.pitch, sm = L == 0 ? Q.pitch : 1;   // LDS strides
-    for (int unit = wave; unit < nl * parts; unit += 4) {
+    for (int unit = wave; unit < nl * parts; unit += kPatchBlock / 64) {
         const int g = unit % nl, part = unit / nl;
         const int l = ol + g * 64 + lane;
         const bool lin = l >= l0 && l < l1;
         if (__builtin_amdgcn_ballot_w64(lin) == 0) continue;
-        const bool lreg = l >= B.lo[L] && l < B.hi[L];
-        W wl[K];
+        const bool lreg = l >= bl0 && l < bl1;
+        W wl[K], wm[K];
 #pragma unroll
-        for (int k = 0; k < K; ++k)
+        for (int k = 0; k < K; ++k) {
             wl[k] = lin && lreg ? wlt[(uL ? 0 : (int64_t)l * K) + k] : W(0);
+            wm[k] = uM ? const_tab(wmt, k) : W(0);
+        }
+        // rows outside the box: weights, first tap, taps, ghost taps
+        double wb[KT] = {}, ga[kPointGhost] = {}, gc = 0.0;
+        int jb = 0, nb = 0, ng = 0, go = 0;
+        bool bnd = false;
+        if (lin && !lreg) {
+            if (l >= XL.rlo && l < XL.rhi) {
+                const W* wt = Acc<ACC>::table(XL) + (XL.uniform ? 0 : l);
+                const int64_t ws = XL.uniform ? 1 : nL;
+                jb = l + XL.dmin;
+                nb = XL.K;
+#pragma unroll
+                for (int k = 0; k < K; ++k)
+                    if (k < nb) wb[k] = (double)tab(wt, k * ws);
+            } else {
+                const bool left = l < XL.rlo;
+                const int b = left ? l : XL.rlo + (l - XL.rhi);
+                const double* wr = XL.bw + (int64_t)b * XL.KB;
+                const double* al = left ? XL.al : XL.ar;
+                bnd = true;
+                jb = tab(XL.bJ0, b) - 1;
+                nb = tab(XL.bn, b);
+                ng = left ? XL.nl : XL.nr;
+                go = left ? 0 : nL - XL.nr;
+                gc = left ? tab(&XL.bl, 0) : tab(&XL.br, 0);
+#pragma unroll
+                for (int k = 0; k < KT; ++k)
+                    if (k < nb) wb[k] = tab(wr, k);
+#pragma unroll
+                for (int k = 0; k < kPointGhost; ++k)
+                    if (k < ng) ga[k] = tab(al, k);
+            }
+        }
         const int mb = m0 + part * per, me = min(mb + per, m1);
         for (int m = mb; m < me; ++m) {
             if (!lin) continue;
-            const bool mreg = m >= B.lo[M] && m < B.hi[M];   // wave-uniform
-            const int p = (l - ol) * sl + (m - om) * sm;
-            const int x = L == 0 ? l : m, y = L == 0 ? m : l;
-            double v;
-            if (lreg && mreg) {
-                T tl[K], tm[K];
-                W wm[K];
+            const bool mreg = m >= bm0 && m < bm1;   // wave-uniform
+            const int pl = in + (m - om) * sm, pm = in + (l - ol) * sl;   // the point's two lines
+            auto atl = [&](int j) { return patch_at<T>(pl + (j - ol) * sl); };
+            auto atm = [&](int j) { return patch_at<T>(pm + (j - om) * sm); };
+            Acc<ACC> a;
+            auto along_l = [&]() {
+                if (lreg) {
+                    T t[K];
 #pragma unroll
-                for (int k = 0; k < K; ++k) {
-                    tl[k] = patch_at<T>(in + (p + (k - H) * sl));
-                    tm[k] = patch_at<T>(in + (p + (k - H) * sm));
-                    wm[k] = const_tab(wmt, (uM ? 0 : (int64_t)m * K) + k);
+                    for (int k = 0; k < K; ++k) t[k] = atl(l - H + k);
+                    if (padl && !mreg) {
+#pragma unroll
+                        for (int k = 0; k < K; ++k)
+                            if (k < kl0 || k >= kl1) t[k] = T(0);
+                    }
+#pragma unroll
+                    for (int k = 0; k < K; ++k) a.add(wl[k], (W)t[k]);
+                } else if (bnd) {
+                    double gv = 0.0;
+#pragma unroll
+                    for (int k = 0; k < kPointGhost; ++k)
+                        if (k < ng) gv = fma(ga[k], (double)atl(go + k), gv);
+                    gv = gv + gc;
+                    double sum = 0.0;
+#pragma unroll
+                    for (int k = 0; k < KT; ++k) {
+                        if (k < nb) {
+                            const int j = jb + k;
+                            const double t = (double)atl(min(max(j, 0), nL - 1));
+                            sum = fma(wb[k], j < 0 || j >= nL ? gv : t, sum);
+                        }
+                    }
+                    a.add_sum(sum);
+                } else {
+#pragma unroll
+                    for (int k = 0; k < K; ++k)
+                        if (k < nb) a.add((W)wb[k], (W)atl(jb + k));
                 }
-                Acc<ACC> a;
+            };
+            auto along_m = [&]() {
+                const int rlo = patch_field(XM.rlo), rhi = patch_field(XM.rhi);
+                if (mreg) {
+                    T t[K];
 #pragma unroll
-                for (int k = 0; k < K; ++k) a.add(L == 0 ? wl[k] : wm[k], (W)(L == 0 ? tl[k] : tm[k]));
+                    for (int k = 0; k < K; ++k) {
+                        t[k] = atm(m - H + k);
+                        if (!uM) wm[k] = const_tab(wmt, (int64_t)m * K + k);
+                    }
+                    if (padm && !lreg) {
 #pragma unroll
-                for (int k = 0; k < K; ++k) a.add(L == 0 ? wm[k] : wl[k], (W)(L == 0 ? tm[k] : tl[k]));
-                v = a.value();
-            } else {
-                const int64_t idx[3] = {x, y, 0};
-                const int px = x - Q.o0, py = y - Q.o1;
-                v = shell_point_f<T, ACC, K, 2>(P, idx, [&](int a, int j) -> T {
-                    return a == 0 ? patch_at<T>(in + (py * Q.pitch + (j - Q.o0)))
-                                  : patch_at<T>(in + ((j - Q.o1) * Q.pitch + px));
-                });
-            }
+                        for (int k = 0; k < K; ++k)
+                            if (k < km0 || k >= km1) t[k] = T(0);
+                    }
+#pragma unroll
+                    for (int k = 0; k < K; ++k) a.add(wm[k], (W)t[k]);
+                } else if (m >= rlo && m < rhi) {
+                    const W* wt = patch_field(axis_table<W>(XM)) + (uM ? 0 : m);
+                    const int64_t ws = uM ? 1 : nM;
+#pragma unroll
+                    for (int k = 0; k < K; ++k)
+                        if (k < km1 - km0) a.add(const_tab(wt, k * ws), (W)atm(m + (km0 - H) + k));
+                } else {
+                    const bool left = m < rlo;
+                    const int b = left ? m : rlo + (m - rhi);
+                    const double* wr = patch_field(XM.bw) + (int64_t)b * patch_field(XM.KB);
+                    const int jm = const_tab(patch_field(XM.bJ0), b) - 1;
+                    const int nt = const_tab(patch_field(XM.bn), b);
+                    const int nr = patch_field(XM.nr);
+                    const int n = left ? patch_field(XM.nl) : nr;
+                    const int o = left ? 0 : nM - nr;
+                    double gv = 0.0;
+#pragma unroll
+                    for (int k = 0; k < kPointGhost; ++k)
+                        if (k < n)
+                            gv = fma(left ? patch_field(XM.al[k]) : patch_field(XM.ar[k]),
+                                     (double)atm(o + k), gv);
+                    gv = gv + (left ? patch_field(XM.bl) : patch_field(XM.br));
+                    double sum = 0.0;
+#pragma unroll
+                    for (int k = 0; k < KT; ++k) {
+                        if (k < nt) {
+                            const int j = jm + k;
+                            const double t = (double)atm(min(max(j, 0), nM - 1));
+                            sum = fma(const_tab(wr, k), j < 0 || j >= nM ? gv : t, sum);
+                        }
+                    }
+                    a.add_sum(sum);
+                }
+            };
+            if (L == 0) along_l(); else along_m();
+            if (L == 0) along_m(); else along_l();
+            const int x = L == 0 ? l : m, y = L == 0 ? m : l;
             const bool own = x >= Q.a0 && x < b0 && y >= Q.a1 && y < b1;
-            patch_update<T>(Q, s, scale * v, dt, p, (y - Q.a1) * Q.ow + (x - Q.a0), own,
-                            out + ((int64_t)y * B.ys + x));
+            patch_update<T>(Q, s, scale * a.value(), c, h, (l - ol) * sl + (m - om) * sm,
+                            (y - Q.a1) * Q.ow + (x - Q.a0), own, out + ((int64_t)y * ys + x));
         }
     }
 }
@@ -359,9 +498,10 @@ __device__ inline void patch_stage1(const BProb& B, const PlanDev& P, const Patc
     const int x0 = patch_region(s, 0), x1 = patch_region(s, 1), b0 = patch_region(3, 1);
     const int in = (s == 0 ? 0 : s == 2 ? 2 : 1) * Q.sz;
     const double scale = B.scale, dt = B.dt;
+    const double c = dt / (s == 0 || s == 3 ? 6.0 : 3.0), h = s == 2 ? dt : 0.5 * dt;
     const W* wt = btab<ACC>(B, 0);
     const bool uni = B.uniform[0] != 0;
-    for (int x = x0 + (int)threadIdx.x; x < x1; x += kBlock) {
+    for (int x = x0 + (int)threadIdx.x; x < x1; x += kPatchBlock) {
         const int p = x - Q.o0;
         double v;
         if (x >= B.lo[0] && x < B.hi[0]) {
@@ -375,13 +515,13 @@ __device__ inline void patch_stage1(const BProb& B, const PlanDev& P, const Patc
             v = shell_point_f<T, ACC, K, 1>(
                 P, idx, [&](int, int j) -> T { return patch_at<T>(in + (j - Q.o0)); });
         }
-        patch_update<T>(Q, s, scale * v, dt, p, x - Q.a0, x >= Q.a0 && x < b0, out + x);
+        patch_update<T>(Q, s, scale * v, c, h, p, x - Q.a0, x >= Q.a0 && x < b0, out + x);
     }
 }
 
 // The points [a, b) x [c, d) of a problem.
 template <typename T, int ACC, int K>
-__global__ __launch_bounds__(kBlock) void k_rk4_patch(const BProb* __restrict__ probs,
+__global__ __launch_bounds__(kPatchBlock) void k_rk4_patch(const BProb* __restrict__ probs,
                                                     const BItem* __restrict__ items, int nitems,
                                                     int parity)
 {
@@ -412,15 +552,25 @@ __global__ __launch_bounds__(kBlock) void k_rk4_patch(const BProb* __restrict__ 
         Q.sz = Q.pitch * lh;
         Q.a0 = I.a;
         Q.a1 = I.c;
-        Q.ow = I.b - I.a;
+        Q.ow = (I.b - I.a) | 1;
         // load: rows in turn (32-bit reciprocal of the width, exact for the fewer than 2^14 points
         // of a patch)
         const uint32_t w = (uint32_t)(x1 - x0), n = w * (uint32_t)lh;
         const uint32_t mul = w > 1 ? (uint32_t)((0x100000000ull + w - 1) / w) : 0;
-        const T* s0 = src + (int64_t)y0 * B.ys + x0;
-        for (uint32_t p = threadIdx.x; p < n; p += kBlock) {
-            const uint32_t q = w > 1 ? __umulhi(p, mul) : p;
-            patch_at<T>((int)(q * Q.pitch + (p - q * w))) = s0[(int64_t)q * B.ys + (p - q * w)];
+        const int64_t ys = patch_field(B.ys);
+        const T* s0 = src + (int64_t)y0 * ys + x0;
+        for (uint32_t p = threadIdx.x; p < n; p += kPatchBlock * 8) {   // eight loads in flight
+            T v[8];
+            int at[8];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const uint32_t pi = min(p + i * kPatchBlock, n - 1);
+                const uint32_t q = w > 1 ? __umulhi(pi, mul) : pi, c = pi - q * w;
+                at[i] = (int)(q * Q.pitch + c);
+                v[i] = s0[(int64_t)q * ys + c];
+            }
+#pragma unroll
+            for (int i = 0; i < 8; ++i) patch_at<T>(at[i]) = v[i];   // (clamped ones: the same value)
         }
         __syncthreads();
 #pragma unroll 1
@@ -482,7 +632,7 @@ hipError_t launch_pass_group(const BGroup& g, const BProb* probs, const BItem* i
         switch (g.K) {
 #define DOP_RP(KK)                                                                                \
     case KK:                                                                                      \
-        hipLaunchKernelGGL((k_rk4_patch<T, ACC, KK>), gr, dim3(kBlock), (size_t)g.lds, s, probs, it, \
+        hipLaunchKernelGGL((k_rk4_patch<T, ACC, KK>), gr, dim3(kPatchBlock), (size_t)g.lds, s, probs, it, \
                            g.count, parity);                                                      \
         return hipGetLastError();
             DOP_RP(3) DOP_RP(5) DOP_RP(7) DOP_RP(9) DOP_RP(11)

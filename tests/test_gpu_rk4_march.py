@@ -86,3 +86,39 @@ def test_served_odd_and_even_steps_equal_stagewise(dtype):
 
     for x, y in zip(serve(), stagewise(serve)):
         assert torch.equal(x, y)
+
+
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+def test_patches_of_mixed_windows_equal_stagewise(dtype):
+    # windows of different widths per axis (regular rows outside the tiles' box, taps the wider
+    # window adds with weight 0), 1-D grids of one and several patches, far patch origins
+    shapes = [((140, 151), (2, 6)), ((180, 97), (6, 2)), ((230, 333), (4, 2)), ((64, 70), (2, 4)),
+              ((66,), (2,)), ((1025,), (6,)), ((65536,), (4,)), ((40000,), (8,))]
+
+    def make(us):
+        ops = []
+        for shape, orders in shapes:
+            js = tuple(reversed(shape))
+            A = None
+            for N, (n, a) in enumerate(zip(js, orders), 1):
+                L = D.CenteredDifference[N](2, a, 1.0 / (n + 1), n)
+                A = L if A is None else A + L
+            dx = tuple(1.0 / (n + 1) for n in js)
+            robin = ((1.0, 0.5, 0.1), (1.0, 0.5, -0.2))
+            if len(js) == 1:
+                ops.append(A * D.RobinBC(*robin, dx[0], 1))
+            else:
+                ops.append(A * D.compose(*D.RobinBC(*robin, dx, 1, js)))
+        return D.RK4(ops, us, [1.0] * len(us), [0.02 / max(s) ** 2 for s, _ in shapes])
+
+    fields = [torch.from_numpy(np.random.default_rng(i).uniform(-1, 1, s)).to("cuda").to(dtype)
+              for i, (s, _) in enumerate(shapes)]
+    a, b = [f.clone() for f in fields], [f.clone() for f in fields]
+    ra, rb = make(a), stagewise(lambda: make(b))
+    for n in (1, 2):
+        ra.step(n)
+        rb.step(n)
+        torch.cuda.synchronize()
+        for c, x, y in zip(shapes, a, b):
+            assert torch.isfinite(y).all()
+            assert torch.equal(x, y), (c, n, (x - y).abs().max().item())
