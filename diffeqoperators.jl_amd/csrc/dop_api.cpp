@@ -291,6 +291,32 @@ int dop_apply(const dop_plan* plan, void* du, const void* u, int accumulate, voi
     return DOP_OK;
 }
 
+int dop_apply_set(int n, const dop_plan* const* plans, void* const* du, const void* const* u,
+                  const int* accumulate, void* stream)
+{
+    if (n < 1 || !plans || !du || !u || !accumulate) return fail(DOP_EINVAL, "bad apply set");
+    for (int i = 0; i < n; ++i) {
+        if (!plans[i] || !du[i] || !u[i]) return fail(DOP_EINVAL, "null plan or buffer");
+        if (du[i] == u[i]) return fail(DOP_EINVAL, "du must not alias u");
+    }
+    // (plans that tune themselves have tiles, and those go one by one)
+    bool tiles = n > 8;
+    const dop::DevicePlan* p[8] = {};
+    for (int i = 0; i < n && !tiles; ++i) {
+        p[i] = &plans[i]->d;
+        tiles = dop::apply_variants(plans[i]->d) > 1;
+    }
+    if (!tiles) {
+        DOP_HIP(dop::launch_apply_set(n, p, du, u, accumulate, (hipStream_t)stream));
+        return DOP_OK;
+    }
+    for (int i = 0; i < n; ++i) {
+        const int rc = dop_apply(plans[i], du[i], u[i], accumulate[i], stream);
+        if (rc != DOP_OK) return rc;
+    }
+    return DOP_OK;
+}
+
 int dop_plan_variant(const dop_plan* plan, int* tuned)
 {
     if (!plan) return fail(DOP_EINVAL, "null plan");

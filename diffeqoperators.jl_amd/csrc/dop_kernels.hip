@@ -303,8 +303,7 @@ static hipError_t launch_line(const PlanDev& host, const PlanDev* dev, void* du,
     return hipGetLastError();
 }
 
-// the single active axis of a plan the line kernel can take, or -1
-static int line_axis(const PlanDev& h)
+int line_axis(const PlanDev& h)
 {
     if (h.total >= ((int64_t)1 << 31)) return -1;
     int a = -1;

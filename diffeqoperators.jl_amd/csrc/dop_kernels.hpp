@@ -68,6 +68,14 @@ constexpr int kChunkPts = 1024;    // points per chunk of a persistent launch
 hipError_t launch_apply(const DevicePlan& p, void* du, const void* u, int accumulate,
                         int variant, int force_generic, hipStream_t s);
 
+// The single active axis of a plan that the single-axis kernel can take, or -1.
+int line_axis(const PlanDev& h);
+
+// n applies in order (du[i] (+)= plan i of u[i]), as one launch where all are single-axis plans of
+// one shape and no output is read by another term or met again after another output.
+hipError_t launch_apply_set(int n, const DevicePlan* const* plans, void* const* du,
+                            const void* const* u, const int* accumulate, hipStream_t s);
+
 // Number of tile-shape candidates of the plan (autotuner).
 int apply_variants(const DevicePlan& p);
 

@@ -86,6 +86,7 @@ def lib():
     L.dop_plan_output_elems.argtypes = [vp]
     L.dop_plan_output_elems.restype = C.c_int64
     L.dop_apply.argtypes = [vp, vp, vp, i, vp]
+    L.dop_apply_set.argtypes = [i, C.POINTER(vp), C.POINTER(vp), C.POINTER(vp), C.POINTER(i), vp]
     L.dop_plan_autotune.argtypes = [vp, vp, C.POINTER(i)]
     L.dop_plan_update.argtypes = [vp, C.POINTER(DopDesc), vp]
     L.dop_plan_variant.argtypes = [vp, C.POINTER(i)]

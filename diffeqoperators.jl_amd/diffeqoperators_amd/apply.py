@@ -67,13 +67,16 @@ class Plan:
                 pass
             self.handle = None
 
-    def apply(self, du: torch.Tensor, u: torch.Tensor, accumulate: bool = False, stream=None):
+    def check(self, du: torch.Tensor, u: torch.Tensor):
         if du.numel() != self.out_elems or u.numel() != self.in_elems:
             raise AssertionError("array sizes do not match the plan")
         if storage_of(du) != self.storage or storage_of(u) != self.storage:
             raise TypeError("tensor dtype does not match the plan's storage type")
         if du.data_ptr() == u.data_ptr():
             raise ValueError("du must not alias u")
+
+    def apply(self, du: torch.Tensor, u: torch.Tensor, accumulate: bool = False, stream=None):
+        self.check(du, u)
         if stream is None:
             stream = torch.cuda.current_stream(u.device).cuda_stream
         _abi.check(_abi.lib().dop_apply(self.handle, C.c_void_p(du.data_ptr()),
@@ -105,6 +108,21 @@ class Plan:
         _abi.check(_abi.lib().dop_plan_autotune(self.handle, C.c_void_p(stream), C.byref(choice)),
                    "dop_plan_autotune")
         return choice.value
+
+
+def apply_set(terms):
+    """The applies (plan, du, u, accumulate) in order, as one launch where the plans allow it
+    (dop_apply_set), on u's current stream."""
+    n = len(terms)
+    for plan, du, u, _ in terms:
+        plan.check(du, u)
+    vp = C.c_void_p * n
+    stream = torch.cuda.current_stream(terms[0][2].device).cuda_stream
+    _abi.check(_abi.lib().dop_apply_set(n, vp(*(t[0].handle.value for t in terms)),
+                                        vp(*(t[1].data_ptr() for t in terms)),
+                                        vp(*(t[2].data_ptr() for t in terms)),
+                                        (C.c_int * n)(*(int(bool(t[3])) for t in terms)),
+                                        C.c_void_p(stream)), "dop_apply_set")
 
 
 def make_desc(terms, jsize, storage, *, input_kind, semantics, bcs=None, padded=(0, 0, 0),

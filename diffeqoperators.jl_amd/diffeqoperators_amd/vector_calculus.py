@@ -1,7 +1,8 @@
 """Gradient, Divergence and Curl (vector_calculus_operators.jl:5-88) on the device.
 
 Each is a tuple of first-derivative CenteredDifference operators, one per axis; applying one
-runs one fused libdop plan per derivative on the padded input (vector_calculus_convolutions.jl):
+runs one libdop plan per derivative on the padded input, all in one launch (dop_apply_set,
+vector_calculus_convolutions.jl):
 component k of `Gradient * M` is L_k along axis k, `Divergence * M` sums L_k over the
 components, `Curl * M` forms (d2 u3 - d3 u2, d3 u1 - d1 u3, d1 u2 - d2 u1) with the negative
 terms as plans of the negated operators.  For 2-D and 3-D arrays the reference's kernels index
@@ -18,7 +19,7 @@ import numbers
 
 import torch
 
-from .apply import _check_device_tensor, _padded_plan
+from .apply import _check_device_tensor, _padded_plan, apply_set
 from .operators import CenteredDifference
 
 __all__ = ["Gradient", "Divergence", "Curl", "GradientOperator", "DivergenceOperator",
@@ -45,9 +46,9 @@ class _VectorOperator:
             return type(self)(tuple(c * L for L in self.ops))
         return NotImplemented
 
-    def _apply(self, L, du, M, accumulate=False):
+    def _term(self, L, du, M, accumulate=False):
         tv = 1 if M.dim() in (2, 3) else 0
-        _padded_plan(self, [L], du, M, transverse_view=tv).apply(du, M, accumulate=accumulate)
+        return _padded_plan(self, [L], du, M, transverse_view=tv), du, M, accumulate
 
 
 class GradientOperator(_VectorOperator):
@@ -57,8 +58,7 @@ class GradientOperator(_VectorOperator):
         if M.dim() != N:
             raise AssertionError(f"Gradient of {N} dimensions applied to a {M.dim()}-D array")
         out = torch.empty((N,) + tuple(s - 2 for s in M.shape), dtype=M.dtype, device=M.device)
-        for k, L in enumerate(self.ops):
-            self._apply(L, out[k], M)
+        apply_set([self._term(L, out[k], M) for k, L in enumerate(self.ops)])
         return out
 
 
@@ -70,8 +70,7 @@ class DivergenceOperator(_VectorOperator):
             raise AssertionError(f"Divergence of {N} dimensions needs an array of shape "
                                  f"({N}, padded...)")
         out = torch.empty(tuple(s - 2 for s in M.shape[1:]), dtype=M.dtype, device=M.device)
-        for k, L in enumerate(self.ops):
-            self._apply(L, out, M[k], accumulate=k > 0)
+        apply_set([self._term(L, out, M[k], accumulate=k > 0) for k, L in enumerate(self.ops)])
         return out
 
 
@@ -87,9 +86,11 @@ class CurlOperator(_VectorOperator):
         out = torch.empty((3,) + tuple(s - 2 for s in M.shape[1:]), dtype=M.dtype,
                           device=M.device)
         # (d2 u3 - d3 u2, d3 u1 - d1 u3, d1 u2 - d2 u1), d_k along Julia axis k (0-based k-1)
+        terms = []
         for c, (kp, up, km, um) in enumerate(((1, 2, 2, 1), (2, 0, 0, 2), (0, 1, 1, 0))):
-            self._apply(self.ops[kp], out[c], M[up])
-            self._apply(self._neg[km], out[c], M[um], accumulate=True)
+            terms.append(self._term(self.ops[kp], out[c], M[up]))
+            terms.append(self._term(self._neg[km], out[c], M[um], accumulate=True))
+        apply_set(terms)
         return out
 
 

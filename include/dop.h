@@ -192,6 +192,12 @@ int64_t dop_plan_output_elems(const dop_plan* plan);
  * convolutions.jl:49).  stream: hipStream_t (NULL = default stream). */
 int dop_apply(const dop_plan* plan, void* du, const void* u, int accumulate, void* stream);
 
+/* n applies in order, du[i] (+)= plans[i] of u[i] (the terms of a gradient, divergence or curl):
+ * the same results as n dop_apply calls, in one launch where the plans are single-axis ones of
+ * one shape (f64 or f32 storage, up to six).  Terms that add to one output follow each other. */
+int dop_apply_set(int n, const dop_plan* const* plans, void* const* du, const void* const* u,
+                  const int* accumulate, void* stream);
+
 /* ---- batching (no counterpart in the reference: it applies one operator per call) ----
  * A batch binds n independent plans (any mix of ndim, sizes, operators, BCs; one storage
  * type) to their du / u device pointers once; dop_batch_apply then evaluates all of them
