@@ -30,6 +30,7 @@ struct BProb {
     // RK4 steps in one pass (dop_rk4_impl.hpp): fused 1: all of the grid in patches, 2: the box
     // [flo, fhi) in marching segments and the rim in patches; 0: stage by stage
     int32_t fused, fnseg, fchunk;
+    int32_t prow;         // rows of a patch at most
     int32_t flo[2], fhi[2];
     int32_t uniform[2];
     int64_t n0, n1, ys;   // extents and row stride
@@ -66,18 +67,19 @@ constexpr int kPatchLds = 80 << 10;   // bytes of LDS a patch may use, its head 
 constexpr int kPatchHead = 64;         // bytes before a patch's arrays (the stages' regions)
 
 // A run of items that one launch takes.  An apply's items: one kind, window width K (points:
-// shell_point's) and accumulator.  Marching segments: one window, accumulator and grid kind;
-// patches: one accumulator, windows up to 7 or up to 11 taps.  The items of an RK4 stage: one
+// shell_point's) and accumulator.  A pass (kItemPatch): the patches and the marching segments of one window
+// and accumulator.  The items of an RK4 stage: one
 // accumulator, the tiles of all kinds and windows together (kItemStage), the points likewise.
 constexpr int32_t kItemStage = 6;
 struct BGroup {
     int32_t kind, K, acc, uniform, first, count;
-    int32_t lds;   // patches: bytes of LDS of the largest one
+    int32_t patches;   // a pass: its patches, which come before its marching segments
+    int32_t lds;       // bytes of LDS of the largest of them
 };
 
 // Fills probs[i] geometry from plan i.  rk4: for RK4 stages (fused where that pays).
 void batch_geometry(const DevicePlan& p, int chunk, BProb* B, bool rk4 = false);
-// Rows per chunk of the marching segments of `probs`, launched together.
+// Rows per chunk of the marching segments and per patch of `probs`, launched together.
 void batch_march_chunks(std::vector<BProb>* probs);
 // Work items of all problems for row chunk B.chunk, sorted into groups; rk4: of RK4 steps.
 void batch_items(const std::vector<BProb>& probs, bool rk4, std::vector<BItem>* items,
@@ -85,7 +87,7 @@ void batch_items(const std::vector<BProb>& probs, bool rk4, std::vector<BItem>* 
 
 // The groups of a launch set: the stages' (or an apply's), the one-pass steps', the copies back.
 inline bool group_is_stage(const BGroup& g) { return g.kind <= kItemTile1 || g.kind == kItemStage; }
-inline bool group_is_pass(const BGroup& g) { return g.kind == kItemPatch || g.kind == kItemMarch; }
+inline bool group_is_pass(const BGroup& g) { return g.kind == kItemPatch; }
 inline bool group_is_back(const BGroup& g) { return g.kind == kItemBack; }
 
 // The state of a fused problem alternates between u and acc: step `parity` reads u (0) or acc (1)

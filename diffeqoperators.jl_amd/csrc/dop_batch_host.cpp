@@ -19,6 +19,8 @@ namespace {
 // pay (its rim, 4H to 5H points a side, and the 4H columns beside every segment are recomputed).
 constexpr int kMarchMin = 96;
 
+constexpr int kPatchRows = 32;   // rows of own points of a patch at most
+
 bool march_box(const PlanDev& P, const FastArgs& A, BProb* B)
 {
     const int VX = march_vx(P.storage, P.accum, A.K), H = A.K / 2;
@@ -36,7 +38,7 @@ bool march_box(const PlanDev& P, const FastArgs& A, BProb* B)
     return true;
 }
 
-// LDS bytes of a patch (k_rk4_patch): u and two stage arrays over all that its points' cones
+// LDS bytes of a patch (rk4_patch): its head, u and two stage arrays over all that its points' cones
 // reach, the stage sums over its points
 int64_t patch_bytes(const PlanDev& P, int H, int x0, int x1, int y0, int y1)
 {
@@ -49,13 +51,12 @@ int64_t patch_bytes(const PlanDev& P, int H, int x0, int x1, int y0, int y1)
 }
 
 // Patch extents (w, h) for a rectangle of points of the grid: lines of up to 128 loaded points
-// (two waves of lanes) by all of a rim's rows if the LDS holds them, else by what it holds; thin
-// rectangles keep their width.  False when even small patches do not fit.
-bool patch_size(const PlanDev& P, int H, int x0, int x1, int y0, int y1, int* w, int* h)
+// (two waves of lanes) by up to `rows` rows as the LDS holds them; thin rectangles keep their width.  False when even small patches do not fit.
+bool patch_size(const PlanDev& P, int H, int rows, int x0, int x1, int y0, int y1, int* w, int* h)
 {
-    // what the patch's points reach beyond them over four stages: along an axis that is not split,
-    // what the rectangle reaches; else at its widest (windows on both sides and, on one side,
-    // boundary rows, whose windows may be one longer than the reach in)
+    // what the patch's points reach beyond them over four stages: at its widest, windows on both
+    // sides and, on one side, boundary rows, whose windows may be one longer than the reach in; and
+    // never beyond what the whole rectangle reaches
     const int lo[2] = {x0, y0}, hi[2] = {x1, y1};
     int ext[2] = {0, 0}, all[2] = {0, 0};
     for (int a = 0; a < P.ndim; ++a) {
@@ -67,9 +68,8 @@ bool patch_size(const PlanDev& P, int H, int x0, int x1, int y0, int y1, int* w,
     const int rw = x1 - x0, rh = y1 - y0;
     const int64_t sb = P.storage == kF64 ? 8 : 4;
     auto fits = [&](int ww, int hh) {
-        const int64_t ew = ww == rw ? all[0] : ext[0], eh = hh == rh ? all[1] : ext[1];
-        return kPatchHead + (3 * ((ww + ew) | 1) * (hh + eh) + (int64_t)(ww | 1) * hh) * sb <=
-               kPatchLds;
+        const int64_t w = std::min(ww + ext[0], rw + all[0]), h = std::min(hh + ext[1], rh + all[1]);
+        return kPatchHead + (3 * (w | 1) * h + (int64_t)(ww | 1) * hh) * sb <= kPatchLds;
     };
     if (P.ndim == 1) {
         *w = std::min(rw, 1024);
@@ -82,7 +82,7 @@ bool patch_size(const PlanDev& P, int H, int x0, int x1, int y0, int y1, int* w,
             if (fits(*w, *h)) return true;
         return false;
     }
-    for (*h = std::min(rh, 32); *h >= 4; *h = *h > 8 ? (*h + 1) / 2 : *h - 2) {
+    for (*h = std::min(rh, rows); *h >= 4; *h = *h > 8 ? (*h + 1) / 2 : *h - 2) {
         for (*w = std::min(rw, 128 - std::min(8 * H, 96)); *w >= 16 || *w == rw; *w -= 4)
             if (fits(*w, *h)) return true;
     }
@@ -90,10 +90,10 @@ bool patch_size(const PlanDev& P, int H, int x0, int x1, int y0, int y1, int* w,
 }
 
 template <typename F>
-void patches(const PlanDev& P, int H, int x0, int x1, int y0, int y1, const F& f)
+void patches(const PlanDev& P, int H, int rows, int x0, int x1, int y0, int y1, const F& f)
 {
     int w, h;
-    if (x1 <= x0 || y1 <= y0 || !patch_size(P, H, x0, x1, y0, y1, &w, &h)) return;
+    if (x1 <= x0 || y1 <= y0 || !patch_size(P, H, rows, x0, x1, y0, y1, &w, &h)) return;
     // even pieces
     const int nx = (int)ceil_div(x1 - x0, w), ny = (int)ceil_div(y1 - y0, h);
     for (int j = 0; j < ny; ++j)
@@ -132,6 +132,7 @@ void batch_geometry(const DevicePlan& p, int chunk, BProb* B, bool rk4)
     B->hplan = &p.host;
     B->pfast = B->tiled && f.args.pfast ? f.args.K : 0;
     B->fused = 0;
+    B->prow = kPatchRows;
     if (B->tiled) {
         const FastArgs& A = f.args;
         const int H = A.K / 2;
@@ -156,8 +157,8 @@ void batch_geometry(const DevicePlan& p, int chunk, BProb* B, bool rk4)
             patch_rects(*B, (int)P.n[0], (int)P.n[1], [&](int x0, int x1, int y0, int y1) {
                 int w, h;
                 if (x1 <= x0 || y1 <= y0) return;
-                fits = fits && patch_size(P, B->K / 2, x0, x1, y0, y1, &w, &h);
-                if (fits) patches(P, B->K / 2, x0, x1, y0, y1, [&](int xa, int xb, int ya, int yb) {
+                fits = fits && patch_size(P, B->K / 2, kPatchRows, x0, x1, y0, y1, &w, &h);
+                if (fits) patches(P, B->K / 2, kPatchRows, x0, x1, y0, y1, [&](int xa, int xb, int ya, int yb) {
                     fits = fits && patch_bytes(P, B->K / 2, xa, xb, ya, yb) <= kPatchLds;
                 });
             });
@@ -191,6 +192,30 @@ void batch_march_chunks(std::vector<BProb>* probs)
     int chunk = 16;
     while (chunk < 64 && waves(chunk) > 2048) chunk += 4;
     for (BProb& B : *probs) B.fchunk = chunk;
+    // Rows of a patch: a block's chain is its rows, so lower patches (more rows recomputed) where
+    // the tall ones would leave CUs without a block of the two they hold
+    // (0: some patch would not fit)
+    auto blocks = [&](int rows) {
+        int64_t n = 0;
+        bool fits = true;
+        for (const BProb& B : *probs) {
+            if (!B.fused) continue;
+            const PlanDev& P = *B.hplan;
+            patch_rects(B, (int)P.n[0], (int)P.n[1], [&](int x0, int x1, int y0, int y1) {
+                int64_t left = x1 > x0 && y1 > y0 ? (int64_t)(x1 - x0) * (y1 - y0) : 0;
+                patches(P, B.K / 2, rows, x0, x1, y0, y1, [&](int xa, int xb, int ya, int yb) {
+                    ++n;
+                    left -= (int64_t)(xb - xa) * (yb - ya);
+                    fits = fits && patch_bytes(P, B.K / 2, xa, xb, ya, yb) <= kPatchLds;
+                });
+                fits = fits && left == 0;
+            });
+        }
+        return fits ? n : 0;
+    };
+    int rows = kPatchRows;
+    while (rows > 8 && blocks(rows) < 512 && blocks(rows / 2) > 0) rows /= 2;
+    for (BProb& B : *probs) B.prow = rows;
 }
 
 void batch_items(const std::vector<BProb>& probs, bool rk4, std::vector<BItem>* items,
@@ -199,9 +224,8 @@ void batch_items(const std::vector<BProb>& probs, bool rk4, std::vector<BItem>* 
     auto key = [&](const BItem& I) {
         const BProb& B = probs[I.prob];
         if (I.kind == kItemBack) return std::make_tuple((int)kItemBack, 0, 0, 0);
-        if (I.kind == kItemPatch) return std::make_tuple((int)kItemPatch, B.K, B.plan_accum, 0);
-        if (I.kind == kItemMarch)
-            return std::make_tuple((int)kItemMarch, B.K, B.plan_accum, B.uniform[0] && B.uniform[1] ? 1 : 0);
+        if (I.kind == kItemPatch || I.kind == kItemMarch)
+            return std::make_tuple((int)kItemPatch, B.K, B.plan_accum, 0);
         if (rk4) return std::make_tuple(I.kind == kItemPoints ? (int)kItemPoints : (int)kItemStage, 0, B.plan_accum, 0);
         return std::make_tuple(I.kind, I.kind == kItemPoints ? B.pfast : B.K, B.plan_accum, 0);
     };
@@ -212,7 +236,7 @@ void batch_items(const std::vector<BProb>& probs, bool rk4, std::vector<BItem>* 
         if (B.fused) {
             const PlanDev& P = *B.hplan;
             patch_rects(B, (int)P.n[0], (int)P.n[1], [&](int x0, int x1, int y0, int y1) {
-                patches(P, B.K / 2, x0, x1, y0, y1, [&](int xa, int xb, int ya, int yb) {
+                patches(P, B.K / 2, B.prow, x0, x1, y0, y1, [&](int xa, int xb, int ya, int yb) {
                     items->push_back({p, kItemPatch, xa, xb, ya, yb});
                 });
             });
@@ -239,17 +263,21 @@ void batch_items(const std::vector<BProb>& probs, bool rk4, std::vector<BItem>* 
         for (int64_t c = 0; c < ns; ++c) items->push_back({p, kItemPoints, (int32_t)c, 0, 0, 0});
     }
     std::stable_sort(items->begin(), items->end(),
-                     [&](const BItem& a, const BItem& b) { return key(a) < key(b); });
+                     [&](const BItem& a, const BItem& b) {
+                         const auto ka = key(a), kb = key(b);
+                         return ka != kb ? ka < kb : a.kind == kItemPatch && b.kind == kItemMarch;
+                     });
     groups->clear();
     for (size_t k = 0; k < items->size(); ++k) {
         const BItem& I = (*items)[k];
         if (groups->empty() || key((*items)[groups->back().first]) != key(I)) {
             const auto t = key(I);
             groups->push_back({std::get<0>(t), std::get<1>(t), std::get<2>(t), std::get<3>(t),
-                               (int32_t)k, 0, 0});
+                               (int32_t)k, 0, 0, 0});
         }
         BGroup& g = groups->back();
         ++g.count;
+        if (I.kind == kItemPatch) ++g.patches;
         if (I.kind == kItemPatch)
             g.lds = std::max(g.lds, (int32_t)patch_bytes(*probs[I.prob].hplan, probs[I.prob].K / 2, I.a, I.b, I.c, I.d));
     }

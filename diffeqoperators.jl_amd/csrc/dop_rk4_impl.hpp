@@ -2,10 +2,10 @@
 //
 // Stage by stage a step moves 16 values per point through memory (stage 0 reads u and writes the
 // stage sum and the next stage's input, ...: 64 bytes per f32 point) and is a chain of four launch
-// sets.  Here u is read once and the new state written once (8 bytes per point), by two kernels that
+// sets.  Here u is read once and the new state written once (8 bytes per point), in two ways that
 // do not depend on each other:
 //
-// k_rk4_march, the bulk of a 2-D grid: a wave marches down a segment of rows with the four stages
+// rk4_march, the bulk of a 2-D grid: a wave marches down a segment of rows with the four stages
 // following each other H rows apart.  While row c of u arrives, stage 0 forms row c of its output,
 // stage 1 row c - H, stage 2 row c - 2H and stage 3 the new state's row c - 3H, each from a
 // register ring of the K rows of the stage before it.  Segments overlap by the 4H columns a step's
@@ -16,20 +16,24 @@
 // in L2).  Bound by its own instructions (f32, K = 7: 22 a point and stage, DPP shifts at a third
 // of the FMA rate among them).
 //
-// k_rk4_patch, the rim of the box (or all of a small or 1-D grid): a block loads a patch with all
+// rk4_patch, the rim of the box (or all of a small or 1-D grid): a block loads a patch with all
 // that its points' cones reach (rows_reach: windows, boundary rows, ghosts) into LDS and runs the
 // four stages there, each over the region the next one reads.  Bound by instruction issue and the
-// latency of a block's chain of rows.  A line's weights and boundary data stay in registers over
-// the rows: with shell_point_f at every point near an edge the mixed problems below took 1.71 ms a
-// step and the served ones 25.1 ms, against 1.52 and 20.9.  Patches of all a rim's rows, for which
-// the LDS holds 80 KB (two blocks a CU), halve the recomputed points at K = 9 and 11: 1.30 ms.
-// Tried: 512 threads and four rows side by side, 1.75 ms (the scalar registers spill).
+// latency of a block's chain of rows: a line's weights and boundary data stay in registers over
+// the rows, patches take all of a rim's rows (the LDS holds 80 KB, two blocks a CU; at K = 9 and 11
+// half the recomputed points of 64 KB), and lower ones where few blocks would leave CUs idle.
+// Tried: 512 threads and four rows side by side, slower (the scalar registers spill).
+//
+// A class of problems (one window and accumulator) is one launch, k_rk4_pass: the two kinds of
+// blocks need the same registers and LDS, so that the patches, whose chains are long, and the
+// segments, which keep the SIMDs busy, share the CUs.
 //
 // Every stage value is rounded to the storage type exactly where the stage-wise kernels store it,
 // and every sum runs in their order, so the new state is the same bit for bit.  The new state goes
 // to acc, so u and acc swap roles from step to step.
 // Measured against the stage-wise step: 256 mixed f32 problems (1-D to 65536, 2-D to 2048 squared,
-// orders 2 to 8) 2.08 -> 1.30 ms a step, 24 served 2-D requests of 100 steps 36.7 -> 20.6 ms.
+// orders 2 to 8) 2.08 -> 1.09 ms a step, 24 served 2-D requests of 100 steps 36.7 -> 19.3 ms (as two launches
+// a class: 1.30 and 20.6).
 #pragma once
 #include "dop_batch_impl.hpp"
 
@@ -99,10 +103,12 @@ __device__ inline W const_tab(const W* p, int64_t i)
     return ((const __attribute__((address_space(4))) W*)p)[i];
 }
 
+// LDS bytes of a marching wave: the stage sums' ring
+template <typename T, int ACC, int K>
+constexpr int kMarchLds = (3 * (K / 2) + 1) * 64 * march_vx(sizeof(T) == 8 ? kF64 : kF32, ACC, K) * (int)sizeof(T);
+
 template <typename T, int ACC, int K, bool UNI>
-__global__ __launch_bounds__(64, 2) void k_rk4_march(const BProb* __restrict__ probs,
-                                                     const BItem* __restrict__ items, int nitems,
-                                                     int parity)
+__device__ inline void rk4_march(const BProb& B, const BItem& I, T* __restrict__ lds, int parity)
 {
     using W = typename Acc<ACC>::W;
     constexpr int VX = march_vx(sizeof(T) == 8 ? kF64 : kF32, ACC, K);
@@ -111,133 +117,129 @@ __global__ __launch_bounds__(64, 2) void k_rk4_march(const BProb* __restrict__ p
     constexpr int PAD = (4 * H + VX - 1) / VX * VX;   // columns recomputed on each side
     constexpr int OUT = 64 * VX - 2 * PAD;
     constexpr int D = 3 * H + 1;                   // rows a stage sum waits
-    __shared__ __attribute__((aligned(16))) T sums[D][64][VX];
-    const int lane = threadIdx.x;
-    for (int it = blockIdx.x; it < nitems; it += gridDim.x) {
-        const BItem I = items[it];
-        const BProb& B = probs[I.prob];
-        const int seg = I.a;
-        const T* u = (const T*)(parity ? B.acc : B.u);
-        T* out = (T*)(parity ? B.u : B.acc);
-        const int y0 = B.flo[1] + I.b * B.fchunk;
-        const int y1 = min(y0 + B.fchunk, B.fhi[1]);
-        const int n0 = (int)B.n0, n1 = (int)B.n1;
-        const int64_t s1 = B.ys;
-        const int xb = B.flo[0] + seg * OUT;        // first output column of the segment
-        const int xs = xb - PAD + lane * VX;
-        const int xe = min(xb + OUT, B.fhi[0]);
-        const bool st_ok = xs >= xb && xs < xe;     // whole groups: OUT and the box are multiples of VX
-        // lanes beyond the array load another group; no output's cone reaches them
-        const int xl = min(max(xs, 0), n0 - VX);
-        const T* ucol = u + xl;
-        const W* wxt = btab<ACC>(B, 0);
-        const W* wyt = btab<ACC>(B, 1);
-        W wx[UNI ? 1 : VX][K], wyu[UNI ? K : 1];
+    const int lane = threadIdx.x & 63;
+    auto sums = [&](int d) -> T* { return lds + (d * 64 + lane) * VX; };
+    const int seg = I.a;
+    const T* u = (const T*)(parity ? B.acc : B.u);
+    T* out = (T*)(parity ? B.u : B.acc);
+    const int y0 = B.flo[1] + I.b * B.fchunk;
+    const int y1 = min(y0 + B.fchunk, B.fhi[1]);
+    const int n0 = (int)B.n0, n1 = (int)B.n1;
+    const int64_t s1 = B.ys;
+    const int xb = B.flo[0] + seg * OUT;        // first output column of the segment
+    const int xs = xb - PAD + lane * VX;
+    const int xe = min(xb + OUT, B.fhi[0]);
+    const bool st_ok = xs >= xb && xs < xe;     // whole groups: OUT and the box are multiples of VX
+    // lanes beyond the array load another group; no output's cone reaches them
+    const int xl = min(max(xs, 0), n0 - VX);
+    const T* ucol = u + xl;
+    const W* wxt = btab<ACC>(B, 0);
+    const W* wyt = btab<ACC>(B, 1);
+    W wx[UNI ? 1 : VX][K], wyu[UNI ? K : 1];
 #pragma unroll
-        for (int v = 0; v < (UNI ? 1 : VX); ++v) {
-            const int64_t xr = UNI ? 0 : min(max(xs + v, 0), n0 - 1);
+    for (int v = 0; v < (UNI ? 1 : VX); ++v) {
+        const int64_t xr = UNI ? 0 : min(max(xs + v, 0), n0 - 1);
 #pragma unroll
-            for (int k = 0; k < K; ++k) wx[v][k] = UNI ? const_tab(wxt, k) : wxt[xr * K + k];
-        }
-        if constexpr (UNI) {
+        for (int k = 0; k < K; ++k) wx[v][k] = UNI ? const_tab(wxt, k) : wxt[xr * K + k];
+    }
+    if constexpr (UNI) {
 #pragma unroll
-            for (int k = 0; k < K; ++k) wyu[k] = const_tab(wyt, k);
-        }
-        const double scale = B.scale, dt = B.dt;
-        const int ylast = min(y1 + 4 * H - 1, n1 - 1);
-        auto load_row = [&](int row, T* dst) {
-            RowIO<T, VX>::ld(ucol + (int64_t)min(max(row, 0), ylast) * s1, dst);
-        };
-        // rings: slot (t + k) % R of step t holds row c - H + k of u (q[0]) and row
-        // c - jH - H + k of stage j's input (q[j])
-        T q[4][R][VX];
-        const int c0 = y0 - 3 * H;
+        for (int k = 0; k < K; ++k) wyu[k] = const_tab(wyt, k);
+    }
+    const double scale = B.scale, dt = B.dt;
+    const int ylast = min(y1 + 4 * H - 1, n1 - 1);
+    auto load_row = [&](int row, T* dst) {
+        RowIO<T, VX>::ld(ucol + (int64_t)min(max(row, 0), ylast) * s1, dst);
+    };
+    // rings: slot (t + k) % R of step t holds row c - H + k of u (q[0]) and row
+    // c - jH - H + k of stage j's input (q[j])
+    T q[4][R][VX];
+    const int c0 = y0 - 3 * H;
 #pragma unroll
-        for (int s = 0; s < R - 1; ++s) load_row(c0 - H + s, q[0][s]);
-        // slots of the waiting sums: rows c, c - H, c - 2H, c - 3H
-        int d0 = 0, d1 = D - H, d2 = D - 2 * H, d3 = D - 3 * H;
-        const int steps = (y1 - y0) + 6 * H;
-        for (int t0 = 0; t0 < steps; t0 += R) {
-            auto step = [&](auto jc) -> bool {
-                constexpr int j = decltype(jc)::value;
-                const int t = t0 + j;
-                if (t >= steps) return false;
-                const int c = c0 + t;
-                load_row(c + H + 1, q[0][(j + K) % R]);
-                T ue[VX];   // u at stage 2's row
-                load_row(c - 2 * H, ue);
-                // one stage: row y of its values v from the window rows of ring Q
-                auto values = [&](const T(*Q)[VX], int y, double* val) {
-                    T xw[VX + 2 * H];
-                    march_window<T, VX, H>(Q[(j + H) % R], xw);
-                    W wy[K];
+    for (int s = 0; s < R - 1; ++s) load_row(c0 - H + s, q[0][s]);
+    // slots of the waiting sums: rows c, c - H, c - 2H, c - 3H
+    int d0 = 0, d1 = D - H, d2 = D - 2 * H, d3 = D - 3 * H;
+    const int steps = (y1 - y0) + 6 * H;
+    for (int t0 = 0; t0 < steps; t0 += R) {
+        auto step = [&](auto jc) -> bool {
+            constexpr int j = decltype(jc)::value;
+            const int t = t0 + j;
+            if (t >= steps) return false;
+            const int c = c0 + t;
+            load_row(c + H + 1, q[0][(j + K) % R]);
+            T ue[VX];   // u at stage 2's row
+            load_row(c - 2 * H, ue);
+            // one stage: row y of its values v from the window rows of ring Q
+            auto values = [&](const T(*Q)[VX], int y, double* val) {
+                T xw[VX + 2 * H];
+                march_window<T, VX, H>(Q[(j + H) % R], xw);
+                W wy[K];
 #pragma unroll
-                    for (int k = 0; k < K; ++k) wy[k] = UNI ? wyu[UNI ? k : 0] : const_tab(wyt, (int64_t)y * K + k);
+                for (int k = 0; k < K; ++k) wy[k] = UNI ? wyu[UNI ? k : 0] : const_tab(wyt, (int64_t)y * K + k);
 #pragma unroll
-                    for (int v = 0; v < VX; ++v) {
-                        Acc<ACC> a;
+                for (int v = 0; v < VX; ++v) {
+                    Acc<ACC> a;
 #pragma unroll
-                        for (int k = 0; k < K; ++k) a.add(wx[UNI ? 0 : v][k], (W)xw[v + k]);
+                    for (int k = 0; k < K; ++k) a.add(wx[UNI ? 0 : v][k], (W)xw[v + k]);
 #pragma unroll
-                        for (int k = 0; k < K; ++k) a.add(wy[k], (W)Q[(j + k) % R][v]);
-                        val[v] = a.value();
-                    }
-                };
-                double val[VX];
-                T sum[VX];
-                constexpr int nw = (j + K - 1) % R;   // slot of the row a stage adds to the next ring
-                // stage 0, row c
-                values(q[0], c, val);
+                    for (int k = 0; k < K; ++k) a.add(wy[k], (W)Q[(j + k) % R][v]);
+                    val[v] = a.value();
+                }
+            };
+            double val[VX];
+            T sum[VX];
+            constexpr int nw = (j + K - 1) % R;   // slot of the row a stage adds to the next ring
+            // stage 0, row c
+            values(q[0], c, val);
+#pragma unroll
+            for (int v = 0; v < VX; ++v) {
+                const double k = scale * val[v];
+                const double up = (double)q[0][(j + H) % R][v];
+                sum[v] = (T)(up + (dt / 6.0) * k);
+                q[1][nw][v] = (T)(up + (0.5 * dt) * k);
+            }
+            RowIO<T, VX>::st(sums(d0), sum);
+            if (t >= 2 * H) {   // stage 1, row c - H (wave-uniform)
+                RowIO<T, VX>::ld(sums(d1), sum);
+                values(q[1], c - H, val);
 #pragma unroll
                 for (int v = 0; v < VX; ++v) {
                     const double k = scale * val[v];
-                    const double up = (double)q[0][(j + H) % R][v];
-                    sum[v] = (T)(up + (dt / 6.0) * k);
-                    q[1][nw][v] = (T)(up + (0.5 * dt) * k);
+                    const double up = (double)q[0][j % R][v];
+                    sum[v] = (T)((double)sum[v] + (dt / 3.0) * k);
+                    q[2][nw][v] = (T)(up + (0.5 * dt) * k);
                 }
-                RowIO<T, VX>::st(&sums[d0][lane][0], sum);
-                if (t >= 2 * H) {   // stage 1, row c - H (wave-uniform)
-                    RowIO<T, VX>::ld(&sums[d1][lane][0], sum);
-                    values(q[1], c - H, val);
+                RowIO<T, VX>::st(sums(d1), sum);
+            }
+            if (t >= 4 * H) {   // stage 2, row c - 2H
+                RowIO<T, VX>::ld(sums(d2), sum);
+                values(q[2], c - 2 * H, val);
 #pragma unroll
-                    for (int v = 0; v < VX; ++v) {
-                        const double k = scale * val[v];
-                        const double up = (double)q[0][j % R][v];
-                        sum[v] = (T)((double)sum[v] + (dt / 3.0) * k);
-                        q[2][nw][v] = (T)(up + (0.5 * dt) * k);
-                    }
-                    RowIO<T, VX>::st(&sums[d1][lane][0], sum);
+                for (int v = 0; v < VX; ++v) {
+                    const double k = scale * val[v];
+                    const double up = (double)ue[v];
+                    sum[v] = (T)((double)sum[v] + (dt / 3.0) * k);
+                    q[3][nw][v] = (T)(up + dt * k);
                 }
-                if (t >= 4 * H) {   // stage 2, row c - 2H
-                    RowIO<T, VX>::ld(&sums[d2][lane][0], sum);
-                    values(q[2], c - 2 * H, val);
+                RowIO<T, VX>::st(sums(d2), sum);
+            }
+            if (t >= 6 * H) {   // stage 3, row c - 3H: the new state
+                RowIO<T, VX>::ld(sums(d3), sum);
+                values(q[3], c - 3 * H, val);
 #pragma unroll
-                    for (int v = 0; v < VX; ++v) {
-                        const double k = scale * val[v];
-                        const double up = (double)ue[v];
-                        sum[v] = (T)((double)sum[v] + (dt / 3.0) * k);
-                        q[3][nw][v] = (T)(up + dt * k);
-                    }
-                    RowIO<T, VX>::st(&sums[d2][lane][0], sum);
+                for (int v = 0; v < VX; ++v) {
+                    const double k = scale * val[v];
+                    sum[v] = (T)((double)sum[v] + (dt / 6.0) * k);
                 }
-                if (t >= 6 * H) {   // stage 3, row c - 3H: the new state
-                    RowIO<T, VX>::ld(&sums[d3][lane][0], sum);
-                    values(q[3], c - 3 * H, val);
-#pragma unroll
-                    for (int v = 0; v < VX; ++v) {
-                        const double k = scale * val[v];
-                        sum[v] = (T)((double)sum[v] + (dt / 6.0) * k);
-                    }
-                    if (st_ok) RowIO<T, VX>::st(out + (int64_t)(c - 3 * H) * s1 + xs, sum);
-                }
-                d0 = d0 + 1 == D ? 0 : d0 + 1;
-                d1 = d1 + 1 == D ? 0 : d1 + 1;
-                d2 = d2 + 1 == D ? 0 : d2 + 1;
-                d3 = d3 + 1 == D ? 0 : d3 + 1;
-                return true;
-            };
-            if (!ring_steps<0, R>(step)) break;
-        }
+                if (st_ok) RowIO<T, VX>::st(out + (int64_t)(c - 3 * H) * s1 + xs, sum);
+            }
+            d0 = d0 + 1 == D ? 0 : d0 + 1;
+            d1 = d1 + 1 == D ? 0 : d1 + 1;
+            d2 = d2 + 1 == D ? 0 : d2 + 1;
+            d3 = d3 + 1 == D ? 0 : d3 + 1;
+            return true;
+        };
+        if (!ring_steps<0, R>(step)) break;
     }
 }
 
@@ -293,6 +295,18 @@ __device__ inline const W* const& axis_table(const AxisDev& X)
 {
     if constexpr (std::is_same<W, double>::value) return X.w64;
     else return X.w32;
+}
+
+__device__ inline float patch_lane(float v, int lane)
+{
+    return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), lane));
+}
+__device__ inline double patch_lane(double v, int lane)
+{
+    const uint64_t b = __builtin_bit_cast(uint64_t, v);
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)b, lane);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(b >> 32), lane);
+    return __builtin_bit_cast(double, (uint64_t)lo | ((uint64_t)hi << 32));
 }
 
 // A field of a plan or problem (they do not change while a launch reads them), in scalar registers
@@ -387,7 +401,20 @@ __device__ inline void patch_stage(const BProb& B, const PlanDev& P, const Patch
             }
         }
         const int mb = m0 + part * per, me = min(mb + per, m1);
+        // weights of the rows to come, row mb + i in lane i: a scalar load a row would be waited for
+        // with the row's LDS reads
+        W wr[K];
+        auto row_weights = [&](int m) {
+#pragma unroll
+            for (int k = 0; k < K; ++k) wr[k] = wmt[(int64_t)min(m + lane, nM - 1) * K + k];
+        };
+        if (!uM) row_weights(mb);
         for (int m = mb; m < me; ++m) {
+            if (!uM) {
+                if (m > mb && ((m - mb) & 63) == 0) row_weights(m);
+#pragma unroll
+                for (int k = 0; k < K; ++k) wm[k] = patch_lane(wr[k], (m - mb) & 63);
+            }
             if (!lin) continue;
             const bool mreg = m >= bm0 && m < bm1;   // wave-uniform
             const int pl = in + (m - om) * sm, pm = in + (l - ol) * sl;   // the point's two lines
@@ -435,7 +462,6 @@ __device__ inline void patch_stage(const BProb& B, const PlanDev& P, const Patch
 #pragma unroll
                     for (int k = 0; k < K; ++k) {
                         t[k] = atm(m - H + k);
-                        if (!uM) wm[k] = const_tab(wmt, (int64_t)m * K + k);
                     }
                     if (padm && !lreg) {
 #pragma unroll
@@ -521,65 +547,84 @@ __device__ inline void patch_stage1(const BProb& B, const PlanDev& P, const Patc
 
 // The points [a, b) x [c, d) of a problem.
 template <typename T, int ACC, int K>
-__global__ __launch_bounds__(kPatchBlock) void k_rk4_patch(const BProb* __restrict__ probs,
-                                                    const BItem* __restrict__ items, int nitems,
-                                                    int parity)
+__device__ inline void rk4_patch(const BProb& B, const BItem& I, int parity)
 {
-    for (int it = blockIdx.x; it < nitems; it += gridDim.x) {
+    const PlanDev& P = *B.plan;
+    const T* src = (const T*)(parity ? B.acc : B.u);
+    T* out = (T*)(parity ? B.u : B.acc);
+    int x0 = I.a, x1 = I.b, y0 = I.c, y1 = I.d;
+    int* reg = reinterpret_cast<int*>(patch_lds);
+#pragma unroll
+    for (int s = 3; s >= 0; --s) {
+        if (threadIdx.x == 0) {
+            reg[4 * s] = x0;
+            reg[4 * s + 1] = x1;
+            reg[4 * s + 2] = y0;
+            reg[4 * s + 3] = y1;
+        }
+        rows_reach(P.ax[0], K / 2, &x0, &x1);
+        if (B.nd == 2) rows_reach(P.ax[1], K / 2, &y0, &y1);
+    }
+    const int lh = y1 - y0;
+    Patch Q;
+    Q.o0 = x0;
+    Q.o1 = y0;
+    Q.pitch = (x1 - x0) | 1;
+    Q.sz = Q.pitch * lh;
+    Q.a0 = I.a;
+    Q.a1 = I.c;
+    Q.ow = (I.b - I.a) | 1;
+    // load: rows in turn (32-bit reciprocal of the width, exact for the fewer than 2^14 points
+    // of a patch)
+    const uint32_t w = (uint32_t)(x1 - x0), n = w * (uint32_t)lh;
+    const uint32_t mul = w > 1 ? (uint32_t)((0x100000000ull + w - 1) / w) : 0;
+    const int64_t ys = patch_field(B.ys);
+    const T* s0 = src + (int64_t)y0 * ys + x0;
+    for (uint32_t p = threadIdx.x; p < n; p += kPatchBlock * 8) {   // eight loads in flight
+        T v[8];
+        int at[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const uint32_t pi = min(p + i * kPatchBlock, n - 1);
+            const uint32_t q = w > 1 ? __umulhi(pi, mul) : pi, c = pi - q * w;
+            at[i] = (int)(q * Q.pitch + c);
+            v[i] = s0[(int64_t)q * ys + c];
+        }
+#pragma unroll
+        for (int i = 0; i < 8; ++i) patch_at<T>(at[i]) = v[i];   // (clamped ones: the same value)
+    }
+    __syncthreads();
+#pragma unroll 1
+    for (int s = 0; s < 4; ++s) {
+        if (B.nd == 1) patch_stage1<T, ACC, K>(B, P, Q, s, out);
+        else if ((int)w >= lh) patch_stage<T, ACC, K, 0>(B, P, Q, s, out);
+        else patch_stage<T, ACC, K, 1>(B, P, Q, s, out);
+        __syncthreads();
+    }
+}
+
+// A step of a class of problems: blocks of the patches first (the longer ones), then blocks of
+// four marching segments, a wave each.
+template <typename T, int ACC, int K>
+__global__ __launch_bounds__(kPatchBlock, 2) void k_rk4_pass(const BProb* __restrict__ probs,
+                                                             const BItem* __restrict__ items,
+                                                             int npatch, int nitems, int parity)
+{
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int units = npatch + (nitems - npatch + 3) / 4;
+    for (int un = blockIdx.x; un < units; un += gridDim.x) {
+        if (un < npatch) {
+            const BItem I = items[un];
+            rk4_patch<T, ACC, K>(probs[I.prob], I, parity);
+            continue;
+        }
+        const int it = npatch + (un - npatch) * 4 + wave;
+        if (it >= nitems) continue;
         const BItem I = items[it];
         const BProb& B = probs[I.prob];
-        const PlanDev& P = *B.plan;
-        const T* src = (const T*)(parity ? B.acc : B.u);
-        T* out = (T*)(parity ? B.u : B.acc);
-        int x0 = I.a, x1 = I.b, y0 = I.c, y1 = I.d;
-        int* reg = reinterpret_cast<int*>(patch_lds);
-#pragma unroll
-        for (int s = 3; s >= 0; --s) {
-            if (threadIdx.x == 0) {
-                reg[4 * s] = x0;
-                reg[4 * s + 1] = x1;
-                reg[4 * s + 2] = y0;
-                reg[4 * s + 3] = y1;
-            }
-            rows_reach(P.ax[0], K / 2, &x0, &x1);
-            if (B.nd == 2) rows_reach(P.ax[1], K / 2, &y0, &y1);
-        }
-        const int lh = y1 - y0;
-        Patch Q;
-        Q.o0 = x0;
-        Q.o1 = y0;
-        Q.pitch = (x1 - x0) | 1;
-        Q.sz = Q.pitch * lh;
-        Q.a0 = I.a;
-        Q.a1 = I.c;
-        Q.ow = (I.b - I.a) | 1;
-        // load: rows in turn (32-bit reciprocal of the width, exact for the fewer than 2^14 points
-        // of a patch)
-        const uint32_t w = (uint32_t)(x1 - x0), n = w * (uint32_t)lh;
-        const uint32_t mul = w > 1 ? (uint32_t)((0x100000000ull + w - 1) / w) : 0;
-        const int64_t ys = patch_field(B.ys);
-        const T* s0 = src + (int64_t)y0 * ys + x0;
-        for (uint32_t p = threadIdx.x; p < n; p += kPatchBlock * 8) {   // eight loads in flight
-            T v[8];
-            int at[8];
-#pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                const uint32_t pi = min(p + i * kPatchBlock, n - 1);
-                const uint32_t q = w > 1 ? __umulhi(pi, mul) : pi, c = pi - q * w;
-                at[i] = (int)(q * Q.pitch + c);
-                v[i] = s0[(int64_t)q * ys + c];
-            }
-#pragma unroll
-            for (int i = 0; i < 8; ++i) patch_at<T>(at[i]) = v[i];   // (clamped ones: the same value)
-        }
-        __syncthreads();
-#pragma unroll 1
-        for (int s = 0; s < 4; ++s) {
-            if (B.nd == 1) patch_stage1<T, ACC, K>(B, P, Q, s, out);
-            else if ((int)w >= lh) patch_stage<T, ACC, K, 0>(B, P, Q, s, out);
-            else patch_stage<T, ACC, K, 1>(B, P, Q, s, out);
-            __syncthreads();
-        }
+        T* lds = reinterpret_cast<T*>(patch_lds) + wave * (kMarchLds<T, ACC, K> / (int)sizeof(T));
+        if (B.uniform[0] && B.uniform[1]) rk4_march<T, ACC, K, true>(B, I, lds, parity);
+        else rk4_march<T, ACC, K, false>(B, I, lds, parity);
     }
 }
 
@@ -607,47 +652,28 @@ __global__ __launch_bounds__(kBlock) void k_rk4_back(const BProb* __restrict__ p
     }
 }
 
-template <typename T, int ACC, int K>
-hipError_t launch_march(bool uni, dim3 gr, const BProb* probs, const BItem* it, int n, int parity,
-                        hipStream_t s)
-{
-    if (uni)
-        hipLaunchKernelGGL((k_rk4_march<T, ACC, K, true>), gr, dim3(64), 0, s, probs, it, n, parity);
-    else
-        hipLaunchKernelGGL((k_rk4_march<T, ACC, K, false>), gr, dim3(64), 0, s, probs, it, n, parity);
-    return hipGetLastError();
-}
-
 template <typename T, int ACC>
 hipError_t launch_pass_group(const BGroup& g, const BProb* probs, const BItem* items, int parity,
                              int grid, hipStream_t s)
 {
     const BItem* it = items + g.first;
-    if (g.kind != kItemMarch) {
+    const int units = g.patches + (g.count - g.patches + 3) / 4;
+    if (g.kind == kItemBack) {
         const dim3 gr((unsigned)(g.count < grid ? g.count : grid));
-        if (g.kind == kItemBack) {
-            hipLaunchKernelGGL((k_rk4_back<T>), gr, dim3(kBlock), 0, s, probs, it, g.count);
-            return hipGetLastError();
-        }
-        switch (g.K) {
-#define DOP_RP(KK)                                                                                \
-    case KK:                                                                                      \
-        hipLaunchKernelGGL((k_rk4_patch<T, ACC, KK>), gr, dim3(kPatchBlock), (size_t)g.lds, s, probs, it, \
-                           g.count, parity);                                                      \
+        hipLaunchKernelGGL((k_rk4_back<T>), gr, dim3(kBlock), 0, s, probs, it, g.count);
         return hipGetLastError();
-            DOP_RP(3) DOP_RP(5) DOP_RP(7) DOP_RP(9) DOP_RP(11)
-#undef DOP_RP
-        }
-        return hipErrorInvalidValue;
     }
-    const dim3 gr((unsigned)(g.count / 4 < grid ? g.count : 4 * grid));   // blocks of one wave
-    const bool uni = g.uniform != 0;
+    const dim3 gr((unsigned)(units < grid ? units : grid));
     switch (g.K) {
-    case 3: return launch_march<T, ACC, 3>(uni, gr, probs, it, g.count, parity, s);
-    case 5: return launch_march<T, ACC, 5>(uni, gr, probs, it, g.count, parity, s);
-    case 7: return launch_march<T, ACC, 7>(uni, gr, probs, it, g.count, parity, s);
-    case 9: return launch_march<T, ACC, 9>(uni, gr, probs, it, g.count, parity, s);
-    case 11: return launch_march<T, ACC, 11>(uni, gr, probs, it, g.count, parity, s);
+#define DOP_RP(KK)                                                                                \
+    case KK: {                                                                                    \
+        const int lds = g.count > g.patches ? std::max(g.lds, 4 * kMarchLds<T, ACC, KK>) : g.lds; \
+        hipLaunchKernelGGL((k_rk4_pass<T, ACC, KK>), gr, dim3(kPatchBlock), (size_t)lds, s,       \
+                           probs, it, g.patches, g.count, parity);                                \
+        return hipGetLastError();                                                                 \
+    }
+        DOP_RP(3) DOP_RP(5) DOP_RP(7) DOP_RP(9) DOP_RP(11)
+#undef DOP_RP
     }
     return hipErrorInvalidValue;
 }
