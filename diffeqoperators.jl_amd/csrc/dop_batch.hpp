@@ -64,7 +64,10 @@ constexpr int march_vx(int storage, int accum, int K)
 constexpr int kBackPts = 16384;    // points per item of the copy back
 constexpr int kRimPts = 256;       // shell points per item where shell_point takes them
 constexpr int kPatchLds = 80 << 10;   // bytes of LDS a patch may use, its head included (two a CU)
-constexpr int kPatchHead = 64;         // bytes before a patch's arrays (the stages' regions)
+// Before a patch's arrays: the stages' regions, and per axis its boundary rows (PatchAxis) with the
+// weights of at most kPatchRowsB rows and kPatchW entries in all
+constexpr int kPatchRowsB = 16, kPatchW = 232, kPatchAxis = 192 + 8 * kPatchW;
+constexpr int kPatchHead = 64 + 2 * kPatchAxis;
 
 // A run of items that one launch takes.  An apply's items: one kind, window width K (points:
 // shell_point's) and accumulator.  A pass (kItemPatch): the patches and the marching segments of one window

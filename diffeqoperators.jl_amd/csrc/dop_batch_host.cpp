@@ -154,6 +154,8 @@ void batch_geometry(const DevicePlan& p, int chunk, BProb* B, bool rk4)
             B->fused = B->tiled == 1 && march_box(P, A, B) ? 2 : 1;
             // every patch must fit the LDS (and be there: patches() leaves out none it could make)
             bool fits = true;
+            for (int a = 0; a < P.ndim; ++a)
+                fits = fits && P.ax[a].nb <= kPatchRowsB && P.ax[a].nb * P.ax[a].KB <= kPatchW;
             patch_rects(*B, (int)P.n[0], (int)P.n[1], [&](int x0, int x1, int y0, int y1) {
                 int w, h;
                 if (x1 <= x0 || y1 <= y0) return;

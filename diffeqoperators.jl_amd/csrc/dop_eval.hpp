@@ -422,7 +422,8 @@ DOP_HD inline double shell_point(const PlanDev& P, const T* src, const int64_t* 
 
 // The rows of a line that rows [*lo, *hi) read: their windows, the tiles' window of H on each side
 // included, boundary rows' windows and ghosts (plans that meet shell_point_ok).
-DOP_HD inline void rows_reach(const AxisDev& X, int H, int* lo, int* hi)
+template <typename A>   // (AxisDev, or its n, rlo, rhi, KB)
+DOP_HD inline void rows_reach(const A& X, int H, int* lo, int* hi)
 {
     const int l = *lo, h = *hi, n = X.n;
     const bool left = l < X.rlo, right = h > X.rhi;   // boundary rows among them

@@ -265,6 +265,71 @@ __device__ inline T& patch_at(int i)
     return reinterpret_cast<T*>(patch_lds + kPatchHead)[i];
 }
 
+constexpr int kPatchBlock = 256;   // threads of a patch's block
+
+// The boundary rows of an axis, read once a patch: the rows' weights wait in LDS, where the stages
+// would read them through the plan's tables, load by load, in every one of a block's rows.
+struct PatchAxis {
+    double ga[2][kPointGhost], gc[2];   // ghost coefficients and constant, left and right
+    int ng[2], go[2];                   // ghost taps, first of them
+    int J0[kPatchRowsB], nt[kPatchRowsB];
+    double w[kPatchW];                  // [nb][KB]
+};
+static_assert(sizeof(PatchAxis) == kPatchAxis, "the head's layout");
+
+__device__ inline PatchAxis& patch_axis(int a)
+{
+    return reinterpret_cast<PatchAxis*>(patch_lds + 64)[a];
+}
+
+// what of an axis the patch kernel uses, in scalar registers
+struct PatchDim {
+    int n, rlo, rhi, KB, nb;
+};
+
+__device__ inline void patch_tables(const AxisDev& X, const PatchDim& D, PatchAxis& T)
+{
+    const int t = threadIdx.x;
+    for (int i = t; i < D.nb * D.KB; i += kPatchBlock) T.w[i] = tab(X.bw, i);
+    if (t < D.nb) {
+        T.J0[t] = tab(X.bJ0, t);
+        T.nt[t] = tab(X.bn, t);
+    }
+    if (t >= 64 && t < 66) {
+        const int s = t - 64, n = s ? X.nr : X.nl;
+        const double* al = s ? X.ar : X.al;
+        T.ng[s] = n;
+        T.go[s] = s ? D.n - n : 0;
+        T.gc[s] = s ? tab(&X.br, 0) : tab(&X.bl, 0);
+#pragma unroll
+        for (int k = 0; k < kPointGhost; ++k) T.ga[s][k] = k < n ? tab(al, k) : 0.0;
+    }
+}
+
+// the FP64 sum of boundary row r (shell_point_f's); ld(j): element j of the point's line
+template <int KT, typename F>
+__device__ inline double patch_boundary(const PatchAxis& T, const PatchDim& D, int r, const F& ld)
+{
+    const int side = r < D.rlo ? 0 : 1;
+    const int b = side ? D.rlo + (r - D.rhi) : r;
+    const int ng = T.ng[side], go = T.go[side], jb = T.J0[b] - 1, nt = T.nt[b];
+    double g = 0.0;
+#pragma unroll
+    for (int k = 0; k < kPointGhost; ++k)
+        if (k < ng) g = fma(T.ga[side][k], (double)ld(go + k), g);
+    g = g + T.gc[side];
+    double s = 0.0;
+#pragma unroll
+    for (int k = 0; k < KT; ++k) {
+        if (k < nt) {
+            const int j = jb + k;
+            const double v = (double)ld(min(max(j, 0), D.n - 1));
+            s = fma(T.w[b * D.KB + k], j < 0 || j >= D.n ? g : v, s);
+        }
+    }
+    return s;
+}
+
 // Stage s of a point: k = scale * its row's sum to the stage sum and the next stage's input (own: one
 // of the patch's own points; p its offset in the loaded area, q among the own points).  c is dt / 6
 // for the first and last stage, else dt / 3; h dt for the third stage, else dt / 2.
@@ -316,8 +381,6 @@ __device__ inline X patch_field(const X& f)
     return const_tab(&f, 0);
 }
 
-constexpr int kPatchBlock = 256;   // threads of a patch's block
-
 // Stage s of a patch over the block: lanes along axis L (0: x), rows along the other one.  A wave
 // takes 64 lines along L and a part of the rows.  What a line's row along L needs stays in its
 // registers over the rows: the weights of a regular row (in the tiles' natural box), or a boundary
@@ -326,8 +389,8 @@ constexpr int kPatchBlock = 256;   // threads of a patch's block
 // shell_point_f outside the box (a tap that the tiles' window adds to the row's with weight 0 is
 // taken as 0 there) and as in the tiles inside.
 template <typename T, int ACC, int K, int L>
-__device__ inline void patch_stage(const BProb& B, const PlanDev& P, const Patch& Q, int s,
-                                   T* __restrict__ out)
+__device__ inline void patch_stage(const BProb& B, const PlanDev& P, const Patch& Q,
+                                   const PatchDim* D, int s, T* __restrict__ out)
 {
     using W = typename Acc<ACC>::W;
     constexpr int H = K / 2, M = 1 - L, KT = K + 1;
@@ -350,7 +413,7 @@ __device__ inline void patch_stage(const BProb& B, const PlanDev& P, const Patch
     const W* wlt = patch_field(btabs<ACC>(B)[L]);
     const W* wmt = patch_field(btabs<ACC>(B)[M]);
     const AxisDev &XL = P.ax[L], &XM = P.ax[M];
-    const int nL = patch_field(XL.n), nM = patch_field(XM.n);
+    const int nL = D[L].n, nM = D[M].n;
     // the row's own taps in the window of K
     const int kl0 = H + patch_field(XL.dmin), kl1 = kl0 + patch_field(XL.K);
     const int km0 = H + patch_field(XM.dmin), km1 = km0 + patch_field(XM.K);
@@ -373,7 +436,7 @@ __device__ inline void patch_stage(const BProb& B, const PlanDev& P, const Patch
         int jb = 0, nb = 0, ng = 0, go = 0;
         bool bnd = false;
         if (lin && !lreg) {
-            if (l >= XL.rlo && l < XL.rhi) {
+            if (l >= D[L].rlo && l < D[L].rhi) {
                 const W* wt = Acc<ACC>::table(XL) + (XL.uniform ? 0 : l);
                 const int64_t ws = XL.uniform ? 1 : nL;
                 jb = l + XL.dmin;
@@ -382,22 +445,20 @@ __device__ inline void patch_stage(const BProb& B, const PlanDev& P, const Patch
                 for (int k = 0; k < K; ++k)
                     if (k < nb) wb[k] = (double)tab(wt, k * ws);
             } else {
-                const bool left = l < XL.rlo;
-                const int b = left ? l : XL.rlo + (l - XL.rhi);
-                const double* wr = XL.bw + (int64_t)b * XL.KB;
-                const double* al = left ? XL.al : XL.ar;
+                const PatchAxis& T2 = patch_axis(L);
+                const int side = l < D[L].rlo ? 0 : 1;
+                const int b = side ? D[L].rlo + (l - D[L].rhi) : l;
                 bnd = true;
-                jb = tab(XL.bJ0, b) - 1;
-                nb = tab(XL.bn, b);
-                ng = left ? XL.nl : XL.nr;
-                go = left ? 0 : nL - XL.nr;
-                gc = left ? tab(&XL.bl, 0) : tab(&XL.br, 0);
+                jb = T2.J0[b] - 1;
+                nb = T2.nt[b];
+                ng = T2.ng[side];
+                go = T2.go[side];
+                gc = T2.gc[side];
 #pragma unroll
                 for (int k = 0; k < KT; ++k)
-                    if (k < nb) wb[k] = tab(wr, k);
+                    if (k < nb) wb[k] = T2.w[b * D[L].KB + k];
 #pragma unroll
-                for (int k = 0; k < kPointGhost; ++k)
-                    if (k < ng) ga[k] = tab(al, k);
+                for (int k = 0; k < kPointGhost; ++k) ga[k] = T2.ga[side][k];
             }
         }
         const int mb = m0 + part * per, me = min(mb + per, m1);
@@ -456,7 +517,6 @@ __device__ inline void patch_stage(const BProb& B, const PlanDev& P, const Patch
                 }
             };
             auto along_m = [&]() {
-                const int rlo = patch_field(XM.rlo), rhi = patch_field(XM.rhi);
                 if (mreg) {
                     T t[K];
 #pragma unroll
@@ -470,38 +530,14 @@ __device__ inline void patch_stage(const BProb& B, const PlanDev& P, const Patch
                     }
 #pragma unroll
                     for (int k = 0; k < K; ++k) a.add(wm[k], (W)t[k]);
-                } else if (m >= rlo && m < rhi) {
+                } else if (m >= D[M].rlo && m < D[M].rhi) {
                     const W* wt = patch_field(axis_table<W>(XM)) + (uM ? 0 : m);
                     const int64_t ws = uM ? 1 : nM;
 #pragma unroll
                     for (int k = 0; k < K; ++k)
                         if (k < km1 - km0) a.add(const_tab(wt, k * ws), (W)atm(m + (km0 - H) + k));
                 } else {
-                    const bool left = m < rlo;
-                    const int b = left ? m : rlo + (m - rhi);
-                    const double* wr = patch_field(XM.bw) + (int64_t)b * patch_field(XM.KB);
-                    const int jm = const_tab(patch_field(XM.bJ0), b) - 1;
-                    const int nt = const_tab(patch_field(XM.bn), b);
-                    const int nr = patch_field(XM.nr);
-                    const int n = left ? patch_field(XM.nl) : nr;
-                    const int o = left ? 0 : nM - nr;
-                    double gv = 0.0;
-#pragma unroll
-                    for (int k = 0; k < kPointGhost; ++k)
-                        if (k < n)
-                            gv = fma(left ? patch_field(XM.al[k]) : patch_field(XM.ar[k]),
-                                     (double)atm(o + k), gv);
-                    gv = gv + (left ? patch_field(XM.bl) : patch_field(XM.br));
-                    double sum = 0.0;
-#pragma unroll
-                    for (int k = 0; k < KT; ++k) {
-                        if (k < nt) {
-                            const int j = jm + k;
-                            const double t = (double)atm(min(max(j, 0), nM - 1));
-                            sum = fma(const_tab(wr, k), j < 0 || j >= nM ? gv : t, sum);
-                        }
-                    }
-                    a.add_sum(sum);
+                    a.add_sum(patch_boundary<KT>(patch_axis(M), D[M], m, atm));
                 }
             };
             if (L == 0) along_l(); else along_m();
@@ -516,8 +552,8 @@ __device__ inline void patch_stage(const BProb& B, const PlanDev& P, const Patch
 
 // The same for a 1-D patch: lines of one point
 template <typename T, int ACC, int K>
-__device__ inline void patch_stage1(const BProb& B, const PlanDev& P, const Patch& Q, int s,
-                                    T* __restrict__ out)
+__device__ inline void patch_stage1(const BProb& B, const PlanDev& P, const Patch& Q,
+                                    const PatchDim* D, int s, T* __restrict__ out)
 {
     using W = typename Acc<ACC>::W;
     constexpr int H = K / 2;
@@ -537,9 +573,19 @@ __device__ inline void patch_stage1(const BProb& B, const PlanDev& P, const Patc
                 a.add(wt[(uni ? 0 : (int64_t)x * K) + k], (W)patch_at<T>(in + (p - H + k)));
             v = a.value();
         } else {
-            const int64_t idx[3] = {x, 0, 0};
-            v = shell_point_f<T, ACC, K, 1>(
-                P, idx, [&](int, int j) -> T { return patch_at<T>(in + (j - Q.o0)); });
+            auto ld = [&](int j) { return patch_at<T>(in + (j - Q.o0)); };
+            Acc<ACC> a;
+            if (x >= D[0].rlo && x < D[0].rhi) {
+                const AxisDev& X = P.ax[0];
+                const W* w = Acc<ACC>::table(X) + (X.uniform ? 0 : x);
+                const int64_t ws = X.uniform ? 1 : D[0].n;
+#pragma unroll
+                for (int k = 0; k < K; ++k)
+                    if (k < X.K) a.add(tab(w, k * ws), (W)ld(x + X.dmin + k));
+            } else {
+                a.add_sum(patch_boundary<K + 1>(patch_axis(0), D[0], x, ld));
+            }
+            v = a.value();
         }
         patch_update<T>(Q, s, scale * v, c, h, p, x - Q.a0, x >= Q.a0 && x < b0, out + x);
     }
@@ -553,6 +599,13 @@ __device__ inline void rk4_patch(const BProb& B, const BItem& I, int parity)
     const T* src = (const T*)(parity ? B.acc : B.u);
     T* out = (T*)(parity ? B.u : B.acc);
     int x0 = I.a, x1 = I.b, y0 = I.c, y1 = I.d;
+    const int nd = patch_field(B.nd);
+    PatchDim D[2];
+#pragma unroll
+    for (int a = 0; a < 2; ++a) {
+        const AxisDev& X = P.ax[a];
+        D[a] = {patch_field(X.n), patch_field(X.rlo), patch_field(X.rhi), patch_field(X.KB), patch_field(X.nb)};
+    }
     int* reg = reinterpret_cast<int*>(patch_lds);
 #pragma unroll
     for (int s = 3; s >= 0; --s) {
@@ -562,9 +615,11 @@ __device__ inline void rk4_patch(const BProb& B, const BItem& I, int parity)
             reg[4 * s + 2] = y0;
             reg[4 * s + 3] = y1;
         }
-        rows_reach(P.ax[0], K / 2, &x0, &x1);
-        if (B.nd == 2) rows_reach(P.ax[1], K / 2, &y0, &y1);
+        rows_reach(D[0], K / 2, &x0, &x1);
+        if (nd == 2) rows_reach(D[1], K / 2, &y0, &y1);
     }
+    patch_tables(P.ax[0], D[0], patch_axis(0));
+    if (nd == 2) patch_tables(P.ax[1], D[1], patch_axis(1));
     const int lh = y1 - y0;
     Patch Q;
     Q.o0 = x0;
@@ -596,9 +651,9 @@ __device__ inline void rk4_patch(const BProb& B, const BItem& I, int parity)
     __syncthreads();
 #pragma unroll 1
     for (int s = 0; s < 4; ++s) {
-        if (B.nd == 1) patch_stage1<T, ACC, K>(B, P, Q, s, out);
-        else if ((int)w >= lh) patch_stage<T, ACC, K, 0>(B, P, Q, s, out);
-        else patch_stage<T, ACC, K, 1>(B, P, Q, s, out);
+        if (nd == 1) patch_stage1<T, ACC, K>(B, P, Q, D, s, out);
+        else if ((int)w >= lh) patch_stage<T, ACC, K, 0>(B, P, Q, D, s, out);
+        else patch_stage<T, ACC, K, 1>(B, P, Q, D, s, out);
         __syncthreads();
     }
 }
