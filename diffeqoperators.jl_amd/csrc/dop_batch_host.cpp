@@ -47,6 +47,8 @@ int64_t patch_bytes(const PlanDev& P, int H, int x0, int x1, int y0, int y1)
         rows_reach(P.ax[0], H, &x0, &x1);
         if (P.ndim == 2) rows_reach(P.ax[1], H, &y0, &y1);
     }
+    // (2-D: the block's four waves take at most 256 lines)
+    if (P.ndim == 2 && std::max(x1 - x0, y1 - y0) > 256) return INT64_MAX;
     return kPatchHead + (3 * (int64_t)((x1 - x0) | 1) * (y1 - y0) + own) * (P.storage == kF64 ? 8 : 4);
 }
 

@@ -32,8 +32,8 @@
 // and every sum runs in their order, so the new state is the same bit for bit.  The new state goes
 // to acc, so u and acc swap roles from step to step.
 // Measured against the stage-wise step: 256 mixed f32 problems (1-D to 65536, 2-D to 2048 squared,
-// orders 2 to 8) 2.08 -> 1.09 ms a step, 24 served 2-D requests of 100 steps 36.7 -> 19.3 ms (as two launches
-// a class: 1.30 and 20.6).
+// orders 2 to 8) 2.08 -> 1.04 ms a step, 24 served 2-D requests of 100 steps 36.7 -> 18.0 ms (as two launches
+// a class: 1.30 and 20.6; with the rows' data read in every stage anew: 1.06 and 18.9).
 #pragma once
 #include "dop_batch_impl.hpp"
 
@@ -381,32 +381,29 @@ __device__ inline X patch_field(const X& f)
     return const_tab(&f, 0);
 }
 
-// Stage s of a patch over the block: lanes along axis L (0: x), rows along the other one.  A wave
-// takes 64 lines along L and a part of the rows.  What a line's row along L needs stays in its
-// registers over the rows: the weights of a regular row (in the tiles' natural box), or a boundary
-// row's (and the few regular rows' that lie outside the box) with its ghost's coefficients; a row's
-// along the other axis are the same for the wave, in scalar registers.  Sums run as in
-// shell_point_f outside the box (a tap that the tiles' window adds to the row's with weight 0 is
-// taken as 0 there) and as in the tiles inside.
+// The four stages of a patch over the block: lanes along axis L (0: x), rows along the other one.  A
+// wave takes 64 lines along L (a patch loads at most 256) and a part of the rows.  What a line's
+// row along L needs is read once and stays in its registers: the weights of a regular row (in the
+// tiles' natural box), or a boundary row's (and the few regular rows' that lie outside the box)
+// with its ghost's coefficients; a row's along the other axis are the same for the wave, in scalar
+// registers.  Sums run as in shell_point_f outside the box (a tap that the tiles' window adds to
+// the row's with weight 0 is taken as 0 there) and as in the tiles inside.
 template <typename T, int ACC, int K, int L>
-__device__ inline void patch_stage(const BProb& B, const PlanDev& P, const Patch& Q,
-                                   const PatchDim* D, int s, T* __restrict__ out)
+__device__ inline void patch_run(const BProb& B, const PlanDev& P, const Patch& Q, const PatchDim* D,
+                                 int width, T* __restrict__ out)
 {
     using W = typename Acc<ACC>::W;
-    constexpr int H = K / 2, M = 1 - L, KT = K + 1;
-    const int l0 = patch_region(s, 2 * L), l1 = patch_region(s, 2 * L + 1);
-    const int m0 = patch_region(s, 2 * M), m1 = patch_region(s, 2 * M + 1);
+    constexpr int H = K / 2, M = 1 - L, KT = K + 1, NWV = kPatchBlock / 64;
     const int ol = L == 0 ? Q.o0 : Q.o1, om = L == 0 ? Q.o1 : Q.o0;
     const int b0 = patch_region(3, 1), b1 = patch_region(3, 3);   // the own points' end
-    const int in = (s == 0 ? 0 : s == 2 ? 2 : 1) * Q.sz;
     const double scale = patch_field(B.scale), dt = patch_field(B.dt);
-    const double c = dt / (s == 0 || s == 3 ? 6.0 : 3.0), h = s == 2 ? dt : 0.5 * dt;
     const int64_t ys = patch_field(B.ys);
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int nl = (l1 - ol + 63) >> 6;             // groups of lines (from the patch's origin)
-    const int parts = max(kPatchBlock / 64 / nl, 1);
-    const int per = (m1 - m0 + parts - 1) / parts;
+    const int nl = (width + 63) >> 6;               // groups of lines
+    const int parts = max(NWV / nl, 1);
+    const int g = wave % nl, part = wave / nl;
+    const bool active = part < parts;
     const bool uL = patch_field(B.uniform[L]) != 0, uM = patch_field(B.uniform[M]) != 0;
     const int bl0 = patch_field(B.lo[L]), bl1 = patch_field(B.hi[L]);
     const int bm0 = patch_field(B.lo[M]), bm1 = patch_field(B.hi[M]);
@@ -419,62 +416,70 @@ __device__ inline void patch_stage(const BProb& B, const PlanDev& P, const Patch
     const int km0 = H + patch_field(XM.dmin), km1 = km0 + patch_field(XM.K);
     const bool padl = kl0 > 0 || kl1 < K, padm = km0 > 0 || km1 < K;
     const int sl = L == 0 ? 1 : Q.pitch, sm = L == 0 ? Q.pitch : 1;   // LDS strides
-    for (int unit = wave; unit < nl * parts; unit += kPatchBlock / 64) {
-        const int g = unit % nl, part = unit / nl;
-        const int l = ol + g * 64 + lane;
+    const int l = ol + g * 64 + lane;
+    const bool lreg = l >= bl0 && l < bl1;
+    W wl[K], wm[K];
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+        wl[k] = l < nL && lreg ? wlt[(uL ? 0 : (int64_t)l * K) + k] : W(0);
+        wm[k] = uM ? const_tab(wmt, k) : W(0);
+    }
+    // weights of 64 rows, row wb0 + i in lane i: a scalar load a row would be waited for with the
+    // row's LDS reads
+    W wr[K];
+    int wb0 = om;
+    auto row_weights = [&]() {
+#pragma unroll
+        for (int k = 0; k < K; ++k) wr[k] = wmt[(int64_t)min(wb0 + lane, nM - 1) * K + k];
+    };
+    if (!uM) row_weights();
+    // rows outside the box: weights, first tap, taps, ghost taps
+    double wb[KT] = {}, ga[kPointGhost] = {}, gc = 0.0;
+    int jb = 0, nb = 0, ng = 0, go = 0;
+    bool bnd = false;
+    if (l < nL && !lreg) {
+        if (l >= D[L].rlo && l < D[L].rhi) {
+            const W* wt = Acc<ACC>::table(XL) + (XL.uniform ? 0 : l);
+            const int64_t ws = XL.uniform ? 1 : nL;
+            jb = l + XL.dmin;
+            nb = XL.K;
+#pragma unroll
+            for (int k = 0; k < K; ++k)
+                if (k < nb) wb[k] = (double)tab(wt, k * ws);
+        } else {
+            const PatchAxis& T2 = patch_axis(L);
+            const int side = l < D[L].rlo ? 0 : 1;
+            const int b = side ? D[L].rlo + (l - D[L].rhi) : l;
+            bnd = true;
+            jb = T2.J0[b] - 1;
+            nb = T2.nt[b];
+            ng = T2.ng[side];
+            go = T2.go[side];
+            gc = T2.gc[side];
+#pragma unroll
+            for (int k = 0; k < KT; ++k)
+                if (k < nb) wb[k] = T2.w[b * D[L].KB + k];
+#pragma unroll
+            for (int k = 0; k < kPointGhost; ++k) ga[k] = T2.ga[side][k];
+        }
+    }
+#pragma unroll 1
+    for (int s = 0; s < 4; ++s) {
+        const int l0 = patch_region(s, 2 * L), l1 = patch_region(s, 2 * L + 1);
+        const int m0 = patch_region(s, 2 * M), m1 = patch_region(s, 2 * M + 1);
+        const int in = (s == 0 ? 0 : s == 2 ? 2 : 1) * Q.sz;
+        const double c = dt / (s == 0 || s == 3 ? 6.0 : 3.0), h = s == 2 ? dt : 0.5 * dt;
+        const int per = (m1 - m0 + parts - 1) / parts;
+        const int mb = m0 + part * per, me = active ? min(mb + per, m1) : mb;
         const bool lin = l >= l0 && l < l1;
-        if (__builtin_amdgcn_ballot_w64(lin) == 0) continue;
-        const bool lreg = l >= bl0 && l < bl1;
-        W wl[K], wm[K];
-#pragma unroll
-        for (int k = 0; k < K; ++k) {
-            wl[k] = lin && lreg ? wlt[(uL ? 0 : (int64_t)l * K) + k] : W(0);
-            wm[k] = uM ? const_tab(wmt, k) : W(0);
-        }
-        // rows outside the box: weights, first tap, taps, ghost taps
-        double wb[KT] = {}, ga[kPointGhost] = {}, gc = 0.0;
-        int jb = 0, nb = 0, ng = 0, go = 0;
-        bool bnd = false;
-        if (lin && !lreg) {
-            if (l >= D[L].rlo && l < D[L].rhi) {
-                const W* wt = Acc<ACC>::table(XL) + (XL.uniform ? 0 : l);
-                const int64_t ws = XL.uniform ? 1 : nL;
-                jb = l + XL.dmin;
-                nb = XL.K;
-#pragma unroll
-                for (int k = 0; k < K; ++k)
-                    if (k < nb) wb[k] = (double)tab(wt, k * ws);
-            } else {
-                const PatchAxis& T2 = patch_axis(L);
-                const int side = l < D[L].rlo ? 0 : 1;
-                const int b = side ? D[L].rlo + (l - D[L].rhi) : l;
-                bnd = true;
-                jb = T2.J0[b] - 1;
-                nb = T2.nt[b];
-                ng = T2.ng[side];
-                go = T2.go[side];
-                gc = T2.gc[side];
-#pragma unroll
-                for (int k = 0; k < KT; ++k)
-                    if (k < nb) wb[k] = T2.w[b * D[L].KB + k];
-#pragma unroll
-                for (int k = 0; k < kPointGhost; ++k) ga[k] = T2.ga[side][k];
-            }
-        }
-        const int mb = m0 + part * per, me = min(mb + per, m1);
-        // weights of the rows to come, row mb + i in lane i: a scalar load a row would be waited for
-        // with the row's LDS reads
-        W wr[K];
-        auto row_weights = [&](int m) {
-#pragma unroll
-            for (int k = 0; k < K; ++k) wr[k] = wmt[(int64_t)min(m + lane, nM - 1) * K + k];
-        };
-        if (!uM) row_weights(mb);
         for (int m = mb; m < me; ++m) {
             if (!uM) {
-                if (m > mb && ((m - mb) & 63) == 0) row_weights(m);
+                if (m - wb0 >= 64 || m < wb0) {
+                    wb0 = om + ((m - om) & ~63);
+                    row_weights();
+                }
 #pragma unroll
-                for (int k = 0; k < K; ++k) wm[k] = patch_lane(wr[k], (m - mb) & 63);
+                for (int k = 0; k < K; ++k) wm[k] = patch_lane(wr[k], m - wb0);
             }
             if (!lin) continue;
             const bool mreg = m >= bm0 && m < bm1;   // wave-uniform
@@ -547,6 +552,7 @@ __device__ inline void patch_stage(const BProb& B, const PlanDev& P, const Patch
             patch_update<T>(Q, s, scale * a.value(), c, h, (l - ol) * sl + (m - om) * sm,
                             (y - Q.a1) * Q.ow + (x - Q.a0), own, out + ((int64_t)y * ys + x));
         }
+        __syncthreads();
     }
 }
 
@@ -649,11 +655,14 @@ __device__ inline void rk4_patch(const BProb& B, const BItem& I, int parity)
         for (int i = 0; i < 8; ++i) patch_at<T>(at[i]) = v[i];   // (clamped ones: the same value)
     }
     __syncthreads();
+    if (nd == 2) {
+        if ((int)w >= lh) patch_run<T, ACC, K, 0>(B, P, Q, D, (int)w, out);
+        else patch_run<T, ACC, K, 1>(B, P, Q, D, lh, out);
+        return;
+    }
 #pragma unroll 1
     for (int s = 0; s < 4; ++s) {
-        if (nd == 1) patch_stage1<T, ACC, K>(B, P, Q, D, s, out);
-        else if ((int)w >= lh) patch_stage<T, ACC, K, 0>(B, P, Q, D, s, out);
-        else patch_stage<T, ACC, K, 1>(B, P, Q, D, s, out);
+        patch_stage1<T, ACC, K>(B, P, Q, D, s, out);
         __syncthreads();
     }
 }
