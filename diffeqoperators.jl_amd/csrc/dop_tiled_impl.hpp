@@ -1,7 +1,7 @@
 // dop_tiled_impl.hpp -- tiled interior kernels for 2-D / 3-D Q*u plans, instantiated per
 // storage type by dop_tiled_f64.hip / dop_tiled_f32.hip / dop_tiled_bf16.hip.
 //
-// 2-D: a wave loads an aligned 64*VX-point row segment and marches a chunk of rows.  The K
+// 2-D: a wave loads a 64*VX-point row segment and marches a chunk of rows.  The K
 //      rows of the y stencil live in a register ring of K+PF rows (PF rows prefetched
 //      ahead), so every row of u is loaded once per chunk; the x window of the centre row
 //      comes from neighbouring lanes (DPP), segments overlapping by the x halo.
@@ -13,7 +13,7 @@
 // sequence as the generic path, so the two agree bitwise on finite inputs.
 //
 // The points outside the interior box (the shell) are evaluated by the first blocks of the
-// same launch with the generic per-point path, so they overlap the tiles.
+// same launch point by point (shell_point), so they overlap the tiles.
 //
 // Blocks are dispatched round-robin over the 8 XCDs; with xcd_remap the logical tile of a
 // block is chosen so that each XCD walks a contiguous band of tiles (halo rows of
