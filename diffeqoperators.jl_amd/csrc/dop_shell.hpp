@@ -215,7 +215,16 @@ __device__ inline void xface_tile(const PlanDev& P, const StripArgs& SA, const S
                 wv[k] = tab(wt, k * ws);
                 const int L = self + (X.dmin + k) * step;
 #pragma unroll
-                for (int i = 0; i < kSW; ++i) xv[k][i] = (C)Store<T>::ld(grp[L], min(i + sh, kSW - 1));
+                for (int i = 0; i < kSW; ++i) xv[k][i] = (C)Store<T>::ld(grp[L], i);   // (one LDS read)
+            }
+        }
+        // (block-uniform; 0 but for the last strip of some row lengths)
+#pragma unroll 1
+        for (int s = 0; s < sh; ++s) {
+#pragma unroll
+            for (int k = 0; k < KM; ++k) {
+#pragma unroll
+                for (int i = 0; i + 1 < kSW; ++i) xv[k][i] = xv[k][i + 1];
             }
         }
 #pragma unroll
