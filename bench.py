@@ -490,9 +490,8 @@ def bench_batched(steps, nprob=1024, plain_sample=48, plain_steps=4):
     _sync()
     plain_s = (time.perf_counter() - t0) / plain_steps
     batched_sample_s = step_s * spts / pts   # batched cost of the same points
-    # algorithmic bytes of one RK4 step: stages read/write 3s, 5s, 5s, 3s bytes per point
-    # (stage 0: u -> acc, s1; 1: s1, u, acc -> acc, s2; 2: s2, u, acc -> acc, s1; 3: s1, acc -> u)
-    step_bytes = 16 * 4 * pts
+    # algorithmic bytes of one RK4 step in one pass: u read, the new state written
+    step_bytes = 2 * 4 * pts
     ach = step_bytes / step_s / 1e9
     return dict(
         roofline=dict(bound="hbm", achieved=round(ach, 1), peak=HBM_PEAK_GBS, unit="GB/s",
@@ -545,9 +544,9 @@ def bench_served(nreq=200, lam=2000.0, nsteps=100, budget=8 << 30):
     t = srv.times()
     lat = t[:, 2] - t[:, 0]
     makespan = t[:, 2].max() - t[:, 0].min()
-    # algorithmic bytes: 16 * 4 bytes per point per RK4 step (FP32), over the makespan (which
+    # algorithmic bytes: 2 * 4 bytes per point per RK4 step (FP32), over the makespan (which
     # includes the arrival gaps: a lower bound on the rate while requests are resident)
-    tot_bytes = sum(64.0 * n * n * nsteps for _, n, _, _, _ in reqs)
+    tot_bytes = sum(8.0 * n * n * nsteps for _, n, _, _, _ in reqs)
     ach = tot_bytes / makespan / 1e9
     sizes = np.array([n * n for _, n, _, _, _ in reqs], dtype=np.float64)
     cuts = np.percentile(sizes, [100 / 3, 200 / 3])
