@@ -3,7 +3,7 @@
 // One host thread runs the service loop; any thread may submit, also while it runs:
 //   release   requests whose release time has passed join the FIFO pending queue
 //   admit     the head of the queue is admitted while its state (u + 3 RK4 stage buffers)
-//             fits in the device arena and fewer than max_active requests are resident;
+//             fits in the device arena (dop_arena.hpp) and fewer than max_active are resident;
 //             its initial field is copied in asynchronously
 //   step      resident requests are split into size classes by grid points; each class has
 //             its own stream (the library's side stream of that index, so the classes and the
@@ -25,11 +25,11 @@
 #include <cstdio>
 #include <cstdlib>
 #include <deque>
-#include <map>
 #include <mutex>
 #include <thread>
 #include <vector>
 
+#include "dop_arena.hpp"
 #include "dop_objects.hpp"
 
 namespace {
@@ -38,64 +38,30 @@ using Clock = std::chrono::steady_clock;
 
 constexpr int kMaxInflight = 2;
 constexpr int kTableSlots = kMaxInflight + 2;
-constexpr size_t kAlign = 256;
 // size classes by grid points: up to 256^2, up to 1024^2, larger
 constexpr int kClasses = 3;
 constexpr int64_t kClassPoints[kClasses - 1] = {(int64_t)256 * 256, (int64_t)1024 * 1024};
 
-size_t round_up(size_t n) { return (n + kAlign - 1) / kAlign * kAlign; }
+size_t round_up(size_t n) { return dop::arena_round(n); }
 
-// First-fit allocator over one device allocation, with coalescing of freed blocks.
-class Arena {
-public:
-    void init(char* base, size_t size)
+// Device memory of a server's arena, on the server's device
+struct ArenaMem {
+    int device = 0;
+    ArenaMem() { (void)hipGetDevice(&device); }
+    char* get(size_t n) const
     {
-        base_ = base;
-        free_.clear();
-        free_[0] = size;
-        used_ = 0;
-    }
-    bool alloc(size_t n, size_t* off)
-    {
-        n = round_up(n);
-        for (auto it = free_.begin(); it != free_.end(); ++it) {
-            if (it->second >= n) {
-                *off = it->first;
-                const size_t rest = it->second - n;
-                const size_t at = it->first + n;
-                free_.erase(it);
-                if (rest) free_[at] = rest;
-                used_ += n;
-                return true;
-            }
+        int cur = device;
+        (void)hipGetDevice(&cur);
+        if (cur != device && hipSetDevice(device) != hipSuccess) return nullptr;
+        void* p = nullptr;
+        if (hipMalloc(&p, n) != hipSuccess) {
+            (void)hipGetLastError();   // (a wait for memory, or an error of ours)
+            p = nullptr;
         }
-        return false;
+        if (cur != device) (void)hipSetDevice(cur);
+        return (char*)p;
     }
-    void release(size_t off, size_t n)
-    {
-        n = round_up(n);
-        used_ -= n;
-        auto it = free_.emplace(off, n).first;
-        auto nx = std::next(it);
-        if (nx != free_.end() && it->first + it->second == nx->first) {
-            it->second += nx->second;
-            free_.erase(nx);
-        }
-        if (it != free_.begin()) {
-            auto pv = std::prev(it);
-            if (pv->first + pv->second == it->first) {
-                pv->second += it->second;
-                free_.erase(it);
-            }
-        }
-    }
-    char* ptr(size_t off) const { return base_ + off; }
-    size_t used() const { return used_; }
-
-private:
-    char* base_ = nullptr;
-    std::map<size_t, size_t> free_;
-    size_t used_ = 0;
+    void put(char* p) const { (void)hipFree(p); }
 };
 
 enum State { kScheduled, kPending, kActive, kDraining, kDone, kFailed };
@@ -107,7 +73,8 @@ struct Request {
     const void* u0 = nullptr;
     void* result = nullptr;
     double release = 0, admitted = -1, completed = -1;
-    size_t off = 0, bytes = 0;
+    char* at = nullptr;   // its state in the arena
+    size_t bytes = 0;
     int cls = 0;
     bool fused = false;   // its steps alternate the state between u and acc
     hipEvent_t done_ev = nullptr;
@@ -153,8 +120,7 @@ struct dop_server {
     int chunk = 16;
     int storage = -1;
     hipStream_t stream = nullptr;
-    char* arena_base = nullptr;
-    Arena arena;
+    dop::Arena<ArenaMem> arena;
     std::mutex mu;                 // guards reqs, storage, open, running, t0
     std::deque<Request> reqs;      // stable references: requests are only appended
     bool open = false;             // run() waits for submissions while open
@@ -179,7 +145,6 @@ struct dop_server {
             }
             for (auto& e : c.step_events) (void)hipEventDestroy(e);
         }
-        if (arena_base) (void)hipFree(arena_base);
     }
 };
 
@@ -187,7 +152,7 @@ namespace {
 
 size_t storage_bytes(int storage) { return storage == DOP_F64 ? 8 : storage == DOP_F32 ? 4 : 2; }
 
-// device bytes of a request's state: u and three stage buffers, each rounded to kAlign
+// device bytes of a request's state: u and three stage buffers, each rounded to the arena's blocks
 size_t state_bytes(const dop_plan* plan, int storage)
 {
     return 4 * round_up((size_t)plan->d.host.total * storage_bytes(storage));
@@ -236,10 +201,10 @@ int class_step(dop_server* srv, Class& C, size_t sb, std::vector<Request*>* drai
             B = dop::BProb{};
             dop::batch_geometry(r.plan->d, srv->chunk, &B, true);
             const size_t n = round_up((size_t)r.plan->d.host.total * sb);
-            B.u = srv->arena.ptr(r.off);
-            B.s1 = srv->arena.ptr(r.off + n);
-            B.s2 = srv->arena.ptr(r.off + 2 * n);
-            B.acc = srv->arena.ptr(r.off + 3 * n);
+            B.u = r.at;
+            B.s1 = r.at + n;
+            B.s2 = r.at + 2 * n;
+            B.acc = r.at + 3 * n;
             B.scale = r.scale;
             B.dt = r.dt;
             r.fused = B.fused != 0;
@@ -280,7 +245,7 @@ int class_step(dop_server* srv, Class& C, size_t sb, std::vector<Request*>* drai
             const size_t n = (size_t)r.plan->d.host.total * sb;
             // a fused request's state after an odd number of steps lies in acc
             const size_t at = r.fused && (r.done_steps & 1) ? 3 * round_up(n) : 0;
-            if (hipMemcpyAsync(r.result, srv->arena.ptr(r.off + at), n, hipMemcpyDeviceToHost, C.st) !=
+            if (hipMemcpyAsync(r.result, r.at + at, n, hipMemcpyDeviceToHost, C.st) !=
                 hipSuccess)
                 return dop::set_error(DOP_EHIP, "server: result copy failed");
             (void)hipEventRecord(r.done_ev, C.st);
@@ -311,16 +276,18 @@ int dop_server_create(int64_t hbm_budget_bytes, int max_active, int chunk, void*
         return dop::set_error(DOP_EINVAL, "server: bad budget or slot count");
     *out = nullptr;
     dop_server* s = new dop_server();
-    // the arena holds whole kAlign blocks
-    s->budget = hbm_budget_bytes / (int64_t)kAlign * (int64_t)kAlign;
+    // the arena holds whole blocks
+    s->budget = hbm_budget_bytes / (int64_t)dop::kArenaAlign * (int64_t)dop::kArenaAlign;
     s->max_active = max_active;
     s->chunk = chunk > 0 ? chunk : 16;
     s->stream = (hipStream_t)stream;
-    if (s->budget <= 0 || hipMalloc((void**)&s->arena_base, (size_t)s->budget) != hipSuccess) {
+    // (a budget that is not there is refused now, although the arena takes it as requests come)
+    size_t avail = 0, all = 0;
+    if (s->budget <= 0 || hipMemGetInfo(&avail, &all) != hipSuccess || (size_t)s->budget > avail) {
         delete s;
-        return dop::set_error(DOP_ENOMEM, "server: arena allocation failed");
+        return dop::set_error(DOP_ENOMEM, "server: the device has less free memory than the budget");
     }
-    s->arena.init(s->arena_base, (size_t)s->budget);
+    s->arena.init((size_t)s->budget);
     static_assert(kClasses <= dop::kSideStreams, "a side stream per class");
     for (int k = 0; k < kClasses; ++k) {
         Class& c = s->cls[k];
@@ -440,16 +407,21 @@ int dop_server_run(dop_server* srv)
         scheduled.erase(scheduled.begin(), scheduled.begin() + nrel);
         if (ndone == nreq && !open) break;
         const size_t sb = storage_bytes(storage < 0 ? DOP_F32 : storage);
-        // admit (FIFO)
+        // admit (FIFO); what the arena may need for the requests that are waiting: their sum
+        auto waiting = [&]() {
+            size_t n = 0;
+            for (const Request* r : pending) n += r->bytes;
+            for (const Request* r : scheduled) n += r->bytes;
+            return n;
+        };
         while (!pending.empty() && nactive < srv->max_active) {
             Request& r = *pending.front();
-            size_t off;
-            if (!srv->arena.alloc(r.bytes, &off)) {
+            r.at = srv->arena.alloc(r.bytes, waiting);
+            if (!r.at) {
                 if (nactive == 0 && draining.empty())
-                    rc = dop::set_error(DOP_EBUDGET, "server: a request does not fit the empty arena");
+                    rc = dop::set_error(DOP_ENOMEM, "server: no device memory for a request");
                 break;
             }
-            r.off = off;
             r.admitted = now();
             r.state = kActive;
             Class& C = srv->cls[r.cls];
@@ -458,7 +430,7 @@ int dop_server_run(dop_server* srv)
             C.dirty = true;
             ++nactive;
             pending.pop_front();
-            if (hipMemcpyAsync(srv->arena.ptr(off), r.u0, n, hipMemcpyHostToDevice, C.st) != hipSuccess) {
+            if (hipMemcpyAsync(r.at, r.u0, n, hipMemcpyHostToDevice, C.st) != hipSuccess) {
                 rc = dop::set_error(DOP_EHIP, "server: initial-field copy failed");
                 break;
             }
@@ -485,7 +457,7 @@ int dop_server_run(dop_server* srv)
             if (hipEventQuery(r.done_ev) == hipSuccess) {
                 r.completed = now();
                 r.state = kDone;
-                srv->arena.release(r.off, r.bytes);
+                srv->arena.release(r.at, r.bytes);
                 draining.erase(draining.begin() + k);
                 ++ndone;
             } else {
@@ -508,14 +480,14 @@ int dop_server_run(dop_server* srv)
         // give back the arena blocks of everything resident; those requests failed
         for (auto& C : srv->cls) {
             for (Request* r : C.active) {
-                srv->arena.release(r->off, r->bytes);
+                srv->arena.release(r->at, r->bytes);
                 r->state = kFailed;
             }
             C.active.clear();
             C.dirty = true;
         }
         for (Request* r : draining) {
-            srv->arena.release(r->off, r->bytes);
+            srv->arena.release(r->at, r->bytes);
             r->state = kFailed;
         }
     }

@@ -235,7 +235,7 @@ void dop_rk4_destroy(dop_rk4* rk);
  * scale, step dt, number of RK4 steps, an initial field and a result buffer in pinned host
  * memory, and a release time (seconds after dop_server_run starts).  dop_server_run
  * releases requests at their times, admits released requests in FIFO order while their state
- * (u and three RK4 stage buffers, carved from one device arena of `hbm_budget_bytes` rounded
+ * (u and three RK4 stage buffers, carved from an arena of `hbm_budget_bytes` rounded
  * down to 256 bytes) fits and fewer than `max_active` are resident, and advances the resident
  * requests by RK4 steps: they are split into size classes by grid points (up to 256^2, up to
  * 1024^2, larger), each class on a stream of its own advancing all its requests one step per
@@ -248,6 +248,10 @@ void dop_rk4_destroy(dop_rk4* rk);
  * is not open (dop_server_set_open(srv, 1) keeps it waiting for submissions until it is set
  * to 0).  A request whose state alone exceeds the budget is refused at submission
  * (DOP_EBUDGET); on an error the run stops and the resident requests' memory is returned.
+ * The arena takes device memory as requests come, up to the budget, and holds it until
+ * dop_server_destroy; dop_server_create refuses a budget larger than the device's free memory
+ * (DOP_ENOMEM), and dop_server_run fails with DOP_ENOMEM when a request finds none although
+ * nothing is resident.
  * `stream` is unused (the classes run on the library's three side streams of the device, the
  * ones the second half of a 3-D apply also uses, synchronized before dop_server_run returns:
  * with the caller's stream they fill HIP's default four hardware queues, so no class waits

@@ -4,6 +4,7 @@
 // can be compared with the FP64 oracle without a GPU.  Never part of libdop.so.
 #include <algorithm>
 #include <cstdint>
+#include <map>
 #include <string>
 #include <vector>
 
@@ -384,5 +385,92 @@ int hc_rk4_items(const dop_desc* d, int* bad, int64_t* info)
     for (int64_t p = 0; p < (int64_t)cover.size(); ++p)
         if (cover[p] != 1) return fail(1, p % n0, p / n0, cover[p], 0);
     return B.fused;
+}
+}  // extern "C"
+
+// ---------------------------------------------------------------------------------------
+// The server's arena over host memory of a given size: random requests and releases.
+#include <random>
+
+#include "../../diffeqoperators.jl_amd/csrc/dop_arena.hpp"
+
+namespace {
+struct FakeMem {
+    static size_t limit, given, most;   // bytes that the "device" has, holds, has held at most
+    static std::map<char*, size_t> held;
+    static char* next;
+    char* get(size_t n)
+    {
+        if (given + n > limit) return nullptr;
+        char* p = next;   // (addresses only: nothing is written)
+        next += n + 4096;
+        held[p] = n;
+        given += n;
+        most = std::max(most, given);
+        return p;
+    }
+    void put(char* p)
+    {
+        given -= held.at(p);
+        held.erase(p);
+    }
+};
+size_t FakeMem::limit, FakeMem::given, FakeMem::most;
+std::map<char*, size_t> FakeMem::held;
+char* FakeMem::next = reinterpret_cast<char*>(1 << 20);
+}  // namespace
+
+extern "C" {
+// 0, or the first rule that fails: 1 a block outside what is held, 2 blocks that overlap, 3 more
+// than the budget held, 4 a request that fits the empty arena (and the memory) refused, 5 memory
+// held after the end, 6 used() wrong.  *most: bytes held at most.
+int hc_arena(int64_t budget, int64_t limit, int64_t ahead, int steps, int seed, int64_t* most)
+{
+    FakeMem::limit = (size_t)limit;
+    FakeMem::given = FakeMem::most = 0;
+    FakeMem::held.clear();
+    std::mt19937_64 rng((unsigned)seed);
+    int bad = 0;
+    {
+        dop::Arena<FakeMem> A;
+        A.init((size_t)budget);
+        std::vector<std::pair<char*, size_t>> live;
+        size_t used = 0;
+        for (int i = 0; i < steps && !bad; ++i) {
+            if (rng() % 50 == 0)   // drain
+                while (!live.empty()) {
+                    A.release(live.back().first, live.back().second);
+                    used -= dop::arena_round(live.back().second);
+                    live.pop_back();
+                }
+            if (!live.empty() && rng() % 2) {
+                std::swap(live[rng() % live.size()], live.back());
+                A.release(live.back().first, live.back().second);
+                used -= dop::arena_round(live.back().second);
+                live.pop_back();
+            } else {
+                // sizes over three decades, up to the whole budget
+                const size_t top = (size_t)budget >> (rng() % 10);
+                const size_t n = std::max<size_t>(top / 2 + rng() % (top / 2 + 1), 1);
+                char* p = A.alloc(n, [&]() { return (size_t)ahead; });
+                if (!p) {
+                    if (live.empty() && dop::arena_round(n) <= (size_t)std::min(budget, limit)) bad = 4;
+                } else {
+                    const size_t r = dop::arena_round(n);
+                    auto it = FakeMem::held.upper_bound(p);
+                    if (it == FakeMem::held.begin() || p + r > std::prev(it)->first + std::prev(it)->second) bad = 1;
+                    for (auto& q : live)
+                        if (p < q.first + dop::arena_round(q.second) && q.first < p + r) bad = 2;
+                    live.emplace_back(p, n);
+                    used += r;
+                }
+            }
+            if (FakeMem::given > (size_t)budget || A.total() != FakeMem::given) bad = 3;
+            if (A.used() != used) bad = 6;
+        }
+    }
+    if (!bad && FakeMem::given) bad = 5;
+    *most = (int64_t)FakeMem::most;
+    return bad;
 }
 }  // extern "C"
