@@ -65,6 +65,66 @@ struct PlanImage {
     }
 };
 
+// Plans that only a destroyed graph held.  Its callback may not call HIP, so the next creation or
+// destruction of a plan frees them (never destroyed: graphs may go at the process' end).
+std::mutex& left_mu()
+{
+    static std::mutex* m = new std::mutex;
+    return *m;
+}
+std::vector<dop_plan*>& left_plans()
+{
+    static auto* v = new std::vector<dop_plan*>;
+    return *v;
+}
+void plan_left(void* p)
+{
+    dop_plan* plan = (dop_plan*)p;
+    if (--plan->refs > 0) return;
+    std::lock_guard<std::mutex> lk(left_mu());
+    left_plans().push_back(plan);
+}
+void free_left_plans()
+{
+    std::vector<dop_plan*> v;
+    {
+        std::lock_guard<std::mutex> lk(left_mu());
+        v.swap(left_plans());
+    }
+    for (dop_plan* p : v) delete p;
+}
+
+// A plan's image on the device.  While a stream is being captured a copy on the default stream would
+// end the capture, so the copy takes a stream of its own, and the thread's capture mode is relaxed
+// around what captures refuse otherwise: what is done here is no part of the graph, and is
+// complete on return.
+hipError_t upload_image(dop_plan* p, PlanImage& img, bool capturing)
+{
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    hipError_t e = hipSuccess;
+    if (capturing && (e = hipThreadExchangeStreamCaptureMode(&mode)) != hipSuccess) return e;
+    if ((e = hipMalloc((void**)&p->dev, img.bytes.size())) != hipSuccess) p->dev = nullptr;
+    if (e == hipSuccess) {
+        for (const auto& q : img.ptrs) *q.first = (const char*)p->dev + q.second;
+        std::memcpy(img.bytes.data(), &p->d.host, sizeof(dop::PlanDev));
+        if (!capturing) {
+            e = hipMemcpy(p->dev, img.bytes.data(), img.bytes.size(), hipMemcpyHostToDevice);
+        } else {
+            hipStream_t s = nullptr;
+            e = hipStreamCreateWithFlags(&s, hipStreamNonBlocking);
+            if (e == hipSuccess)
+                e = hipMemcpyAsync(p->dev, img.bytes.data(), img.bytes.size(), hipMemcpyHostToDevice, s);
+            if (s) {
+                const hipError_t w = hipStreamSynchronize(s);
+                if (e == hipSuccess) e = w;
+                (void)hipStreamDestroy(s);
+            }
+        }
+    }
+    if (capturing) (void)hipThreadExchangeStreamCaptureMode(&mode);
+    return e;
+}
+
 size_t storage_bytes(int storage)
 {
     return storage == DOP_F64 ? 8 : storage == DOP_F32 ? 4 : 2;
@@ -201,7 +261,10 @@ int dop_version(void) { return DOP_ABI_VERSION; }
 
 const char* dop_last_error(void) { return g_err.c_str(); }
 
-int dop_plan_create(const dop_desc* desc, dop_plan** out)
+}  // extern "C"
+
+namespace {
+int create_plan(const dop_desc* desc, bool capturing, dop_plan** out)
 {
     if (!desc || !out) return fail(DOP_EINVAL, "null argument");
     *out = nullptr;
@@ -251,23 +314,75 @@ int dop_plan_create(const dop_desc* desc, dop_plan** out)
         img.table(T.bw, &X.bw);
         img.table(T.lbc, &X.lbc);
     }
-    if (hipMalloc((void**)&p->dev, img.bytes.size()) != hipSuccess) {
-        p->dev = nullptr;
+    const hipError_t e = upload_image(p, img, capturing);
+    if (e != hipSuccess) {
+        const bool mem = p->dev == nullptr;
         delete p;
-        return fail(DOP_ENOMEM, "hipMalloc of plan failed");
-    }
-    for (const auto& q : img.ptrs) *q.first = (const char*)p->dev + q.second;
-    std::memcpy(img.bytes.data(), &p->d.host, sizeof(dop::PlanDev));
-    if (hipMemcpy(p->dev, img.bytes.data(), img.bytes.size(), hipMemcpyHostToDevice) != hipSuccess) {
-        delete p;
-        return fail(DOP_EHIP, "upload of plan failed");
+        return mem ? fail(DOP_ENOMEM, "hipMalloc of plan failed") : fail(DOP_EHIP, "upload of plan failed");
     }
     p->d.dev = p->dev;
     *out = p;
     return DOP_OK;
 }
+}  // namespace
 
-void dop_plan_destroy(dop_plan* plan) { delete plan; }
+extern "C" {
+
+int dop_plan_create(const dop_desc* desc, dop_plan** out)
+{
+    free_left_plans();
+    return create_plan(desc, false, out);
+}
+
+int dop_plan_create_capturing(const dop_desc* desc, void* stream, dop_plan** out)
+{
+    const int rc = create_plan(desc, true, out);
+    if (rc != DOP_OK) return rc;
+    const int held = dop_plan_hold(*out, stream);
+    if (held == DOP_OK) return DOP_OK;
+    delete *out;
+    *out = nullptr;
+    return held;
+}
+
+int dop_capturing(void* stream)
+{
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    return stream && hipStreamIsCapturing((hipStream_t)stream, &st) == hipSuccess &&
+           st == hipStreamCaptureStatusActive;
+}
+
+int dop_plan_hold(dop_plan* plan, void* stream)
+{
+    if (!plan) return fail(DOP_EINVAL, "null plan");
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    unsigned long long id = 0;
+    hipGraph_t graph = nullptr;
+    const hipGraphNode_t* deps = nullptr;
+    size_t ndeps = 0;
+    DOP_HIP(hipStreamGetCaptureInfo_v2((hipStream_t)stream, &st, &id, &graph, &deps, &ndeps));
+    if (st != hipStreamCaptureStatusActive || !graph)
+        return fail(DOP_EINVAL, "dop_plan_hold: the stream is not being captured");
+    std::lock_guard<std::mutex> lk(plan->hold_mu);
+    if (plan->held == id) return DOP_OK;
+    hipUserObject_t obj = nullptr;
+    DOP_HIP(hipUserObjectCreate(&obj, plan, plan_left, 1, hipUserObjectNoDestructorSync));
+    ++plan->refs;
+    // (on failure the release's callback gives the reference back)
+    const hipError_t e = hipGraphRetainUserObject(graph, obj, 1, hipGraphUserObjectMove);
+    if (e != hipSuccess) {
+        (void)hipUserObjectRelease(obj, 1);
+        return fail(DOP_EHIP, std::string("hipGraphRetainUserObject: ") + hipGetErrorString(e));
+    }
+    plan->held = id;
+    return DOP_OK;
+}
+
+void dop_plan_destroy(dop_plan* plan)
+{
+    if (plan && --plan->refs == 0) delete plan;
+    free_left_plans();
+}
 
 int64_t dop_plan_input_elems(const dop_plan* plan) { return plan ? plan->in_elems : -1; }
 int64_t dop_plan_output_elems(const dop_plan* plan) { return plan ? plan->out_elems : -1; }

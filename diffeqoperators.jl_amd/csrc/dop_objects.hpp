@@ -25,6 +25,9 @@ struct dop_plan {
     std::mutex tune_mu;           // one tuning at a time
     int64_t in_elems = 0, out_elems = 0;
     int device = 0;
+    std::atomic<int> refs{1};     // the caller's handle, and the captured graphs that hold the plan
+    std::mutex hold_mu;           // guards held
+    unsigned long long held = 0;  // the last capture whose graph holds it
     ~dop_plan()
     {
         if (dev) (void)hipFree(dev);

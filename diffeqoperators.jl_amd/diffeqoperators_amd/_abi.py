@@ -81,6 +81,9 @@ def lib():
     L.dop_plan_create.argtypes = [C.POINTER(DopDesc), C.POINTER(vp)]
     L.dop_plan_destroy.argtypes = [vp]
     L.dop_plan_destroy.restype = None
+    L.dop_plan_hold.argtypes = [vp, vp]
+    L.dop_plan_create_capturing.argtypes = [C.POINTER(DopDesc), vp, C.POINTER(vp)]
+    L.dop_capturing.argtypes = [vp]
     L.dop_plan_input_elems.argtypes = [vp]
     L.dop_plan_input_elems.restype = C.c_int64
     L.dop_plan_output_elems.argtypes = [vp]

@@ -11,7 +11,6 @@ import ctypes as C
 import itertools
 import os
 import threading
-import weakref
 
 import torch
 
@@ -48,10 +47,15 @@ def julia_size(t: torch.Tensor):
 class Plan:
     """An immutable libdop plan (dop_plan_create)."""
 
-    def __init__(self, desc: _abi.DopDesc, keep):
+    def __init__(self, desc: _abi.DopDesc, keep, capturing=None):
+        """capturing: the raw stream that is being captured, whose graph then holds the plan."""
         self._keep = keep
         h = C.c_void_p()
-        _abi.check(_abi.lib().dop_plan_create(C.byref(desc), C.byref(h)), "dop_plan_create")
+        if capturing is None:
+            _abi.check(_abi.lib().dop_plan_create(C.byref(desc), C.byref(h)), "dop_plan_create")
+        else:
+            _abi.check(_abi.lib().dop_plan_create_capturing(C.byref(desc), C.c_void_p(capturing),
+                                                            C.byref(h)), "dop_plan_create_capturing")
         self.handle = h
         self.storage = desc.storage
         self.in_elems = _abi.lib().dop_plan_input_elems(h)
@@ -309,6 +313,8 @@ def _bc_structure(bc):
 # operators of one structure used in turn a table rebuild and upload per call: 460 us on the
 # 4096^2 FP64 Laplacian whose apply takes 50, 10 ms on a 1-D line of 2^18 points.)  The pool holds
 # at most _POOL_MAX sets, the oldest dropped first, and is guarded by a lock.
+# Plans that a captured graph reads keep their values: they are never handed on, and the graph
+# holds them (dop_plan_hold), so a replay does not depend on the owner or on what was applied since.
 _POOL = {}           # number -> (structure, plans, stream they were last applied on)
 _POOL_MAX = 64
 _POOL_LOCK = threading.RLock()
@@ -318,27 +324,28 @@ _MIXED = object()    # applied on several streams
 
 class _Bound:
     """The plans of one owner for one kind of array, the descriptors of its values, and the
-    stream the plans have been applied on (None: not yet; _MIXED: several)."""
+    stream the plans have been applied on (None: not yet; _MIXED: several).  updated: the plans came
+    from the pool, so their values were set on that stream.  graph: the plans that graphs read (the
+    same ones, or others made in a capture)."""
 
-    __slots__ = ("skey", "descs", "plans", "stream", "__weakref__")
+    __slots__ = ("skey", "descs", "plans", "stream", "updated", "graph", "__weakref__")
 
     def __init__(self, skey, descs):
         self.skey, self.descs, self.plans, self.stream = skey, descs, None, None
+        self.updated, self.graph = False, None
 
     def __del__(self):
         # plans applied on several streams are not reused: an update on one of them would not
         # wait for applies still queued on another
         try:
-            if self.plans is not None and self.stream is not None and self.stream is not _MIXED:
+            if (self.plans is not None and self.plans is not self.graph and self.stream is not None
+                    and self.stream is not _MIXED):
                 with _POOL_LOCK:
                     _POOL[next(_POOL_COUNT)] = (self.skey, self.plans, self.stream)
                     while len(_POOL) > _POOL_MAX:
                         _POOL.pop(next(iter(_POOL)))
         except Exception:   # interpreter shutdown
             pass
-
-
-_LIVE = weakref.WeakSet()
 
 
 def ghost_plans(owner, terms, u: torch.Tensor, accum=_abi.ACC_AUTO):
@@ -369,48 +376,62 @@ def _ghost_descs(terms, u, accum):
     return out
 
 
-def _take_pooled(skey, stream, any_stream):
+def _take_pooled(skey, stream):
     for k, (s, plans, st) in list(_POOL.items())[::-1]:
-        if s == skey and (any_stream or st == stream) and _POOL.pop(k, None) is not None:
+        if s == skey and st == stream and _POOL.pop(k, None) is not None:
             return plans
     return None
 
 
-def _bind(owner, key, u, accum, bound, stream):
+def _bound_of(owner, key, u, accum):
+    """The owner's _Bound for arrays like u (under the lock)."""
+    bound = _plan_cache(owner).get(key)
+    if bound is None:
+        descs = _ghost_descs(_ghost_terms(owner), u, accum)
+        # plans are created with the kernel selection the environment asks for
+        skey = (julia_size(u), u.dtype, accum, u.device.index,
+                os.environ.get("DOP_FORCE_GENERIC"), os.environ.get("DOP_TILE_VARIANT"),
+                tuple(d[2] for d in descs))
+        bound = _plan_cache(owner)[key] = _Bound(skey, descs)
+    return bound
+
+
+def _bind(owner, key, u, accum, stream):
     """The owner's _Bound for arrays like u, with plans holding its values."""
     with _POOL_LOCK, torch.cuda.device(u.device):
-        if bound is None:
-            bound = _plan_cache(owner).get(key)
-        if bound is None:
-            descs = _ghost_descs(_ghost_terms(owner), u, accum)
-            # plans are created with the kernel selection the environment asks for
-            skey = (julia_size(u), u.dtype, accum, u.device.index,
-                    os.environ.get("DOP_FORCE_GENERIC"), os.environ.get("DOP_TILE_VARIANT"),
-                    tuple(d[2] for d in descs))
-            bound = _Bound(skey, descs)
+        bound = _bound_of(owner, key, u, accum)
         if bound.plans is None:
-            # a stream being captured admits neither allocations nor new plans: there the plans
-            # of any owner of this structure are taken (a live one then gets others on its next use)
-            capturing = torch.cuda.is_current_stream_capturing()
-            plans = _take_pooled(bound.skey, stream, capturing)
-            if plans is None and capturing:
-                other = next((b for b in _LIVE if b.skey == bound.skey and b.plans is not None), None)
-                if other is not None:
-                    plans, other.plans, other.stream = other.plans, None, None
+            plans = bound.graph
             if plans is None:
-                plans = [Plan(d, keep) for d, keep, _ in bound.descs]
-            else:
-                for i, (d, keep, _) in enumerate(bound.descs):
-                    try:
-                        plans[i].update(d, keep, stream)
-                    except _abi.DopError:
-                        # same kinds and sizes but a different row structure (e.g. coefficients
-                        # that are no longer uniform): a plan of its own
-                        plans[i] = Plan(d, keep)
+                plans = _take_pooled(bound.skey, stream)
+                if plans is None:
+                    plans = [Plan(d, keep) for d, keep, _ in bound.descs]
+                else:
+                    for i, (d, keep, _) in enumerate(bound.descs):
+                        try:
+                            plans[i].update(d, keep, stream)
+                        except _abi.DopError:
+                            # same kinds and sizes but a different row structure (e.g. coefficients
+                            # that are no longer uniform): a plan of its own
+                            plans[i] = Plan(d, keep)
+                    bound.updated = True
             bound.plans, bound.stream = plans, stream
-        _plan_cache(owner)[key] = bound
-        _LIVE.add(bound)
     return bound
+
+
+def _graph_plans(owner, key, u, accum, stream):
+    """The owner's plans for the graph that is being captured on `stream`, which holds them: its
+    plans if their values have been there since they were made, else plans made now."""
+    with _POOL_LOCK, torch.cuda.device(u.device):
+        bound = _bound_of(owner, key, u, accum)
+        if bound.graph is None:
+            if bound.plans is not None and not bound.updated:
+                bound.graph = bound.plans
+            else:
+                bound.graph = [Plan(d, keep, stream) for d, keep, _ in bound.descs]
+        for p in bound.graph:
+            _abi.check(_abi.lib().dop_plan_hold(p.handle, C.c_void_p(stream)), "dop_plan_hold")
+        return bound.graph
 
 
 _raw_stream = torch._C._cuda_getCurrentRawStream if hasattr(
@@ -427,14 +448,18 @@ def _apply_bound(owner, du, u, accum=_abi.ACC_AUTO, accumulate=False):
     dev = u.device
     stream = _raw_stream(dev.index)
     key = (u.shape, u.dtype, dev, accum)
-    bound = owner._plans.get(key)
-    plans = None if bound is None else bound.plans
-    if plans is None:
-        bound = _bind(owner, key, u, accum, bound, stream)
-        plans = bound.plans
-    elif bound.stream != stream:
-        bound.stream = _MIXED
-    apply = _abi.lib().dop_apply
+    lib = _abi.lib()
+    if stream and lib.dop_capturing(stream):   # (the default stream cannot be captured)
+        plans = _graph_plans(owner, key, u, accum, stream)
+    else:
+        bound = owner._plans.get(key)
+        plans = None if bound is None else bound.plans
+        if plans is None:
+            bound = _bind(owner, key, u, accum, stream)
+            plans = bound.plans
+        elif bound.stream != stream:
+            bound.stream = _MIXED
+    apply = lib.dop_apply
     for p in plans:
         rc = apply(p.handle, dp, up, 1 if accumulate else 0, stream)
         if rc:

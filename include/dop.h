@@ -162,6 +162,16 @@ const char* dop_last_error(void);
 int dop_plan_create(const dop_desc* desc, dop_plan** out);
 void dop_plan_destroy(dop_plan* plan);
 
+/* Plans in captured graphs.  A graph reads its plans' device memory at every replay:
+ * dop_plan_hold makes the graph that is being captured on `stream` hold the plan, so that
+ * dop_plan_destroy frees it only once that graph and every executable made from it are gone (the
+ * caller must not dop_plan_update it meanwhile).  dop_plan_create_capturing creates a plan
+ * while `stream` is being captured, where dop_plan_create would end the capture, and lets its
+ * graph hold it.  dop_capturing: whether `stream` is being captured. */
+int dop_plan_hold(dop_plan* plan, void* stream);
+int dop_plan_create_capturing(const dop_desc* desc, void* stream, dop_plan** out);
+int dop_capturing(void* stream);
+
 /* New values for an existing plan, in place: the BCs' taps and constants (also per line) and
  * the operators' tables and coefficients of `desc`, which must describe the same structure as
  * the descriptor the plan was created from (ndim, sizes, storage, accumulation, input kind,
