@@ -348,8 +348,12 @@ int dop_plan_create_capturing(const dop_desc* desc, void* stream, dop_plan** out
 int dop_capturing(void* stream)
 {
     hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-    return stream && hipStreamIsCapturing((hipStream_t)stream, &st) == hipSuccess &&
-           st == hipStreamCaptureStatusActive;
+    if (!stream) return 0;   // (the default stream cannot be captured)
+    if (hipStreamIsCapturing((hipStream_t)stream, &st) != hipSuccess) {
+        (void)hipGetLastError();   // (the next launch's check must not find it)
+        return 0;
+    }
+    return st == hipStreamCaptureStatusActive;
 }
 
 int dop_plan_hold(dop_plan* plan, void* stream)

@@ -315,33 +315,32 @@ def _bc_structure(bc):
 # at most _POOL_MAX sets, the oldest dropped first, and is guarded by a lock.
 # Plans that a captured graph reads keep their values: they are never handed on, and the graph
 # holds them (dop_plan_hold), so a replay does not depend on the owner or on what was applied since.
-_POOL = {}           # number -> (structure, plans, stream they were last applied on)
+_POOL = {}           # number -> (structure, plans, the stream they were applied on)
 _POOL_MAX = 64
 _POOL_LOCK = threading.RLock()
 _POOL_COUNT = itertools.count()
-_MIXED = object()    # applied on several streams
 
 
 class _Bound:
     """The plans of one owner for one kind of array, the descriptors of its values, and the
-    stream the plans have been applied on (None: not yet; _MIXED: several).  updated: the plans came
-    from the pool, so their values were set on that stream.  graph: the plans that graphs read (the
-    same ones, or others made in a capture)."""
+    streams that they have been applied on.  updated: the stream that set the values of plans from
+    the pool, which others wait for before their first apply (None: plans made for the owner,
+    complete from the start).  graph: the plans that graphs read (the same ones, or others made in
+    a capture)."""
 
-    __slots__ = ("skey", "descs", "plans", "stream", "updated", "graph", "__weakref__")
+    __slots__ = ("skey", "descs", "plans", "streams", "updated", "graph", "__weakref__")
 
     def __init__(self, skey, descs):
-        self.skey, self.descs, self.plans, self.stream = skey, descs, None, None
-        self.updated, self.graph = False, None
+        self.skey, self.descs, self.plans, self.streams = skey, descs, None, set()
+        self.updated, self.graph = None, None
 
     def __del__(self):
         # plans applied on several streams are not reused: an update on one of them would not
         # wait for applies still queued on another
         try:
-            if (self.plans is not None and self.plans is not self.graph and self.stream is not None
-                    and self.stream is not _MIXED):
+            if self.plans is not None and self.plans is not self.graph and len(self.streams) == 1:
                 with _POOL_LOCK:
-                    _POOL[next(_POOL_COUNT)] = (self.skey, self.plans, self.stream)
+                    _POOL[next(_POOL_COUNT)] = (self.skey, self.plans, *self.streams)
                     while len(_POOL) > _POOL_MAX:
                         _POOL.pop(next(iter(_POOL)))
         except Exception:   # interpreter shutdown
@@ -383,6 +382,21 @@ def _take_pooled(skey, stream):
     return None
 
 
+def _wait_for(stream):
+    """The current stream waits for what is queued on the raw `stream`; False where it cannot (a
+    stream that is being captured now, or is gone).  Only an owner's first apply on a second stream
+    comes here: an event at every update cost a temporary owner's apply 7 us of 48."""
+    if _abi.lib().dop_capturing(stream):
+        return False
+    try:
+        event = torch.cuda.Event()
+        event.record(torch.cuda.ExternalStream(stream))
+        torch.cuda.current_stream().wait_event(event)
+    except RuntimeError:
+        return False
+    return True
+
+
 def _bound_of(owner, key, u, accum):
     """The owner's _Bound for arrays like u (under the lock)."""
     bound = _plan_cache(owner).get(key)
@@ -397,7 +411,8 @@ def _bound_of(owner, key, u, accum):
 
 
 def _bind(owner, key, u, accum, stream):
-    """The owner's _Bound for arrays like u, with plans holding its values."""
+    """The owner's _Bound for arrays like u, with plans holding its values on `stream`, u's
+    current one."""
     with _POOL_LOCK, torch.cuda.device(u.device):
         bound = _bound_of(owner, key, u, accum)
         if bound.plans is None:
@@ -414,8 +429,12 @@ def _bind(owner, key, u, accum, stream):
                             # same kinds and sizes but a different row structure (e.g. coefficients
                             # that are no longer uniform): a plan of its own
                             plans[i] = Plan(d, keep)
-                    bound.updated = True
-            bound.plans, bound.stream = plans, stream
+                    bound.updated = stream
+            bound.plans = plans
+        elif bound.updated is not None and stream not in bound.streams and not _wait_for(bound.updated):
+            bound.plans = [Plan(d, keep) for d, keep, _ in bound.descs]
+            bound.updated = None
+        bound.streams.add(stream)
     return bound
 
 
@@ -425,7 +444,7 @@ def _graph_plans(owner, key, u, accum, stream):
     with _POOL_LOCK, torch.cuda.device(u.device):
         bound = _bound_of(owner, key, u, accum)
         if bound.graph is None:
-            if bound.plans is not None and not bound.updated:
+            if bound.plans is not None and bound.updated is None:
                 bound.graph = bound.plans
             else:
                 bound.graph = [Plan(d, keep, stream) for d, keep, _ in bound.descs]
@@ -453,12 +472,9 @@ def _apply_bound(owner, du, u, accum=_abi.ACC_AUTO, accumulate=False):
         plans = _graph_plans(owner, key, u, accum, stream)
     else:
         bound = owner._plans.get(key)
-        plans = None if bound is None else bound.plans
-        if plans is None:
+        if bound is None or stream not in bound.streams:
             bound = _bind(owner, key, u, accum, stream)
-            plans = bound.plans
-        elif bound.stream != stream:
-            bound.stream = _MIXED
+        plans = bound.plans
     apply = lib.dop_apply
     for p in plans:
         rc = apply(p.handle, dp, up, 1 if accumulate else 0, stream)
