@@ -84,6 +84,21 @@ void plan_left(void* p)
     std::lock_guard<std::mutex> lk(left_mu());
     left_plans().push_back(plan);
 }
+
+// The thread's capture mode, relaxed around what a capture refuses otherwise and would end with: an
+// allocation, a free, another stream's work.  What is done within is no part of a graph.
+struct RelaxedCapture {
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    const bool on;
+    RelaxedCapture() : on(hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess) {}
+    ~RelaxedCapture()
+    {
+        if (on) (void)hipThreadExchangeStreamCaptureMode(&mode);
+    }
+    RelaxedCapture(const RelaxedCapture&) = delete;
+    RelaxedCapture& operator=(const RelaxedCapture&) = delete;
+};
+
 void free_left_plans()
 {
     std::vector<dop_plan*> v;
@@ -91,18 +106,17 @@ void free_left_plans()
         std::lock_guard<std::mutex> lk(left_mu());
         v.swap(left_plans());
     }
+    if (v.empty()) return;
+    RelaxedCapture relaxed;
     for (dop_plan* p : v) delete p;
 }
 
 // A plan's image on the device.  While a stream is being captured a copy on the default stream would
-// end the capture, so the copy takes a stream of its own, and the thread's capture mode is relaxed
-// around what captures refuse otherwise: what is done here is no part of the graph, and is
-// complete on return.
+// end the capture, so the copy takes a stream of its own; it is complete on return.
 hipError_t upload_image(dop_plan* p, PlanImage& img, bool capturing)
 {
-    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    RelaxedCapture relaxed;
     hipError_t e = hipSuccess;
-    if (capturing && (e = hipThreadExchangeStreamCaptureMode(&mode)) != hipSuccess) return e;
     if ((e = hipMalloc((void**)&p->dev, img.bytes.size())) != hipSuccess) p->dev = nullptr;
     if (e == hipSuccess) {
         for (const auto& q : img.ptrs) *q.first = (const char*)p->dev + q.second;
@@ -121,7 +135,6 @@ hipError_t upload_image(dop_plan* p, PlanImage& img, bool capturing)
             }
         }
     }
-    if (capturing) (void)hipThreadExchangeStreamCaptureMode(&mode);
     return e;
 }
 
@@ -384,7 +397,11 @@ int dop_plan_hold(dop_plan* plan, void* stream)
 
 void dop_plan_destroy(dop_plan* plan)
 {
-    if (plan && --plan->refs == 0) delete plan;
+    // (an owner may go at any time, also while a stream is being captured)
+    if (plan && --plan->refs == 0) {
+        RelaxedCapture relaxed;
+        delete plan;
+    }
     free_left_plans();
 }
 

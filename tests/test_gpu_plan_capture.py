@@ -131,3 +131,24 @@ def test_plans_are_given_back_with_the_graph():
         cycle()
     torch.cuda.synchronize()
     assert before - torch.cuda.mem_get_info()[0] < 32 << 20
+
+
+def test_plans_freed_in_a_capture():
+    # plans of owners that go while a stream is being captured, and plans that earlier graphs have
+    # left: freeing them neither ends the capture nor becomes part of it
+    u, out = field(7), torch.empty(N, dtype=torch.float64, device="cuda")
+    for k in range(4):
+        held = [D.plans_for(owner(0.3 + i), u) for i in range(3)]
+        a = owner(9.0 + k)
+        gone = captured(lambda: D.mul_(out, owner(0.7), u))
+
+        def work():
+            gone.reset()
+            held.clear()
+            gc.collect()
+            D.mul_(out, a, u)
+        g = captured(work)
+        for _ in range(3):
+            out.zero_()
+            g.replay()
+            assert torch.equal(out, fresh(9.0 + k, u))
