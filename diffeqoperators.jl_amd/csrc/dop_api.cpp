@@ -334,6 +334,7 @@ int create_plan(const dop_desc* desc, bool capturing, dop_plan** out)
         return mem ? fail(DOP_ENOMEM, "hipMalloc of plan failed") : fail(DOP_EHIP, "upload of plan failed");
     }
     p->d.dev = p->dev;
+    p->bytes = (int64_t)img.bytes.size();
     *out = p;
     return DOP_OK;
 }
@@ -405,6 +406,7 @@ void dop_plan_destroy(dop_plan* plan)
     free_left_plans();
 }
 
+int64_t dop_plan_device_bytes(const dop_plan* plan) { return plan ? plan->bytes : -1; }
 int64_t dop_plan_input_elems(const dop_plan* plan) { return plan ? plan->in_elems : -1; }
 int64_t dop_plan_output_elems(const dop_plan* plan) { return plan ? plan->out_elems : -1; }
 

@@ -24,6 +24,7 @@ struct dop_plan {
     std::atomic<int> tuned{0};    // variant chosen by the autotuner (or the tuning cache)
     std::mutex tune_mu;           // one tuning at a time
     int64_t in_elems = 0, out_elems = 0;
+    int64_t bytes = 0;            // of dev
     int device = 0;
     std::atomic<int> refs{1};     // the caller's handle, and the captured graphs that hold the plan
     std::mutex hold_mu;           // guards held

@@ -84,6 +84,8 @@ def lib():
     L.dop_plan_hold.argtypes = [vp, vp]
     L.dop_plan_create_capturing.argtypes = [C.POINTER(DopDesc), vp, C.POINTER(vp)]
     L.dop_capturing.argtypes = [vp]
+    L.dop_plan_device_bytes.argtypes = [vp]
+    L.dop_plan_device_bytes.restype = C.c_int64
     L.dop_plan_input_elems.argtypes = [vp]
     L.dop_plan_input_elems.restype = C.c_int64
     L.dop_plan_output_elems.argtypes = [vp]

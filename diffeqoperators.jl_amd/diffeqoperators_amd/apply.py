@@ -7,8 +7,8 @@ contiguous device tensors (float64, float32 or bfloat16); there is no CPU path.
 """
 from __future__ import annotations
 
+import collections
 import ctypes as C
-import itertools
 import os
 import threading
 
@@ -58,6 +58,7 @@ class Plan:
                                                             C.byref(h)), "dop_plan_create_capturing")
         self.handle = h
         self.storage = desc.storage
+        self.device_bytes = _abi.lib().dop_plan_device_bytes(h)
         self.in_elems = _abi.lib().dop_plan_input_elems(h)
         self.out_elems = _abi.lib().dop_plan_output_elems(h)
         self.desc = desc
@@ -312,13 +313,49 @@ def _bc_structure(bc):
 # other's values.  (One plan per structure, rebound to whichever owner was applied last, cost two
 # operators of one structure used in turn a table rebuild and upload per call: 460 us on the
 # 4096^2 FP64 Laplacian whose apply takes 50, 10 ms on a 1-D line of 2^18 points.)  The pool holds
-# at most _POOL_MAX sets, the oldest dropped first, and is guarded by a lock.
+# at most _POOL_MAX sets and, beside the newest, _POOL_BYTES of device memory (tables of long
+# non-uniform lines take hundreds of MB a plan); the oldest are dropped first.  A lock guards it,
+# and every step of a search leaves it whole: an owner may go, and leave its plans, in any of them.
 # Plans that a captured graph reads keep their values: they are never handed on, and the graph
 # holds them (dop_plan_hold), so a replay does not depend on the owner or on what was applied since.
-_POOL = {}           # number -> (structure, plans, the stream they were applied on)
+_POOL = collections.deque()   # (structure, plans, the stream they were applied on, bytes), oldest first
 _POOL_MAX = 64
+_POOL_BYTES = 256 << 20
 _POOL_LOCK = threading.RLock()
-_POOL_COUNT = itertools.count()
+_pool_held = 0                # bytes of the sets in the pool
+
+
+def _pool_put(skey, plans, stream):
+    global _pool_held
+    nbytes = sum(p.device_bytes for p in plans)
+    with _POOL_LOCK:
+        _POOL.append((skey, plans, stream, nbytes))
+        _pool_held += nbytes
+        _pool_trim()
+
+
+def _pool_trim():
+    global _pool_held
+    while len(_POOL) > 1 and (len(_POOL) > _POOL_MAX or _pool_held > _POOL_BYTES):
+        old = _POOL.popleft()
+        _pool_held -= old[3]
+
+
+def _pool_take(skey, stream):
+    """The newest set of the structure that was applied on the stream, or None."""
+    global _pool_held
+    newer, found = 0, None        # sets moved to the old end, newest first
+    for _ in range(len(_POOL)):
+        e = _POOL.pop()
+        if e[0] == skey and e[2] == stream:
+            _pool_held -= e[3]
+            found = e[1]
+            break
+        _POOL.appendleft(e)
+        newer += 1
+    _POOL.rotate(-newer)
+    _pool_trim()
+    return found
 
 
 class _Bound:
@@ -339,10 +376,7 @@ class _Bound:
         # wait for applies still queued on another
         try:
             if self.plans is not None and self.plans is not self.graph and len(self.streams) == 1:
-                with _POOL_LOCK:
-                    _POOL[next(_POOL_COUNT)] = (self.skey, self.plans, *self.streams)
-                    while len(_POOL) > _POOL_MAX:
-                        _POOL.pop(next(iter(_POOL)))
+                _pool_put(self.skey, self.plans, *self.streams)
         except Exception:   # interpreter shutdown
             pass
 
@@ -373,13 +407,6 @@ def _ghost_descs(terms, u, accum):
         out.append((d, keep + [bcs], (sem, tuple(_op_structure(L) for L in ops),
                                       tuple(sorted((ax, _bc_structure(bc)) for ax, bc in bcs.items())))))
     return out
-
-
-def _take_pooled(skey, stream):
-    for k, (s, plans, st) in list(_POOL.items())[::-1]:
-        if s == skey and st == stream and _POOL.pop(k, None) is not None:
-            return plans
-    return None
 
 
 def _wait_for(stream):
@@ -418,7 +445,7 @@ def _bind(owner, key, u, accum, stream):
         if bound.plans is None:
             plans = bound.graph
             if plans is None:
-                plans = _take_pooled(bound.skey, stream)
+                plans = _pool_take(bound.skey, stream)
                 if plans is None:
                     plans = [Plan(d, keep) for d, keep, _ in bound.descs]
                 else:

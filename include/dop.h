@@ -187,6 +187,9 @@ int dop_capturing(void* stream);
  * so their later launches see the update. */
 int dop_plan_update(dop_plan* plan, const dop_desc* desc, void* stream);
 
+/* Device memory that a plan holds, in bytes. */
+int64_t dop_plan_device_bytes(const dop_plan* plan);
+
 /* Number of bytes of u and du the plan reads/writes per dop_apply (storage elements). */
 int64_t dop_plan_input_elems(const dop_plan* plan);
 int64_t dop_plan_output_elems(const dop_plan* plan);

@@ -32,7 +32,7 @@ def fresh(g, u):
 
 
 def pooled():
-    return [e for e in ap._POOL.values() if e[0][0] == (N,)]
+    return [e for e in list(ap._POOL) if e[0][0] == (N,)]
 
 
 def test_other_streams_wait_for_a_pooled_plans_values():
