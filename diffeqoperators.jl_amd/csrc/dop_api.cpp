@@ -437,14 +437,24 @@ int dop_apply_set(int n, const dop_plan* const* plans, void* const* du, const vo
         if (!plans[i] || !du[i] || !u[i]) return fail(DOP_EINVAL, "null plan or buffer");
         if (du[i] == u[i]) return fail(DOP_EINVAL, "du must not alias u");
     }
-    // (plans that tune themselves have tiles, and those go one by one)
-    bool tiles = n > 8;
+    // One by one: plans that tune themselves (they have tiles), and terms whose output another term
+    // reads or writes a part of (an output that terms share, whole, is one of launch_apply_set's)
+    auto meet = [](const void* a, int64_t na, const void* b, int64_t nb) {
+        return (uintptr_t)a < (uintptr_t)b + (uintptr_t)nb && (uintptr_t)b < (uintptr_t)a + (uintptr_t)na;
+    };
+    bool ordered = n > 8;
     const dop::DevicePlan* p[8] = {};
-    for (int i = 0; i < n && !tiles; ++i) {
+    for (int i = 0; i < n && !ordered; ++i) {
         p[i] = &plans[i]->d;
-        tiles = dop::apply_variants(plans[i]->d) > 1;
+        ordered = dop::apply_variants(plans[i]->d) > 1;
+        const int64_t out = plans[i]->out_elems * (int64_t)storage_bytes(plans[i]->d.host.storage);
+        for (int j = 0; j < n && !ordered; ++j) {
+            const int64_t sb = (int64_t)storage_bytes(plans[j]->d.host.storage);
+            ordered = meet(du[i], out, u[j], plans[j]->in_elems * sb) ||
+                      (du[j] != du[i] && meet(du[i], out, du[j], plans[j]->out_elems * sb));
+        }
     }
-    if (!tiles) {
+    if (!ordered) {
         DOP_HIP(dop::launch_apply_set(n, p, du, u, accumulate, (hipStream_t)stream));
         return DOP_OK;
     }
