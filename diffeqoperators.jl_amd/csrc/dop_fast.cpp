@@ -104,9 +104,7 @@ bool build_strips(const PlanDev& P, const HostPlan& H, const int32_t* lo, const 
     const AxisDev& X0 = P.ax[0];
     // items start at multiples of 4 along x and load groups of four values (element-aligned, so
     // the rows may have any length; the last item of a ragged row is narrower)
-    S.vec_ok = lo[0] % kStripPts != 0 || hi[0] % kStripPts != 0 || n[0] < kStripStage ? kVecNone
-               : n[0] % kStripPts                                                    ? kVecRagged
-                                                                                     : kVecWhole;
+    S.vec_ok = lo[0] % kStripPts == 0 && hi[0] % kStripPts == 0 && n[0] >= kStripStage ? 1 : 0;
     S.stage_ok = strips_stage_ok(P, H.axis[0], lo[0], hi[0]) ? 1 : 0;
     // x strips of four regular rows
     const int32_t ax = (X0.rlo + kStripPts - 1) / kStripPts * kStripPts;
@@ -344,24 +342,11 @@ bool fast_variant(const FastPlan& fp, int v, FastArgs* out)
     return true;
 }
 
-bool fast_candidate(const FastPlan& fp, int v)
-{
-    // 3-D chunks of 16 planes read K - 1 more for each 16, 16 % more than chunks of 32 (K = 7), for
-    // more blocks: where chunks of 32 give every CU four they only win the tuner's short runs (512^3
-    // f32: 321 us against 326 there, 337 against 333 in an application's loop).
-    FastArgs A;
-    if (fp.kind != 3 || !fast_variant(fp, v, &A) || A.chunk > 16) return true;
-    return (int64_t)A.nxseg * A.nyblk * ceil_div(A.hi[2] - A.lo[2], 32) < 4 * 256;
-}
-
 int fast_default(const FastPlan& fp)
 {
     if (fp.kind < 2) return 0;
     // the order of preference with plenty of points; the first that gives every CU two blocks
-    // (four waves of a 2-D block, eight of a 3-D one) is taken, else the one of most blocks.
-    // us by chunk, longest first: 512^2 f32 14.8 / 8.7 / 7.0 / 6.9, 1000 x 3000 16.6 / 10.1 / 8.4 /
-    // 8.4 (64, 32, 16, 8 rows; none there has 512 blocks); 128^3 f32 40.3 / 37.9 / 37.4, 203 x 190 x
-    // 177 f32 47.8 / 47.1 / 48.5 and f64 57.7 / 61.1 / 60.4
+    // (four waves of a 2-D block, eight of a 3-D one) is taken, else the one of most blocks
     static const int v2[4] = {4, 0, 2, 6};                    // 2-D chunks 64, 32, 16, 8
     static const int w3[3] = {0, 6, 7};                       // 3-D (8,2)x32, (8,2)x16, (8,1)x16
     const bool half = fp.kind == 3 && fp.VX > 1 && fp.args.hi[0] - fp.args.lo[0] <= 32 * fp.VX;

@@ -41,16 +41,12 @@ struct ShellSeg {
     int32_t items;   // work items per row (general: strips of the box)
     int32_t first;   // first block (in the order the XCDs take them)
 };
-// Whether strips load whole groups of 4 values (items start at multiples of 4 along x): never; but for
-// a group that would leave its row; always (rows of whole groups).
-enum StripVec : int32_t { kVecNone = 0, kVecRagged = 1, kVecWhole = 2 };
-
 struct StripArgs {
     int32_t nseg;
     int32_t nblocks;                 // blocks of the launch
     int32_t nfirst;                  // blocks of the leading kind-4 segments (taken in hardware
                                      // order; the rest XCD-contiguous)
-    int32_t vec_ok;                  // StripVec
+    int32_t vec_ok;                  // items start at multiples of 4 along x (groups of 4 values)
     int32_t stage_ok;                // every x tap and ghost of a strip touching x boundary rows
                                      // lies in the kStripStage values at its end of the line
     ShellSeg seg[kMaxShellSegs];
@@ -124,8 +120,6 @@ void build_fast(const HostPlan& H, FastPlan* fp);
 // not a valid variant.
 bool fast_variant(const FastPlan& fp, int v, FastArgs* out);
 int fast_variant_count(const FastPlan& fp);
-// Whether the tuner tries variant v.
-bool fast_candidate(const FastPlan& fp, int v);
 // The variant of a plan that is not tuned (fewer than 2^20 points, or before its first apply).
 int fast_default(const FastPlan& fp);
 

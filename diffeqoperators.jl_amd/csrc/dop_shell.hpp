@@ -146,7 +146,7 @@ __device__ inline int64_t strip_block(int i, int nb)
 // the tile and its kXfHalo-line border (the y and z taps) into LDS; then each thread evaluates
 // its points with the generic arithmetic: x term per point (row programs uniform over the
 // block), y and z terms as regular rows (the plan's own windows) from LDS.
-template <typename T, int ACC, int KM, int VEC>
+template <typename T, int ACC, int KM>
 __device__ inline void xface_tile(const PlanDev& P, const StripArgs& SA, const ShellSeg& G, int tile,
                                   T (*full)[kStage + 1], T (*grp)[kSW], T* __restrict__ du,
                                   const T* __restrict__ src, int accumulate)
@@ -169,8 +169,7 @@ __device__ inline void xface_tile(const PlanDev& P, const StripArgs& SA, const S
     const int x0 = G.r0;
     const int w = min(kSW, G.xend - x0);
     const int g0 = x0 < n0 / 2 ? 0 : n0 - kStage;
-    // the strip's group, kept in the row
-    const int xl = VEC == kVecWhole ? x0 : min(x0, n0 - kSW), sh = VEC == kVecWhole ? 0 : x0 - xl;
+    const int xl = min(x0, n0 - kSW), sh = x0 - xl;   // the strip's group, kept in the row
     const int64_t s1 = P.ssrc[1], s2 = P.ssrc[2];
     const int64_t xb = P.tshift[0] + g0;
     // the strip's group of every line of the tile and border
@@ -243,7 +242,7 @@ __device__ inline void xface_tile(const PlanDev& P, const StripArgs& SA, const S
     strip::store_item<T, ACC, LD>(P, idx, w, sh == 0, acc, du, accumulate);
 }
 
-template <typename T, int ACC, int KM, int VEC>
+template <typename T, int ACC, int KM, bool VEC>
 __global__ __launch_bounds__(kShellBlock) void k_shell_strips(const PlanDev* __restrict__ Pp,
                                                              const StripArgs SA,
                                                              T* __restrict__ du,
@@ -267,11 +266,11 @@ __global__ __launch_bounds__(kShellBlock) void k_shell_strips(const PlanDev* __r
     const int nr = SA.seg[s].nr;
     const int j = rb % nr;
     const int l = (rb / nr) * kShellBlock + (int)threadIdx.x;
-    if constexpr (VEC != kVecNone && KM / 2 <= kXfHalo) {
+    if constexpr (VEC && KM / 2 <= kXfHalo) {
         if (SA.seg[s].kind == 4) {
             // one tile of lines per block (the block-wide branch precedes the block barrier)
             if (rb >= SA.seg[s].items / kShellBlock) return;
-            xface_tile<T, ACC, KM, VEC>(*Pp, SA, SA.seg[s], rb, stage, xgrp, du, src, accumulate);
+            xface_tile<T, ACC, KM>(*Pp, SA, SA.seg[s], rb, stage, xgrp, du, src, accumulate);
             return;
         }
     }

@@ -375,9 +375,9 @@ DOP_HD inline void store_item(const PlanDev& P, const int64_t* idx, int w, bool 
 // kStage values and `slots` kSW accumulators of this thread (LDS on the device); LD loads up
 // to kSW consecutive values.  KM >= the window of every regular row (the tiles' window).  VEC:
 // SA.vec_ok (items start at multiples of 4, so whole groups are loaded, also for items of fewer
-// than 4 points; where rows end in part of a group, 1, unless the group would leave the row).
-// Plans with ghost-point input only (the tiled path's condition).
-template <typename T, int ACC, int KM, int VEC, typename LD>
+// than 4 points, unless the group would leave the row).  Plans with ghost-point input only (the
+// tiled path's condition).
+template <typename T, int ACC, int KM, bool VEC, typename LD>
 DOP_HD inline void eval_strip(const PlanDev& P, const StripArgs& SA, int b, int l, T* stage,
                               Slot<ACC>* slots, T* __restrict__ du, const T* __restrict__ src,
                               int accumulate)
@@ -399,7 +399,7 @@ DOP_HD inline void eval_strip(const PlanDev& P, const StripArgs& SA, int b, int 
     }
     const int64_t wl = SA.org[b][0] + SA.ext[b][0] - idx[0];
     const int w = wl < kSW ? (int)wl : kSW;
-    const bool vec = VEC == kVecWhole || (VEC == kVecRagged && idx[0] + kSW <= P.n[0]);
+    const bool vec = VEC && idx[0] + kSW <= P.n[0];   // a whole group lies in the row
     Acc<ACC> acc[kSW];
 
     // x term
@@ -441,7 +441,7 @@ DOP_HD inline void eval_strip(const PlanDev& P, const StripArgs& SA, int b, int 
 // starts at x0 = row and ends before xend): the other two axes are regular rows at every point,
 // the row along A is the same for the whole block.  The host builds face segments only when
 // SA.vec_ok, n0 >= 16, the A axis has one BC for all lines and (kind 0) SA.stage_ok.
-template <typename T, int ACC, int KM, int A, int VEC, typename LD>
+template <typename T, int ACC, int KM, int A, typename LD>
 DOP_HD inline void eval_face(const PlanDev& P, const StripArgs& SA, int row, int xend, int l, T* stage,
                              Slot<ACC>* slots, T* __restrict__ du, const T* __restrict__ src,
                              int accumulate)
@@ -464,7 +464,7 @@ DOP_HD inline void eval_face(const PlanDev& P, const StripArgs& SA, int row, int
         idx[2] = SA.flo[0][1] + v;
         w = xend - row < kSW ? xend - row : kSW;
     }
-    const bool vec = A != 0 || VEC == kVecWhole || row + kSW <= (int)P.n[0];
+    const bool vec = A != 0 || row + kSW <= (int)P.n[0];   // a whole group lies in the row
     Acc<ACC> acc[kSW];
     const AxisDev& X0 = P.ax[0];
     const AxisDev& X1 = P.ax[1];
@@ -489,7 +489,7 @@ DOP_HD inline void eval_face(const PlanDev& P, const StripArgs& SA, int row, int
 }
 
 // Work item `l` of row j of segment `s`: the kernel's (and the CPU check's) dispatch.
-template <typename T, int ACC, int KM, int VEC, typename LD>
+template <typename T, int ACC, int KM, bool VEC, typename LD>
 DOP_HD inline void eval_item(const PlanDev& P, const StripArgs& SA, int s, int j, int l, T* stage,
                              Slot<ACC>* slots, T* __restrict__ du, const T* __restrict__ src,
                              int accumulate)
@@ -500,14 +500,14 @@ DOP_HD inline void eval_item(const PlanDev& P, const StripArgs& SA, int s, int j
         eval_strip<T, ACC, KM, VEC, LD>(P, SA, G.r0, l, stage, slots, du, src, accumulate);
         return;
     }
-    if constexpr (VEC != kVecNone) {
+    if constexpr (VEC) {
         if (G.kind == 2)
-            eval_face<T, ACC, KM, 2, VEC, LD>(P, SA, G.r0 + j, 0, l, stage, slots, du, src, accumulate);
+            eval_face<T, ACC, KM, 2, LD>(P, SA, G.r0 + j, 0, l, stage, slots, du, src, accumulate);
         else if (G.kind == 1)
-            eval_face<T, ACC, KM, 1, VEC, LD>(P, SA, G.r0 + j, 0, l, stage, slots, du, src, accumulate);
+            eval_face<T, ACC, KM, 1, LD>(P, SA, G.r0 + j, 0, l, stage, slots, du, src, accumulate);
         else
-            eval_face<T, ACC, KM, 0, VEC, LD>(P, SA, G.r0 + j * kSW, G.xend, l, stage, slots, du, src,
-                                              accumulate);
+            eval_face<T, ACC, KM, 0, LD>(P, SA, G.r0 + j * kSW, G.xend, l, stage, slots, du, src,
+                                         accumulate);
     }
 }
 

@@ -905,16 +905,14 @@ hipError_t launch_shell3d(const DevicePlan& p, void* du, const void* u, int accu
         if (fp.kind == 3 && fp.strips.nblocks > 0) {
             const dim3 sg((unsigned)fp.strips.nblocks);
             const StripArgs& SA = fp.strips;
-#define DOP_STRIPS(VEC)                                                                      \
-    hipLaunchKernelGGL((shell::k_shell_strips<T, ACC, K, VEC>), sg, dim3(shell::kShellBlock), 0, \
-                       s2, p.dev, SA, (T*)du, (const T*)u, accumulate)
-            // Rows of whole groups: no test per item, which beside the tiles made the 512^3 bf16 apply
-            // 270 us (268 without; f32 333.4 and 334.5).  FP64 groups are two loads each and take the
-            // tested form, 0.6 % faster there (602 us, 605).
-            if (sizeof(T) < 8 && SA.vec_ok == kVecWhole) DOP_STRIPS(kVecWhole);
-            else if (SA.vec_ok != kVecNone) DOP_STRIPS(kVecRagged);
-            else DOP_STRIPS(kVecNone);
-#undef DOP_STRIPS
+            if (SA.vec_ok)
+                hipLaunchKernelGGL((shell::k_shell_strips<T, ACC, K, true>), sg,
+                                   dim3(shell::kShellBlock), 0, s2, p.dev, SA, (T*)du, (const T*)u,
+                                   accumulate);
+            else
+                hipLaunchKernelGGL((shell::k_shell_strips<T, ACC, K, false>), sg,
+                                   dim3(shell::kShellBlock), 0, s2, p.dev, SA, (T*)du, (const T*)u,
+                                   accumulate);
             const hipError_t e = hipGetLastError();
             if (e != hipSuccess) return e;
         }

@@ -96,8 +96,8 @@ int hc_apply(const dop_desc* d, void* du, const void* u, int accumulate)
 }
 
 namespace {
-template <typename T, int ACC, int KM, int VEC>
-void run_shell_v(const dop::PlanDev& P, const dop::StripArgs& S, T* du, const T* src, int accumulate)
+template <typename T, int ACC, int KM>
+void run_shell_k(const dop::PlanDev& P, const dop::StripArgs& S, T* du, const T* src, int accumulate)
 {
     T stage[dop::strip::kStage + 1];
     dop::strip::Slot<ACC> slots[dop::strip::kSW];
@@ -106,25 +106,21 @@ void run_shell_v(const dop::PlanDev& P, const dop::StripArgs& S, T* du, const T*
         if (G.kind == 4) {
             // the device marches these x-face points along z; the same points as face items
             for (int l = 0; l < S.fn[0][0] * S.fn[0][1]; ++l)
-                dop::strip::eval_face<T, ACC, KM, 0, VEC, dop::strip::ScalarLoad<T>>(P, S, G.r0, G.xend, l, stage,
-                                                                                    slots, du, src, accumulate);
+                dop::strip::eval_face<T, ACC, KM, 0, dop::strip::ScalarLoad<T>>(P, S, G.r0, G.xend, l, stage, slots,
+                                                                               du, src, accumulate);
             continue;
         }
         for (int j = 0; j < G.nr; ++j) {
             for (int l = 0; l < G.items; ++l) {
-                dop::strip::eval_item<T, ACC, KM, VEC, dop::strip::ScalarLoad<T>>(P, S, s, j, l, stage, slots, du,
-                                                                                 src, accumulate);
+                if (S.vec_ok)
+                    dop::strip::eval_item<T, ACC, KM, true, dop::strip::ScalarLoad<T>>(P, S, s, j, l, stage, slots,
+                                                                                     du, src, accumulate);
+                else
+                    dop::strip::eval_item<T, ACC, KM, false, dop::strip::ScalarLoad<T>>(P, S, s, j, l, stage,
+                                                                                      slots, du, src, accumulate);
             }
         }
     }
-}
-
-template <typename T, int ACC, int KM>
-void run_shell_k(const dop::PlanDev& P, const dop::StripArgs& S, T* du, const T* src, int accumulate)
-{
-    if (S.vec_ok == dop::kVecWhole) run_shell_v<T, ACC, KM, dop::kVecWhole>(P, S, du, src, accumulate);
-    else if (S.vec_ok == dop::kVecRagged) run_shell_v<T, ACC, KM, dop::kVecRagged>(P, S, du, src, accumulate);
-    else run_shell_v<T, ACC, KM, dop::kVecNone>(P, S, du, src, accumulate);
 }
 
 // the tiles' window K (3, 5, 7 or 9) as the strips' compile-time width, as the launch does
@@ -476,23 +472,5 @@ int hc_arena(int64_t budget, int64_t limit, int64_t ahead, int steps, int seed, 
     if (!bad && FakeMem::given) bad = 5;
     *most = (int64_t)FakeMem::most;
     return bad;
-}
-}  // extern "C"
-
-extern "C" {
-// A tile-shape candidate of the plan: whether the tuner tries it, and its chunk and points per lane;
-// -1 when there is no such candidate.
-int hc_candidate(const dop_desc* d, int v, int* chunk, int* rows, int* vx)
-{
-    dop::HostPlan H;
-    if (dop::build_host_plan(*d, &H, &g_err) != DOP_OK) return -1;
-    dop::FastPlan F;
-    dop::build_fast(H, &F);
-    dop::FastArgs A;
-    if (!dop::fast_variant(F, v, &A)) return -1;
-    *chunk = A.chunk;
-    *rows = A.W * A.VY;
-    *vx = A.VX;
-    return dop::fast_candidate(F, v) ? 1 : 0;
 }
 }  // extern "C"
