@@ -215,7 +215,8 @@ int tune_variants(dop_plan* p, void* du, const void* u, hipStream_t s, int* choi
     std::vector<float> per(nv, 1e30f);
     std::vector<char> okv(nv, 1);
     for (int v = 0; v < nv; ++v)   // warm-up (code objects, caches)
-        okv[v] = dop::launch_apply(p->d, du, u, 0, v, 0, s) == hipSuccess;
+        okv[v] = dop::fast_candidate(p->d.fast, v) &&
+                 dop::launch_apply(p->d, du, u, 0, v, 0, s) == hipSuccess;
     // launches per measurement: enough for about 1 ms of back-to-back work (8 to 64), so that
     // short kernels are timed in their steady state rather than by their first launches
     int kReps = 8;

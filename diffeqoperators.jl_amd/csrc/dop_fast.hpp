@@ -120,6 +120,8 @@ void build_fast(const HostPlan& H, FastPlan* fp);
 // not a valid variant.
 bool fast_variant(const FastPlan& fp, int v, FastArgs* out);
 int fast_variant_count(const FastPlan& fp);
+// Whether the tuner tries variant v.
+bool fast_candidate(const FastPlan& fp, int v);
 // The variant of a plan that is not tuned (fewer than 2^20 points, or before its first apply).
 int fast_default(const FastPlan& fp);
 

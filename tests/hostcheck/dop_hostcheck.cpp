@@ -474,3 +474,21 @@ int hc_arena(int64_t budget, int64_t limit, int64_t ahead, int steps, int seed, 
     return bad;
 }
 }  // extern "C"
+
+extern "C" {
+// A tile-shape candidate of the plan: whether the tuner tries it, and its chunk and points per lane;
+// -1 when there is no such candidate.
+int hc_candidate(const dop_desc* d, int v, int* chunk, int* rows, int* vx)
+{
+    dop::HostPlan H;
+    if (dop::build_host_plan(*d, &H, &g_err) != DOP_OK) return -1;
+    dop::FastPlan F;
+    dop::build_fast(H, &F);
+    dop::FastArgs A;
+    if (!dop::fast_variant(F, v, &A)) return -1;
+    *chunk = A.chunk;
+    *rows = A.W * A.VY;
+    *vx = A.VX;
+    return dop::fast_candidate(F, v) ? 1 : 0;
+}
+}  // extern "C"
