@@ -25,6 +25,12 @@ public:
     ~Arena() { clear(); }
     void init(size_t budget) { budget_ = budget; }
 
+    // Memory for n bytes (the budget at most) in one segment, when there is none yet.
+    void reserve(size_t n)
+    {
+        if (total_ == 0 && n > 0) (void)grow(std::min(arena_round(n), budget_));
+    }
+
     // n bytes, or null when they do not fit now (always after a release, and when nothing is
     // allocated only if memory is short).  want(): bytes that the caller expects to need soon.
     template <typename F>

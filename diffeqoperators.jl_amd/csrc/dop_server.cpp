@@ -355,12 +355,16 @@ int dop_server_run(dop_server* srv)
         std::lock_guard<std::mutex> lk(srv->mu);
         if (srv->running) return dop::set_error(DOP_EINVAL, "server: already running");
         srv->running = true;
+        size_t need = 0;
         for (auto& r : srv->reqs) {
             if (r.state == kDone) continue;
             r.state = kScheduled;
             r.done_steps = 0;
             r.admitted = r.completed = -1;
+            need += r.bytes;
         }
+        // (before the clock starts: an allocation of some GB in the loop holds up every class)
+        srv->arena.reserve(need);
         srv->t0 = Clock::now();
     }
     srv->peak_active = 0;

@@ -423,7 +423,7 @@ char* FakeMem::next = reinterpret_cast<char*>(1 << 20);
 extern "C" {
 // 0, or the first rule that fails: 1 a block outside what is held, 2 blocks that overlap, 3 more
 // than the budget held, 4 a request that fits the empty arena (and the memory) refused, 5 memory
-// held after the end, 6 used() wrong.  *most: bytes held at most.
+// held after the end, 6 used() wrong.  *most: bytes held at most.  ahead < 0: reserved at first.
 int hc_arena(int64_t budget, int64_t limit, int64_t ahead, int steps, int seed, int64_t* most)
 {
     FakeMem::limit = (size_t)limit;
@@ -434,6 +434,7 @@ int hc_arena(int64_t budget, int64_t limit, int64_t ahead, int steps, int seed, 
     {
         dop::Arena<FakeMem> A;
         A.init((size_t)budget);
+        if (ahead < 0) A.reserve((size_t)-ahead);
         std::vector<std::pair<char*, size_t>> live;
         size_t used = 0;
         for (int i = 0; i < steps && !bad; ++i) {
@@ -452,7 +453,7 @@ int hc_arena(int64_t budget, int64_t limit, int64_t ahead, int steps, int seed, 
                 // sizes over three decades, up to the whole budget
                 const size_t top = (size_t)budget >> (rng() % 10);
                 const size_t n = std::max<size_t>(top / 2 + rng() % (top / 2 + 1), 1);
-                char* p = A.alloc(n, [&]() { return (size_t)ahead; });
+                char* p = A.alloc(n, [&]() { return (size_t)std::max<int64_t>(ahead, 0); });
                 if (!p) {
                     if (live.empty() && dop::arena_round(n) <= (size_t)std::min(budget, limit)) bad = 4;
                 } else {

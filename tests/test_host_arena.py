@@ -24,7 +24,7 @@ def hc():
 
 @pytest.mark.parametrize("seed", range(8))
 @pytest.mark.parametrize("limit", [1 << 40, BUDGET, BUDGET * 3 // 5])
-@pytest.mark.parametrize("ahead", [0, BUDGET // 7, 4 * BUDGET])
+@pytest.mark.parametrize("ahead", [0, BUDGET // 7, 4 * BUDGET, -BUDGET // 3, -4 * BUDGET])
 def test_random_requests(hc, seed, limit, ahead):
     most = C.c_int64()
     assert hc.hc_arena(BUDGET, limit, ahead, 4000, seed, C.byref(most)) == 0
