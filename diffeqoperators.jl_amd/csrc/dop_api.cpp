@@ -484,7 +484,8 @@ int dop_plan_update(dop_plan* plan, const dop_desc* desc, void* stream)
     if (!plan->d.generic_only) dop::build_fast(H, &F);
     const dop::FastPlan& F0 = plan->d.fast;
     bool same = dop::same_structure(plan->H.meta, H.meta) && F.kind == F0.kind &&
-                F.args.K == F0.args.K && F.VX == F0.VX && F.shell_total == F0.shell_total;
+                F.args.K == F0.args.K && F.VX == F0.VX && F.shell_total == F0.shell_total &&
+                (F.strips.stage_ok || !F0.strips.stage_ok);   // (lines made periodic read their far end)
     for (int a = 0; a < dop::kMaxDim && same; ++a) {
         const dop::AxisTables &A0 = plan->H.axis[a], &A1 = H.axis[a];
         same = A0.w64.size() == A1.w64.size() && A0.w32.size() == A1.w32.size() &&
