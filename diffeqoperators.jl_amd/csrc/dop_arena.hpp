@@ -18,7 +18,7 @@ namespace dop {
 constexpr size_t kArenaAlign = 256;
 inline size_t arena_round(size_t n) { return (n + kArenaAlign - 1) / kArenaAlign * kArenaAlign; }
 
-// Mem: char* get(size_t) (null: no memory) and void put(char*)
+// Mem: char* get(size_t) (null: no memory) and void put(char*, size_t)
 template <typename Mem>
 class Arena {
 public:
@@ -77,6 +77,13 @@ public:
             return;
         }
     }
+    // Gives all memory back (nothing may be resident).
+    void clear()
+    {
+        for (Segment& s : segs_) mem_.put(s.base, s.size);
+        segs_.clear();
+        total_ = used_ = 0;
+    }
     size_t used() const { return used_; }
     size_t total() const { return total_; }
 
@@ -107,12 +114,6 @@ private:
         segs_.push_back({p, size, {{0, size}}});
         total_ += size;
         return true;
-    }
-    void clear()
-    {
-        for (Segment& s : segs_) mem_.put(s.base);
-        segs_.clear();
-        total_ = 0;
     }
     Mem mem_;
     std::vector<Segment> segs_;

@@ -44,10 +44,25 @@ constexpr int64_t kClassPoints[kClasses - 1] = {(int64_t)256 * 256, (int64_t)102
 
 size_t round_up(size_t n) { return dop::arena_round(n); }
 
+// What the servers of a device may still take of its memory: their budgets less what they hold.  A
+// new server's budget must fit beside it.
+constexpr int kMaxDevices = 64;
+std::mutex g_promised_mu;
+size_t g_promised[kMaxDevices] = {};
+
 // Device memory of a server's arena, on the server's device
 struct ArenaMem {
     int device = 0;
-    ArenaMem() { (void)hipGetDevice(&device); }
+    ArenaMem()
+    {
+        (void)hipGetDevice(&device);
+        if (device < 0 || device >= kMaxDevices) device = 0;
+    }
+    static void taken(int device, size_t n, bool back)
+    {
+        std::lock_guard<std::mutex> lk(g_promised_mu);
+        g_promised[device] = back ? g_promised[device] + n : g_promised[device] - n;
+    }
     char* get(size_t n) const
     {
         int cur = device;
@@ -59,9 +74,14 @@ struct ArenaMem {
             p = nullptr;
         }
         if (cur != device) (void)hipSetDevice(cur);
+        if (p) taken(device, n, false);
         return (char*)p;
     }
-    void put(char* p) const { (void)hipFree(p); }
+    void put(char* p, size_t n) const
+    {
+        (void)hipFree(p);
+        taken(device, n, true);
+    }
 };
 
 enum State { kScheduled, kPending, kActive, kDraining, kDone, kFailed };
@@ -116,6 +136,8 @@ int class_of(int64_t points)
 
 struct dop_server {
     int64_t budget = 0;
+    int device = 0;
+    bool promised = false;         // its budget is among g_promised
     int max_active = 0;
     int chunk = 16;
     int storage = -1;
@@ -133,6 +155,8 @@ struct dop_server {
     int64_t iterations = 0;
     ~dop_server()
     {
+        arena.clear();
+        if (promised) ArenaMem::taken(device, (size_t)budget, false);
         for (auto& r : reqs)
             if (r.done_ev) (void)hipEventDestroy(r.done_ev);
         for (auto& c : cls) {
@@ -282,8 +306,16 @@ int dop_server_create(int64_t hbm_budget_bytes, int max_active, int chunk, void*
     s->chunk = chunk > 0 ? chunk : 16;
     s->stream = (hipStream_t)stream;
     // (a budget that is not there is refused now, although the arena takes it as requests come)
+    s->device = ArenaMem().device;
     size_t avail = 0, all = 0;
-    if (s->budget <= 0 || hipMemGetInfo(&avail, &all) != hipSuccess || (size_t)s->budget > avail) {
+    if (s->budget > 0 && hipMemGetInfo(&avail, &all) == hipSuccess) {
+        std::lock_guard<std::mutex> lk(g_promised_mu);
+        if (avail > g_promised[s->device] && (size_t)s->budget <= avail - g_promised[s->device]) {
+            g_promised[s->device] += (size_t)s->budget;
+            s->promised = true;
+        }
+    }
+    if (!s->promised) {
         delete s;
         return dop::set_error(DOP_ENOMEM, "server: the device has less free memory than the budget");
     }

@@ -409,8 +409,9 @@ struct FakeMem {
         most = std::max(most, given);
         return p;
     }
-    void put(char* p)
+    void put(char* p, size_t n)
     {
+        if (held.at(p) != n) given += n;   // (shows as memory held after the end)
         given -= held.at(p);
         held.erase(p);
     }

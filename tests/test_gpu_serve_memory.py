@@ -69,3 +69,17 @@ def test_pieces_and_the_whole_budget():
     for i, w in zip(ids, want):
         assert torch.equal(srv.results[i], w)
     assert srv.stats()["peak_bytes"] == budget
+
+
+def test_budgets_of_two_servers_must_fit_together():
+    free = torch.cuda.mem_get_info()[0]
+    a = D.Server(free * 6 // 10)
+    with pytest.raises(D._abi.DopError) as e:
+        D.Server(free * 6 // 10)
+    assert e.value.code == D._abi.ENOMEM
+    p, u0, dt = request(64, 1)
+    got = serve(a, [(p, u0, dt)])
+    with pytest.raises(D._abi.DopError):
+        D.Server(free * 6 // 10)
+    del a
+    assert torch.equal(got[0], serve(D.Server(free * 6 // 10), [(p, u0, dt)])[0])
