@@ -413,7 +413,7 @@ int dop_server_run(dop_server* srv)
     size_t known = 0;                  // requests taken from srv->reqs so far
     size_t ndone = 0;
     int rc = DOP_OK;
-    int nactive = 0;
+    int nactive = 0;   // admitted requests with steps to come
     for (;;) {
         const double t = now();
         size_t nreq;
@@ -471,7 +471,9 @@ int dop_server_run(dop_server* srv)
                 break;
             }
         }
-        srv->peak_active = std::max(srv->peak_active, nactive);
+        // (a request on its way back holds its memory, and its slot until another needs it)
+        srv->peak_active = std::max(srv->peak_active,
+                                    std::min(nactive + (int)draining.size(), srv->max_active));
         srv->peak_bytes = std::max(srv->peak_bytes, (int64_t)srv->arena.used());
         if (rc != DOP_OK) break;
         // step every class whose queue ahead of the GPU has room

@@ -282,7 +282,8 @@ double dop_server_now(const dop_server* srv);
 /* times (s, relative to the run start) of request `id`: release, admission, completion */
 int dop_server_times(const dop_server* srv, int64_t id, double* release, double* admitted,
                      double* completed);
-/* peak resident requests and peak arena bytes during the last run */
+/* peak resident requests (at most max_active: a request whose last step is queued keeps its slot
+ * until its state is back or another request needs the slot) and peak arena bytes in the last run */
 int dop_server_stats(const dop_server* srv, int* peak_active, int64_t* peak_bytes,
                      int64_t* iterations);
 void dop_server_destroy(dop_server* srv);

@@ -83,3 +83,15 @@ def test_budgets_of_two_servers_must_fit_together():
         D.Server(free * 6 // 10)
     del a
     assert torch.equal(got[0], serve(D.Server(free * 6 // 10), [(p, u0, dt)])[0])
+
+
+def test_a_request_is_resident_until_its_state_is_back():
+    # one slot: the second of two requests takes it over; two slots: a state of 64 MB is on its way back
+    # for longer than the few steps of a small request that comes when the last step is queued
+    big, small = request(2048, 1, torch.float64), request(64, 2, torch.float64)
+    srv = D.Server(1 << 30, max_active=1)
+    serve(srv, [big, small], nsteps=1)
+    assert srv.stats()["peak_active"] == 1
+    srv = D.Server(1 << 30, max_active=2)
+    serve(srv, [big, small], nsteps=1)
+    assert srv.stats()["peak_active"] == 2
