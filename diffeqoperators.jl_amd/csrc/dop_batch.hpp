@@ -55,8 +55,11 @@ enum BItemKind : int32_t {
 struct BItem {
     int32_t prob, kind, a, b, c, d;
 };
-// Points per lane of a marching segment: a 16-byte load, or half of one where four rings of that
-// many would not fit 256 registers (f32: wide windows, and sums of more than one register).
+// Points per lane of a marching segment: a 16-byte load, or half of one for the widest windows of f32
+// (and sums of more than one register), whose four rings of K + 1 rows would take all of the 256
+// registers by themselves.  That leaves some short of registers still: the compiler spills 33 at f32
+// sums and K = 9, 84 / 17 / 74 at f32 values summed in f64 and K = 7 / 9 / 11, 43 at f64 and K = 11
+// (72 to 316 bytes of scratch a lane), the others none.  Half the points there was not measured.
 constexpr int march_vx(int storage, int accum, int K)
 {
     return storage == kF64 ? 2 : K >= 11 || (accum != kAccF32 && K >= 9) || (accum == kAccF32Kahan && K >= 7) ? 2 : 4;

@@ -17,6 +17,8 @@ namespace {
 // The box of a 2-D tiled problem that marching segments take: the points whose four-stage cone (4H
 // in x and y) holds regular rows only, whole lane groups along x.  False when it is too small to
 // pay (its rim, 4H to 5H points a side, and the 4H columns beside every segment are recomputed).
+// Against patches alone, us a step (K = 5, 2 / 24 problems): 125^2 f32 33 / 33 and 34 / 64, f64 33 / 34 and
+// 34 / 49; at 100^2, a box of 76, f32 35 / 34 and 38 / 38, f64 34 / 34 and 25 / 32.
 constexpr int kMarchMin = 96;
 
 constexpr int kPatchRows = 32;   // rows of own points of a patch at most

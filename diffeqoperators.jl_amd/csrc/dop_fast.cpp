@@ -346,7 +346,7 @@ bool fast_candidate(const FastPlan& fp, int v)
 {
     // 3-D chunks of 16 planes read K - 1 more for each 16, 16 % more than chunks of 32 (K = 7), for
     // more blocks: where chunks of 32 give every CU four they only win the tuner's short runs (512^3
-    // f32: 321 us against 326 there, 337 against 333 in an application's loop).
+    // f32: 321 us against 326 there, 337 against 334 in an application's loop).
     FastArgs A;
     if (fp.kind != 3 || !fast_variant(fp, v, &A) || A.chunk > 16) return true;
     return (int64_t)A.nxseg * A.nyblk * ceil_div(A.hi[2] - A.lo[2], 32) < 4 * 256;

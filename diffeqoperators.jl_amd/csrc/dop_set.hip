@@ -17,9 +17,9 @@
 // a plane's rows and their halo along axis 1 are loaded once, a plane ahead: 2.5 loads of a value
 // pair a point in place of 24 (curl, K = 5).  The shell of the box goes to the last blocks of the
 // same launch, which run k_apply_set's code (first: 157 us).  Curl of 256^3 f32: 148 us, of which
-// the box alone takes 125.  Bound by memory: 0.77 GB moved at 5.2 TB/s, as rows of the halos along
-// axis 1 are read by up to three waves at different times (neighbouring groups of rows on one XCD:
-// 156 us; R = 2: 154), and at its end by the shell's points.
+// the box alone takes 125.  Bound by memory: 0.72 GB moved (reads 2.4 times, writes 1.1) at 4.9 TB/s, as
+// rows of the halos along axis 1 are read by up to three waves at different times (neighbouring
+// groups of rows on one XCD: 156 us; R = 2: 154), and at its end by the shell's points.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>

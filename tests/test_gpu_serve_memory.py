@@ -86,8 +86,7 @@ def test_budgets_of_two_servers_must_fit_together():
 
 
 def test_a_request_is_resident_until_its_state_is_back():
-    # one slot: the second of two requests takes it over; two slots: a state of 64 MB is on its way back
-    # for longer than the few steps of a small request that comes when the last step is queued
+    # one slot: the second request takes it over while the first one's state (34 MB) is on its way back
     big, small = request(2048, 1, torch.float64), request(64, 2, torch.float64)
     srv = D.Server(1 << 30, max_active=1)
     serve(srv, [big, small], nsteps=1)
