@@ -4,8 +4,8 @@
 // One allocation of the whole budget per server cost small bursts more than their steps: of a
 // 2 GiB budget 0.3 ms to make and 0.45 ms to free at best, and now and then 40 to 1260 ms to make
 // or 43 to 57 ms to free, for bursts of 1.5 to 6 ms (two to twelve requests of 64^2 to 600^2).  A
-// segment is as large as the requests known when it is made, so a burst has one, and one that
-// fills the budget has the whole budget in one, as before.
+// segment is as large as the requests known when it is made, so a burst has one, and a long stream
+// that needs it has the whole budget in one.
 #pragma once
 #include <algorithm>
 #include <cstddef>
