@@ -356,7 +356,10 @@ int fast_default(const FastPlan& fp)
 {
     if (fp.kind < 2) return 0;
     // the order of preference with plenty of points; the first that gives every CU two blocks
-    // (four waves of a 2-D block, eight of a 3-D one) is taken, else the one of most blocks
+    // (four waves of a 2-D block, eight of a 3-D one) is taken, else the one of most blocks.
+    // us by chunk, longest first: 512^2 f32 14.8 / 8.7 / 7.0 / 6.9, 1000 x 3000 16.6 / 10.1 / 8.4 /
+    // 8.4 (64, 32, 16, 8 rows; none there has 512 blocks); 128^3 f32 40.3 / 37.9 / 37.4, 203 x 190 x
+    // 177 f32 47.8 / 47.1 / 48.5 and f64 57.7 / 61.1 / 60.4
     static const int v2[4] = {4, 0, 2, 6};                    // 2-D chunks 64, 32, 16, 8
     static const int w3[3] = {0, 6, 7};                       // 3-D (8,2)x32, (8,2)x16, (8,1)x16
     const bool half = fp.kind == 3 && fp.VX > 1 && fp.args.hi[0] - fp.args.lo[0] <= 32 * fp.VX;
